@@ -141,8 +141,7 @@ __global__ __launch_bounds__(MARCH_BLOCK) __attribute__((amdgpu_waves_per_eu(8))
 
 // The closest hit of each path over its bounded hit and its unbounded objects' marches, in list order with
 // strict < (object/list.rs:120-125).  The paths whose closest hit becomes an unbounded object are appended to
-// sdf_queue for k_sdf_normal: each wave takes strips of MERGE_STRIP * 64 queue positions, stages those slots in
-// its part of LDS and appends them with one atomic per strip.
+// sdf_queue for k_sdf_normal, block by block as k_shade appends to the next queue.
 constexpr uint32_t MERGE_STRIP = 16;
 
 template <bool BATCH>
@@ -152,15 +151,15 @@ __global__ __launch_bounds__(BLOCK) void k_march_merge(SceneView sv, FrameParams
                                                        int32_t *sdf_queue, uint32_t *sdf_count, BatchView bv) {
     const uint32_t count = queue ? *count_ptr : fp.n_slots;
     __shared__ uint32_t staged[BLOCK * MERGE_STRIP];
-    uint32_t *mine = staged + (threadIdx.x / 64) * 64 * MERGE_STRIP;
-    const uint32_t lane = __lane_id();
+    __shared__ uint32_t kept[BLOCK / 64], strip_base;
+    const uint32_t lane = __lane_id(), wave = threadIdx.x / 64;
+    uint32_t *mine = staged + wave * 64 * MERGE_STRIP;
     const unsigned long long below = (1ull << lane) - 1ull;
-    const uint32_t n_waves = gridDim.x * (BLOCK / 64);
-    const uint32_t wave = blockIdx.x * (BLOCK / 64) + threadIdx.x / 64;
-    for (uint32_t base = wave * 64 * MERGE_STRIP; base < count; base += n_waves * 64 * MERGE_STRIP) {
+    const uint32_t strip = queue_strip(count, MERGE_STRIP);
+    for (uint32_t base = blockIdx.x * BLOCK * strip; base < count; base += gridDim.x * BLOCK * strip) {
       uint32_t n_kept = 0;
-      for (uint32_t jx = 0; jx < MERGE_STRIP; ++jx) {
-        const uint32_t q = base + jx * 64 + lane;
+      for (uint32_t jx = 0; jx < strip; ++jx) {
+        const uint32_t q = base + (wave * strip + jx) * 64 + lane;
         bool changed = false;
         uint32_t slot = 0;
         if (q < count) {
@@ -198,18 +197,7 @@ __global__ __launch_bounds__(BLOCK) void k_march_merge(SceneView sv, FrameParams
         if (changed) mine[n_kept + (uint32_t)__popcll(mask & below)] = slot;
         n_kept += (uint32_t)__popcll(mask);
       }
-      if (n_kept != 0u) {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        uint32_t wbase = 0;
-        if (lane == 0u) wbase = atomicAdd(sdf_count, n_kept);
-        wbase = __shfl(wbase, 0);
-        for (uint32_t i = lane; i < n_kept; i += 64) sdf_queue[wbase + i] = (int32_t)mine[i];
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      }
+      append_strip(mine, n_kept, kept, &strip_base, sdf_queue, sdf_count);
     }
 }
 
