@@ -76,11 +76,10 @@ struct Pipeline {
     int32_t *queue[2] = {nullptr, nullptr};
     uint32_t *queue_count = nullptr;
     uint32_t queue_count_len = 0;
-    uint32_t *claims = nullptr;    // extend claim counters, EXTEND_CLAIM_WORDS per depth
+    uint32_t *claims = nullptr;    // claim counters, CLAIM_WORDS for k_extend and for k_march per depth
     unsigned long long *segments = nullptr;
     float *mt = nullptr;           // march outcomes, 2 * capacity * n_sdf_max
     int32_t *sdf_queue = nullptr;  // scenes with unbounded objects: SDF-hit slots (normals in pb.sdf_n*)
-    uint32_t *sdf_count = nullptr;
     int2 *overflow = nullptr;      // traversal stack entries beyond the LDS part
 };
 
@@ -168,7 +167,6 @@ void free_pipe(rayna_batch *b, Pipeline &P) {
     P.segments = nullptr;
     P.mt = nullptr;
     P.sdf_queue = nullptr;
-    P.sdf_count = nullptr;
     P.overflow = nullptr;
     P.capacity = 0;
     free_graph(b);
@@ -204,10 +202,10 @@ rayna_status alloc_pipe(rayna_batch *b, int p, uint64_t slots, uint32_t max_dept
     if ((st = alloc(slots * sizeof(uint32_t), (void **)&P.slot_req)) != RAYNA_OK) return st;
     for (int q = 0; q < 2; ++q)
         if ((st = alloc(slots * sizeof(int32_t), (void **)&P.queue[q])) != RAYNA_OK) return st;
-    // [0, D+2) paths entering each depth; [D+2, 2(D+2)) extend counters; [2(D+2), 3(D+2)) march counters
+    // [0, D+2) paths entering each depth; [2(D+2), 3(D+2)) SDF hits at each depth
     const uint32_t qlen = 3 * (std::max<uint32_t>(max_depth, 16) + 2);
     if ((st = alloc(qlen * sizeof(uint32_t), (void **)&P.queue_count)) != RAYNA_OK) return st;
-    if ((st = alloc((size_t)(qlen / 3) * EXTEND_CLAIM_WORDS * sizeof(uint32_t), (void **)&P.claims)) != RAYNA_OK)
+    if ((st = alloc((size_t)(qlen / 3) * 2 * CLAIM_WORDS * sizeof(uint32_t), (void **)&P.claims)) != RAYNA_OK)
         return st;
     if ((st = alloc(sizeof(unsigned long long), (void **)&P.segments)) != RAYNA_OK) return st;
     if (b->n_sdf_max) {
@@ -216,7 +214,6 @@ rayna_status alloc_pipe(rayna_batch *b, int p, uint64_t slots, uint32_t max_dept
         for (float **f : planes)
             if ((st = alloc(slots * sizeof(float), (void **)f)) != RAYNA_OK) return st;
         if ((st = alloc(slots * sizeof(int32_t), (void **)&P.sdf_queue)) != RAYNA_OK) return st;
-        if ((st = alloc(sizeof(uint32_t), (void **)&P.sdf_count)) != RAYNA_OK) return st;
     }
     if (b->overflow_entries && (st = alloc(b->overflow_entries * sizeof(int2), (void **)&P.overflow)) != RAYNA_OK)
         return st;
@@ -463,7 +460,7 @@ hipError_t enqueue(rayna_batch *b, const Plan &pl, int used, bool timing) {
         const uint32_t D = pl.depth[c];
         const SceneView cv = chunk_view(b->view, pl.features[c]);
         launch_fill_u32(P.queue_count, 0u, 3 * (D + 2), s);
-        launch_fill_u32(P.claims, 0u, (D + 1) * EXTEND_CLAIM_WORDS, s);
+        launch_fill_u32(P.claims, 0u, (D + 1) * 2 * CLAIM_WORDS, s);
         // the camera rays are stored only where a kernel loads them: k_extend and k_march at depth 0 (the camera-ray
         // packets and the first k_shade compute them); k_generate records every slot's request either way
         fp.rays_stored = (pl.features[c] & SCENE_SDFS) != 0u || !extend_packets(cv, fp, b->tune, bv, 0);
@@ -473,11 +470,11 @@ hipError_t enqueue(rayna_batch *b, const Plan &pl, int used, bool timing) {
             const uint32_t *cin = depth == 0 ? nullptr : P.queue_count + depth;
             int32_t *qout = P.queue[(depth + 1) & 1];
             uint32_t *cout = P.queue_count + depth + 1;
-            uint32_t *work = P.claims + (size_t)depth * EXTEND_CLAIM_WORDS;
+            uint32_t *work = P.claims + (size_t)depth * 2 * CLAIM_WORDS;
             launch_extend(cv, fp, P.pb, qin, cin, depth, b->grid_extend, P.overflow, work, b->tune, bv, s);
             launch_march(cv, fp, P.pb, qin, cin, pl.n_sdf[c], P.mt, P.capacity * b->n_sdf_max,
-                         P.queue_count + 2 * (D + 2) + depth, b->grid_march, b->grid_shade, b->tune, bv,
-                         P.sdf_queue, P.sdf_count, s);
+                         work + CLAIM_WORDS, b->grid_march, b->grid_shade, b->tune, bv, P.sdf_queue,
+                         P.queue_count + 2 * (D + 2) + depth, s);
             launch_shade(cv, fp, P.pb, qin, cin, qout, cout, depth, b->grid_shade, nullptr, bv, s);
         }
         launch_count_segments(P.queue_count, D + 1, fp.n_slots, P.segments, s);

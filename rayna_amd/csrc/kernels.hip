@@ -479,6 +479,77 @@ __device__ __forceinline__ uint32_t queue_strip(uint32_t count, uint32_t most) {
     return n < most ? n : most;
 }
 
+// The positions of a launch's work, [0, count), as its persistent waves take them.  The range is cut into CLAIM_PARTS
+// contiguous parts with a counter each, one 128-byte line apart; a wave starts on part blockIdx.x % CLAIM_PARTS and
+// moves to the next part when its own is used up.  Workgroups go to the eight XCDs in turn, so each part (a band of
+// neighbouring pixels) is worked through by two XCDs, whose L2s then hold its nodes, and no single counter takes
+// every claim of the launch.  A wave's first claim is fixed by its place in the grid and costs no atomic; the
+// counters hand out what is left after those.  Atomics on one address are served one at a time, about 7 ns each, so
+// where the first claims cover a part nobody touches its counter (a launch over a few thousand positions spent
+// 50-75 us on some 7000 waves each asking every counter), and a wave looks at a foreign part's counter before it
+// adds to it.  A claim is the wave's even share of the launch, within bounds: a small launch runs on every wave with
+// few lanes each, instead of on the few waves that full claims would feed.  (Against claims of 128 rays or 512 march
+// items and one atomic each: the 64x36, 2-sample sphere frame 1074 -> 525 us, the 161x91, 9-sample SDF frame 13.7 ->
+// 9.3 ms; shares a half or a quarter as large were 1-10% slower below 400x225x32.)  Every field is wave-uniform.
+struct WaveClaims {
+    uint32_t count, claim, waves_per_block;
+    uint32_t *work;
+    uint32_t part, parts_done;
+    bool first, last;  // first: no claim taken yet; last: every part is used up
+
+    // least, most: the bounds of a claim's size
+    __device__ __forceinline__ WaveClaims(uint32_t n, uint32_t wpb, uint32_t least, uint32_t most, uint32_t *counters)
+        : count(n), waves_per_block(wpb), work(counters), part(blockIdx.x % CLAIM_PARTS), parts_done(0), first(true),
+          last(false) {
+        const uint32_t waves = gridDim.x * wpb;
+        const uint32_t per = n / waves + (n % waves != 0u ? 1u : 0u);
+        claim = per < least ? least : per;
+        claim = claim < most ? claim : most;
+    }
+    __device__ __forceinline__ uint32_t bound(uint32_t p) const {
+        return (uint32_t)(((uint64_t)count * p) / CLAIM_PARTS);
+    }
+    // The wave's next claim [*from, *to), empty once there is none left (last).  `leader`: the active lane that does
+    // the atomic.
+    __device__ __forceinline__ void take(int leader, uint32_t *from, uint32_t *to) {
+        for (;;) {
+            const uint32_t lo = bound(part), size = bound(part + 1) - lo;
+            const uint32_t blocks = (gridDim.x + CLAIM_PARTS - 1u - part) / CLAIM_PARTS;
+            const uint64_t fixed = (uint64_t)blocks * waves_per_block * claim;  // the part's first claims
+            uint32_t base = size;
+            if (first) {
+                const uint64_t at =
+                    ((uint64_t)(blockIdx.x / CLAIM_PARTS) * waves_per_block +
+                     __builtin_amdgcn_readfirstlane(threadIdx.x / 64u)) * claim;
+                base = at < size ? (uint32_t)at : size;
+                first = false;
+            } else if (fixed < size) {
+                const uint32_t left = size - (uint32_t)fixed;
+                uint32_t taken = 0;
+                if ((int)__lane_id() == leader) {
+                    uint32_t *counter = work + 32 * part;
+                    taken = parts_done == 0u
+                                ? 0u
+                                : __hip_atomic_load(counter, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    if (taken < left) taken = atomicAdd(counter, claim);
+                }
+                taken = __builtin_amdgcn_readlane(taken, leader);
+                if (taken < left) base = (uint32_t)fixed + taken;
+            }
+            const bool got = base < size;
+            if (got) {
+                *from = lo + base;
+                *to = size - base > claim ? lo + base + claim : lo + size;
+            }
+            if (!got || *to == lo + size) {  // this part is used up
+                part = part + 1 == CLAIM_PARTS ? 0 : part + 1;
+                if (++parts_done == CLAIM_PARTS) last = true;
+            }
+            if (got || last) return;
+        }
+    }
+};
+
 // Appends the n_kept slots each wave of the block has staged at `mine` to queue_out, wave by wave in order, with one
 // atomic on *count_out.  The whole block calls it; kept and strip_base are the block's LDS.
 __device__ __forceinline__ void append_strip(const uint32_t *mine, uint32_t n_kept, uint32_t *kept,
@@ -1443,7 +1514,6 @@ void launch_march(const SceneView &sv, const FrameParams &fp, const PathBuffers 
                   int merge_grid, const ExtendTuning &tune, const BatchView &bv, int32_t *sdf_queue,
                   uint32_t *sdf_count, hipStream_t s) {
     if (n_sdf == 0) return;
-    launch_fill_u32(sdf_count, 0u, 1, s);
     if (bv.reqs) {
         hipLaunchKernelGGL(k_march<true>, dim3(grid), dim3(MARCH_BLOCK), 0, s, fp, pb, sv.sdfs, sv.spheres, queue,
                            count, n_sdf, mt, mt_stride, work, tune, bv);

@@ -87,17 +87,17 @@ constexpr int SHADE_BLOCKS_PER_CU = 16;
 // them as 1 and 0, and the adjoint replay reads the primal radiance still held there).  With bv.reqs,
 // fp.n_slots is the chunk's slot count and the requests come from bv.
 void launch_generate(const FrameParams &fp, const PathBuffers &pb, const BatchView &bv, hipStream_t s);
-// Claim counters of one extend launch: the queue is cut into EXTEND_PARTS contiguous parts, each with its own
-// counter, one 128-byte line apart (EXTEND_CLAIM_WORDS words in all, zeroed before the launch).
-#ifndef RAYNA_EXTEND_PARTS
-#define RAYNA_EXTEND_PARTS 4
+// Claim counters of one k_extend or k_march launch: its work is cut into CLAIM_PARTS contiguous parts, each with its
+// own counter, one 128-byte line apart (CLAIM_WORDS words in all, zeroed before the launch).
+#ifndef RAYNA_CLAIM_PARTS
+#define RAYNA_CLAIM_PARTS 4
 #endif
-constexpr uint32_t EXTEND_PARTS = RAYNA_EXTEND_PARTS;
-constexpr uint32_t EXTEND_CLAIM_WORDS = EXTEND_PARTS * 32;
+constexpr uint32_t CLAIM_PARTS = RAYNA_CLAIM_PARTS;
+constexpr uint32_t CLAIM_WORDS = CLAIM_PARTS * 32;
 
 // queue == nullptr: identity queue of fp.n_slots entries; else queue[0 .. *count)
 // overflow: traversal stack entries beyond the LDS part, extend_block() * grid * (stack_need - extend_lds_stack());
-// work: EXTEND_CLAIM_WORDS zeroed words, the counters the launch's waves take rays from
+// work: CLAIM_WORDS zeroed words, the counters the launch's waves take rays from
 void launch_extend(const SceneView &sv, const FrameParams &fp, const PathBuffers &pb, const int32_t *queue,
                    const uint32_t *count, uint32_t depth, int grid, int2 *overflow, uint32_t *work,
                    const ExtendTuning &tune, const BatchView &bv, hipStream_t s);
@@ -107,8 +107,8 @@ void launch_shade(const SceneView &sv, const FrameParams &fp, const PathBuffers 
 // The unbounded SDF objects of each queued path (n_sdf per path; in a batch, each request's own), marched
 // after launch_extend with its hit as the cut, then merged into the hit record; the paths whose closest hit
 // becomes an SDF get their shading normal in pb.sdf_n*.  mt: two planes of mt_stride >= count * n_sdf floats
-// (outcome, march iteration).  work: a zeroed counter.  sdf_queue: room for every queued path; sdf_count: one
-// counter (zeroed here).  No-op for n_sdf == 0.
+// (outcome, march iteration).  work: CLAIM_WORDS zeroed words.  sdf_queue: room for every queued path; sdf_count: one
+// zeroed counter.  No-op for n_sdf == 0.
 void launch_march(const SceneView &sv, const FrameParams &fp, const PathBuffers &pb, const int32_t *queue,
                   const uint32_t *count, uint32_t n_sdf, float *mt, uint64_t mt_stride, uint32_t *work, int grid,
                   int merge_grid, const ExtendTuning &tune, const BatchView &bv, int32_t *sdf_queue,

@@ -25,6 +25,8 @@ constexpr int MARCH_BLOCK = 256;
 // counter: with claims as small as the extend kernels' the waves waited on that counter (the SDF frame at 128,
 // 512, 1024 and 2048 items per claim for both kinds of kernel: 85.6, 76.7, 79.3 and 89.3 ms).
 constexpr uint32_t MARCH_CLAIM_FACTOR = 4;
+// Fewest items a wave claims (the 161x91, 9-sample SDF frame at 32, 16 and 8: 9.68, 9.39 and 9.26 ms).
+constexpr uint32_t MARCH_CLAIM_LEAST = 8;
 
 // The state of a lane's march (k_march): its item, ray and cut, the march distance and step.
 struct MarchLane {
@@ -66,9 +68,10 @@ __global__ __launch_bounds__(MARCH_BLOCK) __attribute__((amdgpu_waves_per_eu(8))
     ExtendTuning tune, BatchView bv) {
     const uint32_t count = queue ? *count_ptr : fp.n_slots;
     const uint32_t n_items = count * n_sdf;
-    const uint32_t refill_lanes = tune.refill_lanes, wave_batch = tune.wave_batch * MARCH_CLAIM_FACTOR;
+    const uint32_t refill_lanes = tune.refill_lanes;
+    WaveClaims claims(n_items, MARCH_BLOCK / 64, MARCH_CLAIM_LEAST, tune.wave_batch * MARCH_CLAIM_FACTOR, work);
     const uint32_t lane = __lane_id();
-    bool active = false, exhausted = false, last_claim = false;
+    bool active = false, exhausted = false;
     uint32_t batch_next = 0, batch_end = 0;
     int32_t j = 0;  // the lane's SDF
     MarchLane L{};
@@ -78,15 +81,8 @@ __global__ __launch_bounds__(MARCH_BLOCK) __attribute__((amdgpu_waves_per_eu(8))
             const uint32_t n = (uint32_t)__popcll(idle);
             const uint32_t rem = batch_end - batch_next;
             uint32_t nb = 0, nb_end = 0;
-            if (rem < n && !last_claim && (idle == ~0ull || n >= refill_lanes)) {
-                const int leader = __ffsll((long long)idle) - 1;
-                uint32_t base = 0;
-                if ((int)lane == leader) base = atomicAdd(work, wave_batch);
-                base = __shfl(base, leader);
-                nb = base < n_items ? base : n_items;
-                nb_end = (n_items - nb > wave_batch) ? nb + wave_batch : n_items;
-                if (nb_end >= n_items) last_claim = true;
-            }
+            if (rem < n && !claims.last && (idle == ~0ull || n >= refill_lanes))
+                claims.take(__ffsll((long long)idle) - 1, &nb, &nb_end);
             const uint32_t idx = (uint32_t)__popcll(idle & ((1ull << lane) - 1ull));
             uint32_t q = 0xffffffffu;
             if (idx < rem) q = batch_next + idx;
@@ -100,7 +96,7 @@ __global__ __launch_bounds__(MARCH_BLOCK) __attribute__((amdgpu_waves_per_eu(8))
             } else {
                 batch_next = batch_end;
             }
-            if (last_claim && batch_next == batch_end) exhausted = true;
+            if (claims.last && batch_next == batch_end) exhausted = true;
             if (!active && q != 0xffffffffu) {
                 const uint32_t jj = q / count, qq = q % count;
                 const uint32_t slot = queue ? (uint32_t)queue[qq] : qq;

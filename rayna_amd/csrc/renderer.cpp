@@ -55,7 +55,7 @@ struct rayna_renderer {
     PathBuffers pb{};
     int32_t *queue[2] = {nullptr, nullptr};
     uint32_t *queue_count = nullptr;
-    uint32_t *claims = nullptr;  // extend claim counters, EXTEND_CLAIM_WORDS per depth and one set for queries
+    uint32_t *claims = nullptr;  // claim counters: CLAIM_WORDS for k_extend and for k_march per depth, and for queries
     unsigned long long *segments = nullptr;
     float *sum = nullptr, *acc = nullptr, *out_dev = nullptr;
     uint8_t *rgba_dev = nullptr;  // the 8-bit output of rayna_render_srgb8
@@ -76,10 +76,9 @@ struct rayna_renderer {
     int grid_extend = 1024, grid_shade = 1024, grid_march = 1024;
     int cus = 1;
     float *mt = nullptr;  // unbounded-object march outcomes, slot_capacity * n_sdfs
-    void *sdf_buf = nullptr;  // scenes with unbounded objects: SDF-hit normals (three planes), their queue, a counter
+    void *sdf_buf = nullptr;  // scenes with unbounded objects: SDF-hit normals (three planes) and their queue
     uint64_t sdf_cap = 0;
     int32_t *sdf_queue = nullptr;
-    uint32_t *sdf_count = nullptr;
     uint64_t mt_cap = 0;
     uint64_t chunk_target = TARGET_SLOTS;
     ExtendTuning tune;
@@ -235,8 +234,8 @@ void free_paths(rayna_renderer *r) {
 }
 
 // The march outcome buffer: two planes (outcome, march iteration) of one float per (slot, unbounded object);
-// and for scenes with unbounded objects the SDF-hit normals (three planes of one float per slot), the queue of
-// SDF-hit slots and its counter.  Sets the path buffers' normal planes (free_paths clears them).
+// and for scenes with unbounded objects the SDF-hit normals (three planes of one float per slot) and the queue of
+// SDF-hit slots.  Sets the path buffers' normal planes (free_paths clears them).
 rayna_status ensure_mt(rayna_renderer *r) {
     const uint64_t need = r->slot_capacity * (uint64_t)std::max(0, r->dev.view.n_sdfs);
     if (need > r->mt_cap) {
@@ -251,7 +250,7 @@ rayna_status ensure_mt(rayna_renderer *r) {
         if (r->sdf_buf) (void)hipFree(r->sdf_buf);
         r->sdf_buf = nullptr;
         r->sdf_cap = 0;
-        HIP_TRY(r, hipMalloc(&r->sdf_buf, cap * (3 * sizeof(float) + sizeof(int32_t)) + sizeof(uint32_t)));
+        HIP_TRY(r, hipMalloc(&r->sdf_buf, cap * (3 * sizeof(float) + sizeof(int32_t))));
         r->sdf_cap = cap;
     }
     if (r->dev.view.n_sdfs > 0) {
@@ -261,7 +260,6 @@ rayna_status ensure_mt(rayna_renderer *r) {
         r->pb.sdf_ny = f + c;
         r->pb.sdf_nz = f + 2 * c;
         r->sdf_queue = reinterpret_cast<int32_t *>(f + 3 * c);
-        r->sdf_count = reinterpret_cast<uint32_t *>(r->sdf_queue + c);
     } else {
         r->pb.sdf_nx = r->pb.sdf_ny = r->pb.sdf_nz = nullptr;
     }
@@ -279,8 +277,8 @@ rayna_status alloc_paths(rayna_renderer *r) {
     const uint64_t slots = P * chunk;
     if (slots > 0x7fffffffull || slots * n_sdf > 0xffffffffull)
         return fail(r, RAYNA_UNSUPPORTED, "image too large for one chunk of paths");
-    // [0, D+2) paths entering each depth; [D+2, 2(D+2)) extend ray counters; [2(D+2), 3(D+2)) march item
-    // counters; [3(D+2)], [3(D+2)+1]: the primary-hit query's two counters
+    // [0, D+2) paths entering each depth; [2(D+2), 3(D+2)) SDF hits at each depth; [3(D+2)]: the primary-hit
+    // query's SDF hits
     const uint32_t qlen = 3 * (o.ray_depth + 2) + 2;
     if (slots <= r->slot_capacity && P <= r->alloc_pixels && qlen <= r->queue_count_len) {
         // the buffers are large enough: keep them (grow-only)
@@ -306,7 +304,7 @@ rayna_status alloc_paths(rayna_renderer *r) {
     for (int q = 0; q < 2; ++q)
         if ((st = alloc(slots * sizeof(int32_t), (void **)&r->queue[q])) != RAYNA_OK) return st;
     if ((st = alloc(qlen * sizeof(uint32_t), (void **)&r->queue_count)) != RAYNA_OK) return st;
-    if ((st = alloc((size_t)(o.ray_depth + 3) * EXTEND_CLAIM_WORDS * sizeof(uint32_t), (void **)&r->claims)) !=
+    if ((st = alloc((size_t)(o.ray_depth + 3) * 2 * CLAIM_WORDS * sizeof(uint32_t), (void **)&r->claims)) !=
         RAYNA_OK)
         return st;
     if ((st = alloc(sizeof(unsigned long long), (void **)&r->segments)) != RAYNA_OK) return st;
@@ -370,7 +368,7 @@ void trace_chunk(rayna_renderer *r, FrameParams &fp, uint32_t s0, uint32_t n, st
     fp.n_slots = fp.n_pixels * n;
     const uint32_t D2 = r->opts.ray_depth + 2;
     launch_fill_u32(r->queue_count, 0u, 3 * D2, r->stream);
-    launch_fill_u32(r->claims, 0u, D2 * EXTEND_CLAIM_WORDS, r->stream);
+    launch_fill_u32(r->claims, 0u, D2 * 2 * CLAIM_WORDS, r->stream);
     // the camera rays are stored only for the kernels that load them: k_extend and k_march at depth 0 and
     // k_shade_mode (k_extend_packet and the first k_shade compute them)
     fp.rays_stored = fp.mode != RAYNA_MODE_PBR || r->dev.view.n_sdfs > 0 ||
@@ -382,12 +380,12 @@ void trace_chunk(rayna_renderer *r, FrameParams &fp, uint32_t s0, uint32_t n, st
         int32_t *qout = r->queue[(depth + 1) & 1];
         uint32_t *cout = r->queue_count + depth + 1;
         if (ev) (void)hipEventRecord((*ev)[(*evi)++], r->stream);
-        uint32_t *work = r->claims + (size_t)depth * EXTEND_CLAIM_WORDS;
+        uint32_t *work = r->claims + (size_t)depth * 2 * CLAIM_WORDS;
         launch_extend(r->dev.view, fp, r->pb, qin, cin, depth, r->grid_extend, r->dev.overflow, work, r->tune,
                       BatchView{}, r->stream);
         launch_march(r->dev.view, fp, r->pb, qin, cin, (uint32_t)r->dev.view.n_sdfs, r->mt, r->mt_cap,
-                     r->queue_count + 2 * D2 + depth, r->grid_march, r->grid_shade, r->tune, BatchView{},
-                     r->sdf_queue, r->sdf_count, r->stream);
+                     work + CLAIM_WORDS, r->grid_march, r->grid_shade, r->tune, BatchView{}, r->sdf_queue,
+                     r->queue_count + 2 * D2 + depth, r->stream);
         if (fp.mode != RAYNA_MODE_PBR) {  // render_px_once: the camera ray's hit coloured by the mode
             if (ev) (void)hipEventRecord((*ev)[(*evi)++], r->stream);
             launch_shade_mode(r->dev.view, fp, r->pb, r->grid_shade, r->stream);
@@ -882,14 +880,15 @@ rayna_status rayna_primary_hits(rayna_renderer *r, uint32_t sample_index, int32_
     pb.hit_rank = rank_dev;
     r->primal_frame = -1;
     launch_generate(fp, pb, BatchView{}, r->stream);
-    uint32_t *work = r->queue_count + 3 * (r->opts.ray_depth + 2);
-    uint32_t *claims = r->claims + (size_t)(r->opts.ray_depth + 2) * EXTEND_CLAIM_WORDS;
-    launch_fill_u32(work, 0u, 2, r->stream);
-    launch_fill_u32(claims, 0u, EXTEND_CLAIM_WORDS, r->stream);
+    uint32_t *sdf_count = r->queue_count + 3 * (r->opts.ray_depth + 2);
+    uint32_t *claims = r->claims + (size_t)(r->opts.ray_depth + 2) * 2 * CLAIM_WORDS;
+    launch_fill_u32(sdf_count, 0u, 1, r->stream);
+    launch_fill_u32(claims, 0u, 2 * CLAIM_WORDS, r->stream);
     launch_extend(r->dev.view, fp, pb, nullptr, nullptr, 0, r->grid_extend, r->dev.overflow, claims, r->tune,
                   BatchView{}, r->stream);
-    launch_march(r->dev.view, fp, pb, nullptr, nullptr, (uint32_t)r->dev.view.n_sdfs, r->mt, r->mt_cap, work + 1,
-                 r->grid_march, r->grid_shade, r->tune, BatchView{}, r->sdf_queue, r->sdf_count, r->stream);
+    launch_march(r->dev.view, fp, pb, nullptr, nullptr, (uint32_t)r->dev.view.n_sdfs, r->mt, r->mt_cap,
+                 claims + CLAIM_WORDS, r->grid_march, r->grid_shade, r->tune, BatchView{}, r->sdf_queue, sdf_count,
+                 r->stream);
     rayna_status ls = launch_status(r, "primary_hits");
     hipError_t e = hipSuccess;
     if (ls == RAYNA_OK) e = hipMemcpyAsync(prim_rank, rank_dev, (size_t)P * 4, hipMemcpyDeviceToHost, r->stream);

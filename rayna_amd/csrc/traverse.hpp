@@ -286,6 +286,11 @@ constexpr uint32_t EXTEND_INNER_EXIT = 8;
 // back from speculation (below) left it at 32.6.
 constexpr uint32_t EXTEND_PRIM_EXIT = 16;
 
+// Fewest queue positions a wave claims: below 4 * 7000 paths the launch runs on fewer waves instead of on waves of one
+// or two lanes.  (Four 641x359, 1-sample mesh frames at 32, 16, 8 and 4: 5.89, 5.79, 5.62 and 5.39 ms; the 64x36,
+// 2-sample sphere frame 0.57, 0.58, 0.58, 0.53; larger frames within 1%.)
+constexpr uint32_t EXTEND_CLAIM_LEAST = 4;
+
 #ifndef RAYNA_EXT_WAVES
 #define RAYNA_EXT_WAVES 6
 #endif
@@ -299,7 +304,7 @@ __global__ __launch_bounds__(EXT_BLOCK) __attribute__((amdgpu_waves_per_eu(
     int2 *overflow, uint32_t *work, ExtendTuning tune, BatchView bv) {
     __shared__ unsigned long long s_entry[EXT_LDS_STACK * EXT_BLOCK];
     const uint32_t count = queue ? *count_ptr : fp.n_slots;
-    const uint32_t refill_lanes = tune.refill_lanes, wave_batch = tune.wave_batch;
+    const uint32_t refill_lanes = tune.refill_lanes;
     dm::Key key{fp.key0, fp.key1};
     const uint32_t gid = blockIdx.x * EXT_BLOCK + threadIdx.x;
     const uint32_t lane = __lane_id();
@@ -311,42 +316,17 @@ __global__ __launch_bounds__(EXT_BLOCK) __attribute__((amdgpu_waves_per_eu(
     int32_t leaf = 0;
     int leaf_i = 0, leaf_n = 0;
     float leaf_t = 0.0f;
-    // The wave's unhanded queue positions [batch_next, batch_end): claimed wave_batch at a time with one atomic,
-    // handed to idle lanes without further atomics.  (All of these are wave-uniform.)  The queue is cut into
-    // EXTEND_PARTS contiguous parts with a counter each; a wave starts on part blockIdx.x % EXTEND_PARTS and moves
-    // to the next part when its own is used up.  Workgroups go to the eight XCDs in turn, so each part (a band
-    // of neighbouring pixels) is worked through by two XCDs, whose L2s then hold its nodes, and no single
-    // counter takes every claim of the launch (four parts measured 1% faster than one or eight).
+    // The wave's unhanded queue positions [batch_next, batch_end), handed to idle lanes without atomics; wave-uniform.
     uint32_t batch_next = 0, batch_end = 0;
-    uint32_t part = blockIdx.x % EXTEND_PARTS, parts_done = 0;
-    auto part_bound = [&](uint32_t p) { return (uint32_t)(((uint64_t)count * p) / EXTEND_PARTS); };
+    WaveClaims claims(count, EXT_BLOCK / 64, EXTEND_CLAIM_LEAST, tune.wave_batch, work);
     RAYNA_STAT_DECL();
-    bool last_claim = false;  // every part is used up: no further claims will yield work
     for (;;) {
         const unsigned long long idle = __ballot(!active);
         if (!exhausted && (idle == ~0ull || (uint32_t)__popcll(idle) >= refill_lanes)) {
             const uint32_t n = (uint32_t)__popcll(idle);
             const uint32_t r = batch_end - batch_next;  // old positions, handed out first
             uint32_t nb = 0, nb_end = 0;                // new batch [nb, nb_end)
-            if (r < n && !last_claim) {
-                const int leader = __ffsll((long long)idle) - 1;
-                for (;;) {
-                    const uint32_t lo = part_bound(part), hi = part_bound(part + 1);
-                    uint32_t base = 0;
-                    if ((int)lane == leader) base = atomicAdd(work + 32 * part, wave_batch);
-                    base = __shfl(base, leader);
-                    const bool got = base < hi - lo;
-                    if (got) {
-                        nb = lo + base;
-                        nb_end = (hi - nb > wave_batch) ? nb + wave_batch : hi;
-                    }
-                    if (!got || nb_end == hi) {  // this part is used up
-                        part = part + 1 == EXTEND_PARTS ? 0 : part + 1;
-                        if (++parts_done == EXTEND_PARTS) last_claim = true;
-                    }
-                    if (got || last_claim) break;
-                }
-            }
+            if (r < n && !claims.last) claims.take(__ffsll((long long)idle) - 1, &nb, &nb_end);
             const uint32_t idx = (uint32_t)__popcll(idle & ((1ull << lane) - 1ull));  // rank among idle lanes
             uint32_t q = 0xffffffffu;
             if (idx < r) q = batch_next + idx;
@@ -358,7 +338,7 @@ __global__ __launch_bounds__(EXT_BLOCK) __attribute__((amdgpu_waves_per_eu(
                 batch_next = nb + from_new;
                 batch_end = nb_end;
             }
-            if (last_claim && batch_next == batch_end) exhausted = true;
+            if (claims.last && batch_next == batch_end) exhausted = true;
             if (!active) {
                 if (q != 0xffffffffu) {
                     slot = queue ? (uint32_t)queue[q] : q;
