@@ -272,13 +272,14 @@ typedef struct rayna_render_opts {
 typedef struct rayna_render_stats {
     double duration_s;       /* host wall time of the render call */
     double kernel_ms;        /* sum of device time of all kernels of the frame (HIP events) */
-    double extend_ms;        /* device time of the extend (closest-hit) kernels */
-    double shade_ms;         /* device time of the shade kernels */
+    double extend_ms;        /* device time of the closest-hit kernels, and of the launch that traces and shades
+                                whole paths */
+    double shade_ms;         /* device time of the other shade kernels */
     uint64_t accum_frames;   /* frames in the accumulation buffer, as AccumulationBuffer::frame_count */
     uint64_t samples;        /* camera samples traced this frame (width * height * samples) */
     uint64_t segments;       /* closest-hit queries this frame (one per path vertex) */
-    uint64_t extend_launches;
-    double extend_camera_ms; /* of extend_ms: the launches for the camera rays (depth 0) */
+    uint64_t extend_launches; /* closest-hit passes: one per chunk and depth */
+    double extend_camera_ms; /* of extend_ms: the launches for the camera rays alone (depth 0) */
 } rayna_render_stats;
 
 /* Output layouts of rayna_render. */

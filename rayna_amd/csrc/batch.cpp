@@ -76,7 +76,9 @@ struct Pipeline {
     int32_t *queue[2] = {nullptr, nullptr};
     uint32_t *queue_count = nullptr;
     uint32_t queue_count_len = 0;
-    uint32_t *claims = nullptr;    // claim counters, CLAIM_WORDS for k_extend and for k_march per depth
+    // SEGMENT_WORDS of k_trace's query counters, then claim counters: CLAIM_WORDS for k_extend (or k_trace) and for
+    // k_march per depth
+    uint32_t *claims = nullptr;
     unsigned long long *segments = nullptr;
     float *mt = nullptr;           // march outcomes, 2 * capacity * n_sdf_max
     int32_t *sdf_queue = nullptr;  // scenes with unbounded objects: SDF-hit slots (normals in pb.sdf_n*)
@@ -205,7 +207,7 @@ rayna_status alloc_pipe(rayna_batch *b, int p, uint64_t slots, uint32_t max_dept
     // [0, D+2) paths entering each depth; [2(D+2), 3(D+2)) SDF hits at each depth
     const uint32_t qlen = 3 * (std::max<uint32_t>(max_depth, 16) + 2);
     if ((st = alloc(qlen * sizeof(uint32_t), (void **)&P.queue_count)) != RAYNA_OK) return st;
-    if ((st = alloc((size_t)(qlen / 3) * 2 * CLAIM_WORDS * sizeof(uint32_t), (void **)&P.claims)) != RAYNA_OK)
+    if ((st = alloc((SEGMENT_WORDS + (size_t)(qlen / 3) * 2 * CLAIM_WORDS) * sizeof(uint32_t), (void **)&P.claims)) != RAYNA_OK)
         return st;
     if ((st = alloc(sizeof(unsigned long long), (void **)&P.segments)) != RAYNA_OK) return st;
     if (b->n_sdf_max) {
@@ -423,11 +425,17 @@ SceneView chunk_view(const SceneView &merged, uint32_t features) {
 }
 
 // Launches of a plan traced on `used` pipelines.
-uint32_t plan_launches(const Plan &pl, int used) {
+uint32_t plan_launches(const rayna_batch *b, const Plan &pl, int used) {
     uint32_t n = (uint32_t)used;  // segment counters
     for (size_t c = 0; c < pl.chunks.size(); ++c) {
+        const SceneView cv = chunk_view(b->view, pl.features[c]);
+        const BatchView bv{b->table, (uint32_t)pl.chunks[c].size(), nullptr};
+        FrameParams fp{};
+        fp.n_slots = pl.slots[c];
+        const uint32_t depths = pl.depth[c] + 1, apart = std::min(depths, launched_depths(cv, fp, b->tune, bv));
         const uint32_t nf = pl.first_final[c + 1] - pl.first_final[c];
-        n += 3 + (pl.n_sdf[c] ? 6 : 2) * (pl.depth[c] + 1) + 2 + (nf ? 1 : 0);
+        const uint32_t traced = (pl.n_sdf[c] ? 5 : 2) * apart + (apart < depths ? 1 : 0);
+        n += 3 + traced + 2 + (nf ? 1 : 0);
     }
     return n;
 }
@@ -460,24 +468,31 @@ hipError_t enqueue(rayna_batch *b, const Plan &pl, int used, bool timing) {
         const uint32_t D = pl.depth[c];
         const SceneView cv = chunk_view(b->view, pl.features[c]);
         launch_fill_u32(P.queue_count, 0u, 3 * (D + 2), s);
-        launch_fill_u32(P.claims, 0u, (D + 1) * 2 * CLAIM_WORDS, s);
+        launch_fill_u32(P.claims, 0u, SEGMENT_WORDS + (D + 1) * 2 * CLAIM_WORDS, s);
+        uint32_t *claims = P.claims + SEGMENT_WORDS;
+        const uint32_t apart = std::min(D + 1, launched_depths(cv, fp, b->tune, bv));
         // the camera rays are stored only where a kernel loads them: k_extend and k_march at depth 0 (the camera-ray
-        // packets and the first k_shade compute them); k_generate records every slot's request either way
-        fp.rays_stored = (pl.features[c] & SCENE_SDFS) != 0u || !extend_packets(cv, fp, b->tune, bv, 0);
+        // packets, k_trace and the first k_shade compute them); k_generate records every slot's request either way
+        fp.rays_stored = apart > 0 && ((pl.features[c] & SCENE_SDFS) != 0u || !extend_packets(cv, fp, b->tune, bv, 0));
         launch_generate(fp, P.pb, bv, s);
         for (uint32_t depth = 0; depth <= D; ++depth) {
             const int32_t *qin = depth == 0 ? nullptr : P.queue[depth & 1];
             const uint32_t *cin = depth == 0 ? nullptr : P.queue_count + depth;
             int32_t *qout = P.queue[(depth + 1) & 1];
             uint32_t *cout = P.queue_count + depth + 1;
-            uint32_t *work = P.claims + (size_t)depth * 2 * CLAIM_WORDS;
+            uint32_t *work = claims + (size_t)depth * 2 * CLAIM_WORDS;
+            if (depth >= apart) {  // every path to its end
+                launch_trace(cv, fp, P.pb, qin, cin, depth, b->grid_extend, P.overflow, work, P.claims, b->tune,
+                             nullptr, bv, s);
+                break;
+            }
             launch_extend(cv, fp, P.pb, qin, cin, depth, b->grid_extend, P.overflow, work, b->tune, bv, s);
             launch_march(cv, fp, P.pb, qin, cin, pl.n_sdf[c], P.mt, P.capacity * b->n_sdf_max,
                          work + CLAIM_WORDS, b->grid_march, b->grid_shade, b->tune, bv, P.sdf_queue,
                          P.queue_count + 2 * (D + 2) + depth, s);
             launch_shade(cv, fp, P.pb, qin, cin, qout, cout, depth, b->grid_shade, nullptr, bv, s);
         }
-        launch_count_segments(P.queue_count, D + 1, fp.n_slots, P.segments, s);
+        launch_count_segments(P.queue_count, apart, apart > 0 ? fp.n_slots : 0, P.claims, P.segments, s);
         // (a dependency on the same pipeline is kept by its stream's order)
         if (used > 1 && pl.dep[c] >= 0 && (size_t)pl.dep[c] % used != c % used)
             check(hipStreamWaitEvent(s, b->resolved[pl.dep[c]], 0));
@@ -595,6 +610,7 @@ rayna_status rayna_batch_create(const rayna_scene_desc *scenes, int32_t n_scenes
     for (const SceneSlot &sl : b->slots) b->n_sdf_max = std::max<uint32_t>(b->n_sdf_max, (uint32_t)sl.n_sdfs);
     clamp_chunk(b);
     v.root = -1;  // per request
+    v.n_nodes = (int32_t)merged.nodes.size();
     v.n_sdfs = (int32_t)merged.sdfs.size();
     v.skybox = RAYNA_SKY_NONE;
     v.stack_need = merged.stack_need;
@@ -688,7 +704,7 @@ rayna_status rayna_render_batch(rayna_batch *b, const rayna_request *reqs, int32
         BHIP(b, hipEventCreateWithFlags(&e, hipEventDisableTiming));
         b->resolved.push_back(e);
     }
-    const uint32_t launches = plan_launches(pl, used);
+    const uint32_t launches = plan_launches(b, pl, used);
     if (graph) {
         const uint64_t key = mix(pl.key, (uint64_t)used);
         if (!b->graph_exec || b->graph_key != key) {

@@ -984,6 +984,72 @@ __device__ __forceinline__ void grad_add(const AdjointParams &ap, uint32_t copy,
     unsafeAtomicAdd(p + 2, g2);
 }
 
+// One vertex of a path, shaded: the radiance it adds (`add`: a light's or the sky's, times the throughput T), and its
+// scatter.  True if the path goes on (the depth limit not reached, the material scattered): go_on has then taken its
+// next ray and throughput.  ref == 0: the ray missed.  sdf_hit: the hit's SDF normal is given as sdf_n.
+//
+// ADJOINT: the replay step of path replay backpropagation instead (see k_shade): nothing is added, L is the radiance
+// the path still gathers from this vertex on, and gradients go to copy `copy` of ap.
+template <bool ADJOINT, bool TEX, bool VALIDATE, bool SDF, class GoOn>
+__device__ __forceinline__ bool shade_vertex(const SceneView &sv, uint32_t *checks, const AdjointParams &ap,
+                                             uint32_t copy, const DRay &ray, uint32_t ref, const float *hit_t,
+                                             const uint32_t *hit_aux, const uint32_t *sub, bool sdf_hit, f3 sdf_n, const dm::Key &key,
+                                             uint32_t pixel, uint32_t sample, uint32_t depth, uint32_t ray_depth,
+                                             int32_t skybox, int32_t sky_img, Col T, Col &L, Col &add, GoOn go_on) {
+    if (ref == 0u) {
+        if (!ADJOINT)
+            add = T * ((TEX && skybox == RAYNA_SKY_HDRI) ? sky_image(sv, sky_img, ray.d) : sky(skybox, ray.d));
+        if (VALIDATE && !colour_ok(add)) count_check(checks, RAYNA_CHECK_COLOUR);
+        return false;
+    }
+    const float t = *hit_t;
+    const uint32_t aux = *hit_aux;
+    SHit h;
+    hit_geometry<SDF>(sv, ray, t, ref, aux, sub, key, pixel, sample, depth, &h, sdf_hit, sdf_n);
+    if (VALIDATE) {
+        float uv[2];
+        int side;
+        hit_uv_side(sv, ray, t, ref, aux, sub, key, pixel, sample, depth, uv, &side);
+        validate_hit(checks, ray, t, h, uv);
+    }
+    const GMaterial m = sv.materials[h.material];
+    const Col colour = material_colour<TEX>(sv, m, ray, t, ref, aux, sub, key, pixel, sample, depth, h);
+    if (VALIDATE && !colour_ok(colour)) count_check(checks, RAYNA_CHECK_COLOUR);
+    const bool graded = !TEX || m.texture < 0;
+    double d0 = 0.0, d1 = 0.0, d2 = 0.0;
+    if (ADJOINT) {
+        d0 = (double)ap.d_image[3 * pixel] * ap.inv_spp;
+        d1 = (double)ap.d_image[3 * pixel + 1] * ap.inv_spp;
+        d2 = (double)ap.d_image[3 * pixel + 2] * ap.inv_spp;
+    }
+    if (m.kind == RAYNA_MAT_LIGHT) {
+        const Col le = colour;
+        if (ADJOINT) {
+            if (graded) grad_add(ap, copy, h.material, d0 * T.r, d1 * T.g, d2 * T.b);
+            L = Col{L.r - T.r * le.r, L.g - T.g * le.g, L.b - T.b * le.b};
+        } else {
+            add = T * le;
+            if (VALIDATE && !colour_ok(add)) count_check(checks, RAYNA_CHECK_COLOUR);
+        }
+    }
+    float u[4];
+    dm::draw4(key, pixel, sample, depth, dm::SLOT_SCATTER, u);
+    f3 dir;
+    if (!scatter(m, ray, h, u, &dir)) return false;
+    if (ADJOINT && depth < ray_depth) {
+        const bool albedo_scales = m.kind != RAYNA_MAT_DIELECTRIC || !h.front;
+        if (albedo_scales && graded)
+            grad_add(ap, copy, h.material, m.r != 0.0f ? d0 * (double)L.r / (double)m.r : 0.0,
+                     m.g != 0.0f ? d1 * (double)L.g / (double)m.g : 0.0,
+                     m.b != 0.0f ? d2 * (double)L.b / (double)m.b : 0.0);
+    }
+    T = reflected(m, ray, h, colour, T);
+    if (VALIDATE && !colour_ok(T)) count_check(checks, RAYNA_CHECK_COLOUR);
+    if (depth >= ray_depth) return false;
+    go_on(make_ray(h.pos, dir), T);
+    return true;
+}
+
 // One bounce of ray_colour_recursive in forward form: L += T * Le; scatter; T = reflected(T); paths that
 // scatter below the depth limit are compacted into the next queue (one atomic per wave).
 //
@@ -1079,74 +1145,25 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(
             // 0 + add, and an exact cancellation rounds to +0).
             Col add{0.0f, 0.0f, 0.0f};
             if (ADJOINT) L = Col{pb.lr[slot], pb.lg[slot], pb.lb[slot]};
-            if (ref == 0u) {
-                if (!ADJOINT)
-                    add = T * ((TEX && skybox == RAYNA_SKY_HDRI) ? sky_image(sv, sky_img, ray.d) : sky(skybox, ray.d));
-                if (VALIDATE && !colour_ok(add)) count_check(fp.checks, RAYNA_CHECK_COLOUR);
-            } else {
-                SHit h;
-                const float t = pb.hit_t[slot];
-                const uint32_t aux = pb.hit_aux[slot];
-                f3 sdf_n{0.0f, 0.0f, 0.0f};
-                const bool sdf_hit = (ref >> HIT_KIND_SHIFT) == (uint32_t)ITEM_SDF && pb.sdf_nx;
+            f3 sdf_n{0.0f, 0.0f, 0.0f};
+            bool sdf_hit = false;
+            if (!WIDE) {
+                sdf_hit = (ref >> HIT_KIND_SHIFT) == (uint32_t)ITEM_SDF && pb.sdf_nx;
                 if (sdf_hit) sdf_n = f3{pb.sdf_nx[slot], pb.sdf_ny[slot], pb.sdf_nz[slot]};
-                hit_geometry<!WIDE>(sv, ray, t, ref, aux, pb.hit_sub + slot, key, pixel, sample, depth, &h, sdf_hit,
-                                    sdf_n);
-                if (VALIDATE) {
-                    float uv[2];
-                    int side;
-                    hit_uv_side(sv, ray, t, ref, aux, pb.hit_sub + slot, key, pixel, sample, depth, uv, &side);
-                    validate_hit(fp.checks, ray, t, h, uv);
-                }
-                const GMaterial m = sv.materials[h.material];
-                const Col colour =
-                    material_colour<TEX>(sv, m, ray, t, ref, aux, pb.hit_sub + slot, key, pixel, sample, depth, h);
-                if (VALIDATE && !colour_ok(colour)) count_check(fp.checks, RAYNA_CHECK_COLOUR);
-                const bool graded = !TEX || m.texture < 0;
-                double d0 = 0.0, d1 = 0.0, d2 = 0.0;
-                if (ADJOINT) {
-                    d0 = (double)ap.d_image[3 * pixel] * ap.inv_spp;
-                    d1 = (double)ap.d_image[3 * pixel + 1] * ap.inv_spp;
-                    d2 = (double)ap.d_image[3 * pixel + 2] * ap.inv_spp;
-                }
-                if (m.kind == RAYNA_MAT_LIGHT) {
-                    const Col le = colour;
-                    if (ADJOINT) {
-                        if (graded) grad_add(ap, copy, h.material, d0 * T.r, d1 * T.g, d2 * T.b);
-                        L = Col{L.r - T.r * le.r, L.g - T.g * le.g, L.b - T.b * le.b};
-                    } else {
-                        add = T * le;
-                        if (VALIDATE && !colour_ok(add)) count_check(fp.checks, RAYNA_CHECK_COLOUR);
-                    }
-                }
-                float u[4];
-                dm::draw4(key, pixel, sample, depth, dm::SLOT_SCATTER, u);
-                f3 dir;
-                if (scatter(m, ray, h, u, &dir)) {
-                    if (ADJOINT && depth < ray_depth) {
-                        const bool albedo_scales = m.kind != RAYNA_MAT_DIELECTRIC || !h.front;
-                        if (albedo_scales && graded)
-                            grad_add(ap, copy, h.material, m.r != 0.0f ? d0 * (double)L.r / (double)m.r : 0.0,
-                                     m.g != 0.0f ? d1 * (double)L.g / (double)m.g : 0.0,
-                                     m.b != 0.0f ? d2 * (double)L.b / (double)m.b : 0.0);
-                    }
-                    T = reflected(m, ray, h, colour, T);
-                    if (VALIDATE && !colour_ok(T)) count_check(fp.checks, RAYNA_CHECK_COLOUR);
-                    if (depth < ray_depth) {
-                        const DRay nr = make_ray(h.pos, dir);
-                        pb.ox[slot] = nr.o.x;
-                        pb.oy[slot] = nr.o.y;
-                        pb.oz[slot] = nr.o.z;
-                        pb.dx[slot] = nr.d.x;
-                        pb.dy[slot] = nr.d.y;
-                        pb.dz[slot] = nr.d.z;
-                        pb.tr[slot] = T.r;
-                        pb.tg[slot] = T.g;
-                        pb.tb[slot] = T.b;
-                        keep = true;
-                    }
-                }
             }
+            keep = shade_vertex<ADJOINT, TEX, VALIDATE, !WIDE>(
+                sv, fp.checks, ap, copy, ray, ref, pb.hit_t + slot, pb.hit_aux + slot, pb.hit_sub + slot, sdf_hit, sdf_n,
+                key, pixel, sample, depth, ray_depth, skybox, sky_img, T, L, add, [&](const DRay &nr, const Col &t) {
+                    pb.ox[slot] = nr.o.x;
+                    pb.oy[slot] = nr.o.y;
+                    pb.oz[slot] = nr.o.z;
+                    pb.dx[slot] = nr.d.x;
+                    pb.dy[slot] = nr.d.y;
+                    pb.dz[slot] = nr.d.z;
+                    pb.tr[slot] = t.r;
+                    pb.tg[slot] = t.g;
+                    pb.tb[slot] = t.b;
+                });
             const bool adds = !(add.r == 0.0f && add.g == 0.0f && add.b == 0.0f);
             if (!ADJOINT && queue_in && (adds || VALIDATE)) L = Col{pb.lr[slot], pb.lg[slot], pb.lb[slot]};
             if (!ADJOINT) L = L + add;
@@ -1164,6 +1181,8 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(
       append_strip(mine, n_kept, kept, &strip_base, queue_out, count_out);
     }
 }
+
+#include "trace.hpp"
 
 // Sum of the gradient copies: out[i] = sum over copies of grad[copy * n + i], n = 3 * materials.
 __global__ __launch_bounds__(BLOCK) void k_sum_grad(const double *grad, uint32_t n, uint32_t copies, double *out) {
@@ -1388,18 +1407,33 @@ __global__ __launch_bounds__(BLOCK) void k_sqrt_check(uint32_t first, uint32_t c
     if (bad) atomicAdd(mismatches, (unsigned long long)bad);
 }
 
-__global__ void k_count_segments(const uint32_t *queue_count, uint32_t n, uint32_t first_count,
+// Adds a chunk's closest-hit queries to *segments: first_count, the lengths of queues 1 to n - 1, and what k_trace
+// counted.  One wave.
+__global__ void k_count_segments(const uint32_t *queue_count, uint32_t n, uint32_t first_count, const uint32_t *parts,
                                  unsigned long long *segments) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        unsigned long long s = first_count;
-        for (uint32_t i = 1; i < n; ++i) s += queue_count[i];
-        *segments += s;
-    }
+    unsigned long long s = 0;
+    for (uint32_t i = 1 + threadIdx.x; i < n; i += 64) s += queue_count[i];
+    for (uint32_t i = threadIdx.x; i < SEGMENT_PARTS; i += 64) s += parts[32 * i];
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+    if (threadIdx.x == 0) *segments += s + first_count;
 }
 
 inline unsigned grid_for(uint64_t n, int block) { return (unsigned)((n + block - 1) / block); }
 
 }  // namespace
+
+using TraceKernel = void (*)(SceneView, FrameParams, PathBuffers, const int32_t *, const uint32_t *, uint32_t, int2 *,
+                             uint32_t *, uint32_t *, ExtendTuning, AdjointParams, BatchView);
+// The k_trace instantiations, [batch, adjoint, neither][textures][instances][form], forms as EXTEND_KERNELS'.
+#define RAYNA_TRACE_FORMS(B, T, I, A)                                                                   \
+    {k_trace<B, I, false, false, T, A>, k_trace<B, I, true, false, T, A>, k_trace<B, I, true, true, T, A>}
+#define RAYNA_TRACE_SET(B, A)                                                                            \
+    {{RAYNA_TRACE_FORMS(B, false, false, A), RAYNA_TRACE_FORMS(B, false, true, A)},                      \
+     {RAYNA_TRACE_FORMS(B, true, false, A), RAYNA_TRACE_FORMS(B, true, true, A)}}
+const TraceKernel TRACE_KERNELS[3][2][2][3] = {RAYNA_TRACE_SET(false, false), RAYNA_TRACE_SET(true, false),
+                                               RAYNA_TRACE_SET(false, true)};
+#undef RAYNA_TRACE_SET
+#undef RAYNA_TRACE_FORMS
 
 using ExtendKernel = void (*)(SceneView, FrameParams, PathBuffers, const int32_t *, const uint32_t *, uint32_t,
                               int2 *, uint32_t *, ExtendTuning, BatchView);
@@ -1416,35 +1450,35 @@ int extend_form(const SceneView &sv) { return sv.media ? 2 : (sv.sphere_tests ? 
 // Resident 128-lane blocks per CU of each instantiation, taken once per process.
 struct ExtendOccupancy {
     int n[2][2][3];
+    int trace[3][2][2][3];
+    int most;
 };
+template <class Kernel>
+int resident_blocks(Kernel kernel) {
+    int n = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, EXT_BLOCK, 0) != hipSuccess || n < 1) n = 4;
+    return n;
+}
 const ExtendOccupancy &extend_occupancy() {
     static ExtendOccupancy o;
     static std::once_flag once;
     std::call_once(once, [] {
-        for (int b = 0; b < 2; ++b)
-            for (int i = 0; i < 2; ++i)
-                for (int f = 0; f < 3; ++f) {
-                    int n = 0;
-                    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, EXTEND_KERNELS[b][i][f], EXT_BLOCK, 0) !=
-                            hipSuccess ||
-                        n < 1)
-                        n = 4;
-                    o.n[b][i][f] = n;
-                }
+        o.most = 1;
+        for (int i = 0; i < 2; ++i)
+            for (int f = 0; f < 3; ++f) {
+                for (int b = 0; b < 2; ++b)
+                    o.most = std::max(o.most, o.n[b][i][f] = resident_blocks(EXTEND_KERNELS[b][i][f]));
+                for (int k = 0; k < 3; ++k)
+                    for (int t = 0; t < 2; ++t)
+                        o.most = std::max(o.most, o.trace[k][t][i][f] = resident_blocks(TRACE_KERNELS[k][t][i][f]));
+            }
     });
     return o;
 }
 
 int extend_lds_stack() { return EXT_LDS_STACK; }
 
-int extend_blocks_per_cu() {
-    const ExtendOccupancy &o = extend_occupancy();
-    int n = 1;
-    for (int b = 0; b < 2; ++b)
-        for (int i = 0; i < 2; ++i)
-            for (int f = 0; f < 3; ++f) n = std::max(n, o.n[b][i][f]);
-    return n;
-}
+int extend_blocks_per_cu() { return extend_occupancy().most; }
 int extend_block() { return EXT_BLOCK; }
 
 int march_blocks_per_cu() {
@@ -1491,6 +1525,24 @@ void launch_extend(const SceneView &sv, const FrameParams &fp, const PathBuffers
     const int g = std::max(1, std::min(grid, std::max(1, grid / extend_blocks_per_cu()) * extend_occupancy().n[b][i][f]));
     hipLaunchKernelGGL(EXTEND_KERNELS[b][i][f], dim3(g), dim3(EXT_BLOCK), 0, s, sv, fp, pb, queue, count, depth,
                        overflow, work, tune, bv);
+}
+
+uint32_t launched_depths(const SceneView &sv, const FrameParams &fp, const ExtendTuning &tune, const BatchView &bv) {
+    if (fp.mode != RAYNA_MODE_PBR || sv.n_sdfs > 0 || fp.checks) return 0xffffffffu;
+    if (!extend_packets(sv, fp, tune, bv, 0)) return 0;
+    const uint32_t n = fp.n_slots >= FIRST_BOUNCE_SLOTS && sv.n_nodes >= FIRST_BOUNCE_NODES ? 2 : 1;
+    return std::max(n, tune.packet_depths);
+}
+
+void launch_trace(const SceneView &sv, const FrameParams &fp, const PathBuffers &pb, const int32_t *queue,
+                  const uint32_t *count, uint32_t first_depth, int grid, int2 *overflow, uint32_t *work,
+                  uint32_t *segments, const ExtendTuning &tune, const AdjointParams *adjoint, const BatchView &bv,
+                  hipStream_t s) {
+    const int k = bv.reqs ? 1 : adjoint ? 2 : 0, t = sv.textured ? 1 : 0, i = sv.instances ? 1 : 0;
+    const int f = extend_form(sv);
+    const int g = std::max(1, std::min(grid, grid / extend_blocks_per_cu() * extend_occupancy().trace[k][t][i][f]));
+    hipLaunchKernelGGL(TRACE_KERNELS[k][t][i][f], dim3(g), dim3(EXT_BLOCK), 0, s, sv, fp, pb, queue, count,
+                       first_depth, overflow, work, segments, tune, adjoint ? *adjoint : AdjointParams{}, bv);
 }
 
 void launch_shade(const SceneView &sv, const FrameParams &fp, const PathBuffers &pb, const int32_t *queue_in,
@@ -1577,9 +1629,9 @@ uint64_t launch_valu_peak(float *out, uint32_t blocks, uint32_t iters, hipStream
     return (uint64_t)blocks * (BLOCK / 64) * iters * (2 * VALU_PEAK_CHAINS);
 }
 
-void launch_count_segments(const uint32_t *queue_count, uint32_t n, uint32_t first_count,
+void launch_count_segments(const uint32_t *queue_count, uint32_t n, uint32_t first_count, const uint32_t *parts,
                            unsigned long long *segments, hipStream_t s) {
-    hipLaunchKernelGGL(k_count_segments, dim3(1), dim3(64), 0, s, queue_count, n, first_count, segments);
+    hipLaunchKernelGGL(k_count_segments, dim3(1), dim3(64), 0, s, queue_count, n, first_count, parts, segments);
 }
 
 // ------------------------------------------------------------------------------------------ static workspace

@@ -95,12 +95,33 @@ void launch_generate(const FrameParams &fp, const PathBuffers &pb, const BatchVi
 constexpr uint32_t CLAIM_PARTS = RAYNA_CLAIM_PARTS;
 constexpr uint32_t CLAIM_WORDS = CLAIM_PARTS * 32;
 
+// k_trace's counters of closest-hit queries, one 128-byte line apart.
+constexpr uint32_t SEGMENT_PARTS = 64;
+constexpr uint32_t SEGMENT_WORDS = SEGMENT_PARTS * 32;
+
 // queue == nullptr: identity queue of fp.n_slots entries; else queue[0 .. *count)
 // overflow: traversal stack entries beyond the LDS part, extend_block() * grid * (stack_need - extend_lds_stack());
 // work: CLAIM_WORDS zeroed words, the counters the launch's waves take rays from
 void launch_extend(const SceneView &sv, const FrameParams &fp, const PathBuffers &pb, const int32_t *queue,
                    const uint32_t *count, uint32_t depth, int grid, int2 *overflow, uint32_t *work,
                    const ExtendTuning &tune, const BatchView &bv, hipStream_t s);
+// How many of a chunk's depths, from the camera rays on, get a launch of extend and one of shade each; the paths that
+// are left go to their ends in one launch (launch_trace).  All depths (2^32 - 1) for the non-PBR modes, scenes with
+// unbounded objects (the march is a pass of its own over all paths) and validation.  Otherwise the camera rays where
+// they are traced as packets, and for a large chunk over a tree that is not small the first bounce too: its rays start
+// from one point per wave, which k_extend's seven waves per SIMD use better than k_trace's mix of depths.  (1080p, 64
+// samples, first bounce apart against not: 45.6 and 48.6 ms with 1.3 M triangles, 34.6 and 36.5 with 1290, 28.2 and
+// 28.3 with 480 spheres, 27.3 and 25.9 in the Cornell box; at 640x360x64, 8.04 and 7.99 ms with 1.3 M triangles.)
+constexpr uint32_t FIRST_BOUNCE_SLOTS = 1u << 24;
+constexpr int32_t FIRST_BOUNCE_NODES = 256;
+uint32_t launched_depths(const SceneView &sv, const FrameParams &fp, const ExtendTuning &tune, const BatchView &bv);
+// first_depth 0: every slot's path from its camera ray; first_depth > 0: the paths launch_shade kept at the depth before.
+// The radiance field holds each path's radiance at the end.  overflow and work as for launch_extend; segments:
+// SEGMENT_WORDS zeroed words, the closest-hit queries (launch_count_segments).
+void launch_trace(const SceneView &sv, const FrameParams &fp, const PathBuffers &pb, const int32_t *queue,
+                  const uint32_t *count, uint32_t first_depth, int grid, int2 *overflow, uint32_t *work,
+                  uint32_t *segments, const ExtendTuning &tune, const AdjointParams *adjoint, const BatchView &bv,
+                  hipStream_t s);
 void launch_shade(const SceneView &sv, const FrameParams &fp, const PathBuffers &pb, const int32_t *queue_in,
                   const uint32_t *count_in, int32_t *queue_out, uint32_t *count_out, uint32_t depth, int grid,
                   const AdjointParams *adjoint, const BatchView &bv, hipStream_t s);
@@ -146,7 +167,7 @@ bool extend_packets(const SceneView &sv, const FrameParams &fp, const ExtendTuni
 // the wave64 VALU instructions its chains issue (loop and set-up instructions not counted).
 uint64_t launch_valu_peak(float *out, uint32_t blocks, uint32_t iters, hipStream_t s);
 void launch_sqrt_check(uint32_t first, uint32_t count, unsigned long long *mismatches, uint32_t blocks, hipStream_t s);
-void launch_count_segments(const uint32_t *queue_count, uint32_t n, uint32_t first_count,
+void launch_count_segments(const uint32_t *queue_count, uint32_t n, uint32_t first_count, const uint32_t *parts,
                            unsigned long long *segments, hipStream_t s);
 
 // The static workspace of rayna_adjoint_static (a file-scope device array of adjoint_scratch_doubles()

@@ -203,6 +203,7 @@ struct SceneView {
     const float *texels;
     const int32_t *perms;
     int32_t root;        // -1: no bounded object
+    int32_t n_nodes;
     int32_t n_sdfs;
     int32_t skybox;
     int32_t stack_need;   // deepest per-lane stack k_extend can need (speculative traversal)

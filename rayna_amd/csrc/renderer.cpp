@@ -55,7 +55,9 @@ struct rayna_renderer {
     PathBuffers pb{};
     int32_t *queue[2] = {nullptr, nullptr};
     uint32_t *queue_count = nullptr;
-    uint32_t *claims = nullptr;  // claim counters: CLAIM_WORDS for k_extend and for k_march per depth, and for queries
+    // SEGMENT_WORDS of k_trace's query counters, then claim counters: CLAIM_WORDS for k_extend (or k_trace) and for
+    // k_march per depth, and for queries
+    uint32_t *claims = nullptr;
     unsigned long long *segments = nullptr;
     float *sum = nullptr, *acc = nullptr, *out_dev = nullptr;
     uint8_t *rgba_dev = nullptr;  // the 8-bit output of rayna_render_srgb8
@@ -83,6 +85,9 @@ struct rayna_renderer {
     uint64_t chunk_target = TARGET_SLOTS;
     ExtendTuning tune;
     std::vector<hipEvent_t> events;
+    // the last pass over a chunk: the event triples it recorded, and whether the first was of the camera rays alone
+    size_t pass_marks = 1;
+    bool camera_apart = true;
     // debug validation (shared/validate.rs): RAYNA_CHECKS counters, counted in PBR frames while `validate`
     uint32_t *checks = nullptr;
     // non-empty once a launch on this renderer failed (the failure's text): every later call is refused
@@ -188,6 +193,7 @@ rayna_status load_scene(rayna_renderer *r, const rayna_scene_desc *d) {
     UP(perms, perms)
 #undef UP
     v.root = ps.root;
+    v.n_nodes = (int32_t)ps.nodes.size();
     v.n_sdfs = (int32_t)ps.sdfs.size();
     v.skybox = ps.skybox;
     v.stack_need = ps.stack_need;
@@ -304,7 +310,8 @@ rayna_status alloc_paths(rayna_renderer *r) {
     for (int q = 0; q < 2; ++q)
         if ((st = alloc(slots * sizeof(int32_t), (void **)&r->queue[q])) != RAYNA_OK) return st;
     if ((st = alloc(qlen * sizeof(uint32_t), (void **)&r->queue_count)) != RAYNA_OK) return st;
-    if ((st = alloc((size_t)(o.ray_depth + 3) * 2 * CLAIM_WORDS * sizeof(uint32_t), (void **)&r->claims)) !=
+    if ((st = alloc((SEGMENT_WORDS + (size_t)(o.ray_depth + 3) * 2 * CLAIM_WORDS) * sizeof(uint32_t),
+                    (void **)&r->claims)) !=
         RAYNA_OK)
         return st;
     if ((st = alloc(sizeof(unsigned long long), (void **)&r->segments)) != RAYNA_OK) return st;
@@ -359,7 +366,7 @@ FrameParams frame_params(const rayna_renderer *r, uint64_t frame_index) {
     return fp;
 }
 
-// Trace the samples [s0, s0 + n) of every pixel: generate, then extend/shade per depth.  With `adjoint`, the
+// Trace the samples [s0, s0 + n) of every pixel: extend and shade per depth, from launched_depths on whole paths.  With `adjoint`, the
 // replay of path replay backpropagation: the radiance field must hold the chunk's primal radiance.
 void trace_chunk(rayna_renderer *r, FrameParams &fp, uint32_t s0, uint32_t n, std::vector<hipEvent_t> *ev, size_t *evi,
                  uint64_t *extend_launches, const AdjointParams *adjoint = nullptr) {
@@ -368,38 +375,49 @@ void trace_chunk(rayna_renderer *r, FrameParams &fp, uint32_t s0, uint32_t n, st
     fp.n_slots = fp.n_pixels * n;
     const uint32_t D2 = r->opts.ray_depth + 2;
     launch_fill_u32(r->queue_count, 0u, 3 * D2, r->stream);
-    launch_fill_u32(r->claims, 0u, D2 * 2 * CLAIM_WORDS, r->stream);
+    launch_fill_u32(r->claims, 0u, SEGMENT_WORDS + D2 * 2 * CLAIM_WORDS, r->stream);
+    uint32_t *claims = r->claims + SEGMENT_WORDS;
+    auto mark = [&] {
+        if (ev) (void)hipEventRecord((*ev)[(*evi)++], r->stream);
+    };
+    const uint32_t depths = r->opts.ray_depth + 1;
+    const uint32_t apart = std::min(depths, launched_depths(r->dev.view, fp, r->tune, BatchView{}));
+    *extend_launches += fp.mode == RAYNA_MODE_PBR ? depths : 1;
     // the camera rays are stored only for the kernels that load them: k_extend and k_march at depth 0 and
-    // k_shade_mode (k_extend_packet and the first k_shade compute them)
-    fp.rays_stored = fp.mode != RAYNA_MODE_PBR || r->dev.view.n_sdfs > 0 ||
-                     !extend_packets(r->dev.view, fp, r->tune, BatchView{}, 0);
+    // k_shade_mode (k_extend_packet, k_trace and the first k_shade compute them)
+    fp.rays_stored = apart > 0 && (fp.mode != RAYNA_MODE_PBR || r->dev.view.n_sdfs > 0 ||
+                                   !extend_packets(r->dev.view, fp, r->tune, BatchView{}, 0));
     if (fp.rays_stored) launch_generate(fp, r->pb, BatchView{}, r->stream);
-    for (uint32_t depth = 0; depth <= r->opts.ray_depth; ++depth) {
+    r->camera_apart = apart > 0;
+    r->pass_marks = 0;
+    for (uint32_t depth = 0; depth < depths; ++depth) {
         const int32_t *qin = depth == 0 ? nullptr : r->queue[depth & 1];
         const uint32_t *cin = depth == 0 ? nullptr : r->queue_count + depth;
         int32_t *qout = r->queue[(depth + 1) & 1];
         uint32_t *cout = r->queue_count + depth + 1;
-        if (ev) (void)hipEventRecord((*ev)[(*evi)++], r->stream);
-        uint32_t *work = r->claims + (size_t)depth * 2 * CLAIM_WORDS;
-        launch_extend(r->dev.view, fp, r->pb, qin, cin, depth, r->grid_extend, r->dev.overflow, work, r->tune,
-                      BatchView{}, r->stream);
+        uint32_t *work = claims + (size_t)depth * 2 * CLAIM_WORDS;
+        const bool rest = depth >= apart;  // this launch takes every path to its end
+        mark();
+        ++r->pass_marks;
+        if (rest)
+            launch_trace(r->dev.view, fp, r->pb, qin, cin, depth, r->grid_extend, r->dev.overflow, work, r->claims,
+                         r->tune, adjoint, BatchView{}, r->stream);
+        else
+            launch_extend(r->dev.view, fp, r->pb, qin, cin, depth, r->grid_extend, r->dev.overflow, work, r->tune,
+                          BatchView{}, r->stream);
         launch_march(r->dev.view, fp, r->pb, qin, cin, (uint32_t)r->dev.view.n_sdfs, r->mt, r->mt_cap,
                      work + CLAIM_WORDS, r->grid_march, r->grid_shade, r->tune, BatchView{}, r->sdf_queue,
                      r->queue_count + 2 * D2 + depth, r->stream);
-        if (fp.mode != RAYNA_MODE_PBR) {  // render_px_once: the camera ray's hit coloured by the mode
-            if (ev) (void)hipEventRecord((*ev)[(*evi)++], r->stream);
+        mark();
+        if (fp.mode != RAYNA_MODE_PBR)  // render_px_once: the camera ray's hit coloured by the mode
             launch_shade_mode(r->dev.view, fp, r->pb, r->grid_shade, r->stream);
-            if (ev) (void)hipEventRecord((*ev)[(*evi)++], r->stream);
-            ++*extend_launches;
-            break;
-        }
-        if (ev) (void)hipEventRecord((*ev)[(*evi)++], r->stream);
-        launch_shade(r->dev.view, fp, r->pb, qin, cin, qout, cout, depth, r->grid_shade, adjoint, BatchView{},
-                     r->stream);
-        if (ev) (void)hipEventRecord((*ev)[(*evi)++], r->stream);
-        ++*extend_launches;
+        else if (!rest)
+            launch_shade(r->dev.view, fp, r->pb, qin, cin, qout, cout, depth, r->grid_shade, adjoint, BatchView{},
+                         r->stream);
+        mark();
+        if (rest || fp.mode != RAYNA_MODE_PBR) break;
     }
-    launch_count_segments(r->queue_count, r->opts.ray_depth + 1, fp.n_slots, r->segments, r->stream);
+    launch_count_segments(r->queue_count, apart, apart > 0 ? fp.n_slots : 0, r->claims, r->segments, r->stream);
 }
 
 rayna_status ensure_events(rayna_renderer *r, size_t n) {
@@ -412,13 +430,11 @@ rayna_status ensure_events(rayna_renderer *r, size_t n) {
 }
 
 // Device times from the events of one call: events[0] before the first kernel, events[evi - 1] after the
-// last, and per trace_chunk depth the triple [before extend, after extend, after shade] in between (each pass
-// over a chunk records one triple per depth, ray_depth + 1 of them; one for the non-PBR modes).
+// last, and pass_marks triples [before extend, after extend, after shade] per pass over a chunk in between.
 rayna_status event_times(rayna_renderer *r, size_t evi, rayna_render_stats *st) {
     float ms = 0;
     HIP_TRY(r, hipEventElapsedTime(&ms, r->events[0], r->events[evi - 1]));
     st->kernel_ms = ms;
-    const size_t per_pass = r->opts.mode == RAYNA_MODE_PBR ? (size_t)r->opts.ray_depth + 1 : 1;
     double ext = 0, sh = 0, ext0 = 0;
     for (size_t i = 1, k = 0; i + 2 < evi; i += 3, ++k) {
         float a = 0, b = 0;
@@ -426,7 +442,7 @@ rayna_status event_times(rayna_renderer *r, size_t evi, rayna_render_stats *st) 
         HIP_TRY(r, hipEventElapsedTime(&b, r->events[i + 1], r->events[i + 2]));
         ext += a;
         sh += b;
-        if (k % per_pass == 0) ext0 += a;
+        if (r->camera_apart && k % r->pass_marks == 0) ext0 += a;
     }
     st->extend_ms = ext;
     st->shade_ms = sh;
@@ -881,7 +897,7 @@ rayna_status rayna_primary_hits(rayna_renderer *r, uint32_t sample_index, int32_
     r->primal_frame = -1;
     launch_generate(fp, pb, BatchView{}, r->stream);
     uint32_t *sdf_count = r->queue_count + 3 * (r->opts.ray_depth + 2);
-    uint32_t *claims = r->claims + (size_t)(r->opts.ray_depth + 2) * 2 * CLAIM_WORDS;
+    uint32_t *claims = r->claims + SEGMENT_WORDS + (size_t)(r->opts.ray_depth + 2) * 2 * CLAIM_WORDS;
     launch_fill_u32(sdf_count, 0u, 1, r->stream);
     launch_fill_u32(claims, 0u, 2 * CLAIM_WORDS, r->stream);
     launch_extend(r->dev.view, fp, pb, nullptr, nullptr, 0, r->grid_extend, r->dev.overflow, claims, r->tune,

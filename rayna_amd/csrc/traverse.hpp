@@ -113,7 +113,7 @@ __device__ __forceinline__ void expand(const SceneView &sv, const DRay &ray, flo
         t0 = fmaxf(t0, fminf(tz1, tz2));
         t1 = fminf(t1, fmaxf(tz1, tz2));
         const float lo = fmaxf(t0, T_MIN), hi = fminf(t1, best);
-        const bool hit = code[k] != ENTRY_NONE && lo <= hi * BOX_SLACK;
+        const bool hit = lo <= hi * BOX_SLACK;  // whatever an unused slot (ENTRY_NONE) gives: it is not pushed
         key[k] = hit ? t0 : -__builtin_inff();
         if (!hit) code[k] = ENTRY_NONE;  // not pushed
     }
