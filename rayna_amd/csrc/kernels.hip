@@ -495,12 +495,14 @@ struct WaveClaims {
     uint32_t count, claim, waves_per_block;
     uint32_t *work;
     uint32_t part, parts_done;
-    bool first, last;  // first: no claim taken yet; last: every part is used up
+    uint32_t next, end;  // the positions claimed and not handed out yet
+    bool first, last;    // first: no claim taken yet; last: every part is used up
+    bool exhausted;      // last, and everything claimed is handed out
 
     // least, most: the bounds of a claim's size
     __device__ __forceinline__ WaveClaims(uint32_t n, uint32_t wpb, uint32_t least, uint32_t most, uint32_t *counters)
-        : count(n), waves_per_block(wpb), work(counters), part(blockIdx.x % CLAIM_PARTS), parts_done(0), first(true),
-          last(false) {
+        : count(n), waves_per_block(wpb), work(counters), part(blockIdx.x % CLAIM_PARTS), parts_done(0), next(0),
+          end(0), first(true), last(false), exhausted(false) {
         const uint32_t waves = gridDim.x * wpb;
         const uint32_t per = n / waves + (n % waves != 0u ? 1u : 0u);
         claim = per < least ? least : per;
@@ -547,6 +549,25 @@ struct WaveClaims {
             }
             if (got || last) return;
         }
+    }
+    // One position for each lane of `idle` (0xffffffff: none left; the other lanes get what is not theirs), what is left
+    // of the last claim first; a new claim only if may_claim.  The whole wave calls it, idle != 0.
+    __device__ __forceinline__ uint32_t hand_out(unsigned long long idle, bool may_claim = true) {
+        const uint32_t lane = __lane_id(), n = (uint32_t)__popcll(idle), left = end - next;
+        uint32_t from = 0, to = 0;
+        if (left < n && !last && may_claim) take(__ffsll((long long)idle) - 1, &from, &to);
+        const uint32_t idx = (uint32_t)__popcll(idle & ((1ull << lane) - 1ull));  // rank among the idle lanes
+        uint32_t q = 0xffffffffu;
+        if (idx < left) q = next + idx;
+        else if (idx - left < to - from) q = from + (idx - left);
+        if (left >= n) {
+            next += n;
+        } else {
+            next = from + (n - left < to - from ? n - left : to - from);
+            end = to;
+        }
+        if (last && next == end) exhausted = true;
+        return q;
     }
 };
 
@@ -1183,6 +1204,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(
 }
 
 #include "trace.hpp"
+#include "trace_sdf.hpp"
 
 // Sum of the gradient copies: out[i] = sum over copies of grad[copy * n + i], n = 3 * materials.
 __global__ __launch_bounds__(BLOCK) void k_sum_grad(const double *grad, uint32_t n, uint32_t copies, double *out) {
@@ -1422,8 +1444,7 @@ inline unsigned grid_for(uint64_t n, int block) { return (unsigned)((n + block -
 
 }  // namespace
 
-using TraceKernel = void (*)(SceneView, FrameParams, PathBuffers, const int32_t *, const uint32_t *, uint32_t, int2 *,
-                             uint32_t *, uint32_t *, ExtendTuning, AdjointParams, BatchView);
+using TraceKernel = void (*)(TraceArgs);
 // The k_trace instantiations, [batch, adjoint, neither][textures][instances][form], forms as EXTEND_KERNELS'.
 #define RAYNA_TRACE_FORMS(B, T, I, A)                                                                   \
     {k_trace<B, I, false, false, T, A>, k_trace<B, I, true, false, T, A>, k_trace<B, I, true, true, T, A>}
@@ -1434,6 +1455,15 @@ const TraceKernel TRACE_KERNELS[3][2][2][3] = {RAYNA_TRACE_SET(false, false), RA
                                                RAYNA_TRACE_SET(false, true)};
 #undef RAYNA_TRACE_SET
 #undef RAYNA_TRACE_FORMS
+
+// The k_trace_sdf instantiations, [batch, adjoint, neither][form]: form 0 without spheres, media, instances and
+// textures, 1 spheres and media, 2 everything.
+#define RAYNA_TRACE_SDF_FORMS(B, A)                                                                       \
+    {k_trace_sdf<B, false, false, false, false, A>, k_trace_sdf<B, false, true, true, false, A>,          \
+     k_trace_sdf<B, true, true, true, true, A>}
+const TraceKernel TRACE_SDF_KERNELS[3][3] = {RAYNA_TRACE_SDF_FORMS(false, false), RAYNA_TRACE_SDF_FORMS(true, false),
+                                                RAYNA_TRACE_SDF_FORMS(false, true)};
+#undef RAYNA_TRACE_SDF_FORMS
 
 using ExtendKernel = void (*)(SceneView, FrameParams, PathBuffers, const int32_t *, const uint32_t *, uint32_t,
                               int2 *, uint32_t *, ExtendTuning, BatchView);
@@ -1451,6 +1481,7 @@ int extend_form(const SceneView &sv) { return sv.media ? 2 : (sv.sphere_tests ? 
 struct ExtendOccupancy {
     int n[2][2][3];
     int trace[3][2][2][3];
+    int trace_sdf[3][3];
     int most;
 };
 template <class Kernel>
@@ -1468,6 +1499,9 @@ const ExtendOccupancy &extend_occupancy() {
             for (int f = 0; f < 3; ++f) {
                 for (int b = 0; b < 2; ++b)
                     o.most = std::max(o.most, o.n[b][i][f] = resident_blocks(EXTEND_KERNELS[b][i][f]));
+                if (i == 0)
+                    for (int k = 0; k < 3; ++k)
+                        o.most = std::max(o.most, o.trace_sdf[k][f] = resident_blocks(TRACE_SDF_KERNELS[k][f]));
                 for (int k = 0; k < 3; ++k)
                     for (int t = 0; t < 2; ++t)
                         o.most = std::max(o.most, o.trace[k][t][i][f] = resident_blocks(TRACE_KERNELS[k][t][i][f]));
@@ -1528,7 +1562,11 @@ void launch_extend(const SceneView &sv, const FrameParams &fp, const PathBuffers
 }
 
 uint32_t launched_depths(const SceneView &sv, const FrameParams &fp, const ExtendTuning &tune, const BatchView &bv) {
-    if (fp.mode != RAYNA_MODE_PBR || sv.n_sdfs > 0 || fp.checks) return 0xffffffffu;
+    if (fp.mode != RAYNA_MODE_PBR || fp.checks) return 0xffffffffu;
+    if (sv.n_sdfs > 0) {
+        const bool camera_rays = fp.n_slots >= SDF_CAMERA_SLOTS && fp.n_slots < SDF_WHOLE_SLOTS;
+        return fp.n_slots >= SDF_BOUNCE_SLOTS ? 2 : camera_rays ? 1 : 0;
+    }
     if (!extend_packets(sv, fp, tune, bv, 0)) return 0;
     const uint32_t n = fp.n_slots >= FIRST_BOUNCE_SLOTS && sv.n_nodes >= FIRST_BOUNCE_NODES ? 2 : 1;
     return std::max(n, tune.packet_depths);
@@ -1539,10 +1577,14 @@ void launch_trace(const SceneView &sv, const FrameParams &fp, const PathBuffers 
                   uint32_t *segments, const ExtendTuning &tune, const AdjointParams *adjoint, const BatchView &bv,
                   hipStream_t s) {
     const int k = bv.reqs ? 1 : adjoint ? 2 : 0, t = sv.textured ? 1 : 0, i = sv.instances ? 1 : 0;
-    const int f = extend_form(sv);
-    const int g = std::max(1, std::min(grid, grid / extend_blocks_per_cu() * extend_occupancy().trace[k][t][i][f]));
-    hipLaunchKernelGGL(TRACE_KERNELS[k][t][i][f], dim3(g), dim3(EXT_BLOCK), 0, s, sv, fp, pb, queue, count,
-                       first_depth, overflow, work, segments, tune, adjoint ? *adjoint : AdjointParams{}, bv);
+    const int f = extend_form(sv), fs = i || t ? 2 : f ? 1 : 0;
+    const ExtendOccupancy &o = extend_occupancy();
+    const TraceKernel kernel = sv.n_sdfs > 0 ? TRACE_SDF_KERNELS[k][fs] : TRACE_KERNELS[k][t][i][f];
+    const int resident = sv.n_sdfs > 0 ? o.trace_sdf[k][fs] : o.trace[k][t][i][f];
+    const int g = std::max(1, std::min(grid, grid / o.most * resident));
+    const TraceArgs args{sv,   fp,   pb,       queue, count,    first_depth,
+                         overflow, work, segments, tune,  adjoint ? *adjoint : AdjointParams{}, bv};
+    hipLaunchKernelGGL(kernel, dim3(g), dim3(EXT_BLOCK), 0, s, args);
 }
 
 void launch_shade(const SceneView &sv, const FrameParams &fp, const PathBuffers &pb, const int32_t *queue_in,

@@ -105,13 +105,23 @@ constexpr uint32_t SEGMENT_WORDS = SEGMENT_PARTS * 32;
 void launch_extend(const SceneView &sv, const FrameParams &fp, const PathBuffers &pb, const int32_t *queue,
                    const uint32_t *count, uint32_t depth, int grid, int2 *overflow, uint32_t *work,
                    const ExtendTuning &tune, const BatchView &bv, hipStream_t s);
-// How many of a chunk's depths, from the camera rays on, get a launch of extend and one of shade each; the paths that
-// are left go to their ends in one launch (launch_trace).  All depths (2^32 - 1) for the non-PBR modes, scenes with
-// unbounded objects (the march is a pass of its own over all paths) and validation.  Otherwise the camera rays where
-// they are traced as packets, and for a large chunk over a tree that is not small the first bounce too: its rays start
-// from one point per wave, which k_extend's seven waves per SIMD use better than k_trace's mix of depths.  (1080p, 64
-// samples, first bounce apart against not: 45.6 and 48.6 ms with 1.3 M triangles, 34.6 and 36.5 with 1290, 28.2 and
-// 28.3 with 480 spheres, 27.3 and 25.9 in the Cornell box; at 640x360x64, 8.04 and 7.99 ms with 1.3 M triangles.)
+// How many of a chunk's depths, from the camera rays on, get a launch of extend (and march) and one of shade each; the
+// paths that are left go to their ends in one launch (launch_trace).  All depths (2^32 - 1) for the non-PBR modes and
+// validation.
+//
+// Without unbounded objects: the camera rays where they are traced as packets, and for a large chunk over a tree that
+// is not small the first bounce too: its rays start from one point per wave, which k_extend's seven waves per SIMD use
+// better than k_trace's mix of depths.  (1080p, 64 samples, first bounce apart against not: 45.6 and 48.6 ms with
+// 1.3 M triangles, 34.6 and 36.5 with 1290, 28.2 and 28.3 with 480 spheres, 27.3 and 25.9 in the Cornell box; at
+// 640x360x64, 8.04 and 7.99 ms with 1.3 M triangles.)
+//
+// With unbounded objects: k_march's waves are full and each at one SDF, k_trace_sdf's do not wait for a depth's
+// longest march.  So the largest chunks launch the camera rays and the first bounce, where most of the work is; small
+// ones the camera rays, most of which march past everything; the smallest, where every launch is a wait, and those in
+// between none.  (The SDF scene with 0, 1, 2 and all depths launched: 64x36x2 3.2, 3.7, 4.3 and 6.2 ms; 640x360x4 8.1,
+// 6.7, 6.9 and 11.3; 640x360x64 18.0, 18.5, 19.2 and 23.4; 1280x720x128 83.1, 75.4, 71.9 and 76.1.  A scene of mostly
+// bounded objects and one SDF: 161x91x9 1.20, 1.04, 0.89 and 1.16; 1280x720x32 7.1, 8.5, 8.3 and 8.1.)
+constexpr uint32_t SDF_CAMERA_SLOTS = 1u << 14, SDF_WHOLE_SLOTS = 1u << 21, SDF_BOUNCE_SLOTS = 1u << 26;
 constexpr uint32_t FIRST_BOUNCE_SLOTS = 1u << 24;
 constexpr int32_t FIRST_BOUNCE_NODES = 256;
 uint32_t launched_depths(const SceneView &sv, const FrameParams &fp, const ExtendTuning &tune, const BatchView &bv);

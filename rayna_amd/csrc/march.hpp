@@ -71,32 +71,13 @@ __global__ __launch_bounds__(MARCH_BLOCK) __attribute__((amdgpu_waves_per_eu(8))
     const uint32_t refill_lanes = tune.refill_lanes;
     WaveClaims claims(n_items, MARCH_BLOCK / 64, MARCH_CLAIM_LEAST, tune.wave_batch * MARCH_CLAIM_FACTOR, work);
     const uint32_t lane = __lane_id();
-    bool active = false, exhausted = false;
-    uint32_t batch_next = 0, batch_end = 0;
+    bool active = false;
     int32_t j = 0;  // the lane's SDF
     MarchLane L{};
     for (;;) {
         const unsigned long long idle = __ballot(!active);
-        if (!exhausted && idle != 0ull) {
-            const uint32_t n = (uint32_t)__popcll(idle);
-            const uint32_t rem = batch_end - batch_next;
-            uint32_t nb = 0, nb_end = 0;
-            if (rem < n && !claims.last && (idle == ~0ull || n >= refill_lanes))
-                claims.take(__ffsll((long long)idle) - 1, &nb, &nb_end);
-            const uint32_t idx = (uint32_t)__popcll(idle & ((1ull << lane) - 1ull));
-            uint32_t q = 0xffffffffu;
-            if (idx < rem) q = batch_next + idx;
-            else if (idx - rem < nb_end - nb) q = nb + (idx - rem);
-            if (rem >= n) {
-                batch_next += n;
-            } else if (nb_end > nb) {
-                const uint32_t from_new = (n - rem < nb_end - nb) ? n - rem : nb_end - nb;
-                batch_next = nb + from_new;
-                batch_end = nb_end;
-            } else {
-                batch_next = batch_end;
-            }
-            if (claims.last && batch_next == batch_end) exhausted = true;
+        if (!claims.exhausted && idle != 0ull) {
+            const uint32_t q = claims.hand_out(idle, idle == ~0ull || (uint32_t)__popcll(idle) >= refill_lanes);
             if (!active && q != 0xffffffffu) {
                 const uint32_t jj = q / count, qq = q % count;
                 const uint32_t slot = queue ? (uint32_t)queue[qq] : qq;
@@ -121,7 +102,7 @@ __global__ __launch_bounds__(MARCH_BLOCK) __attribute__((amdgpu_waves_per_eu(8))
             }
         }
         if (!__any(active)) {
-            if (exhausted) break;
+            if (claims.exhausted) break;
             continue;
         }
         if (!active) continue;

@@ -399,15 +399,16 @@ void trace_chunk(rayna_renderer *r, FrameParams &fp, uint32_t s0, uint32_t n, st
         const bool rest = depth >= apart;  // this launch takes every path to its end
         mark();
         ++r->pass_marks;
-        if (rest)
+        if (rest) {
             launch_trace(r->dev.view, fp, r->pb, qin, cin, depth, r->grid_extend, r->dev.overflow, work, r->claims,
                          r->tune, adjoint, BatchView{}, r->stream);
-        else
+        } else {
             launch_extend(r->dev.view, fp, r->pb, qin, cin, depth, r->grid_extend, r->dev.overflow, work, r->tune,
                           BatchView{}, r->stream);
-        launch_march(r->dev.view, fp, r->pb, qin, cin, (uint32_t)r->dev.view.n_sdfs, r->mt, r->mt_cap,
-                     work + CLAIM_WORDS, r->grid_march, r->grid_shade, r->tune, BatchView{}, r->sdf_queue,
-                     r->queue_count + 2 * D2 + depth, r->stream);
+            launch_march(r->dev.view, fp, r->pb, qin, cin, (uint32_t)r->dev.view.n_sdfs, r->mt, r->mt_cap,
+                         work + CLAIM_WORDS, r->grid_march, r->grid_shade, r->tune, BatchView{}, r->sdf_queue,
+                         r->queue_count + 2 * D2 + depth, r->stream);
+        }
         mark();
         if (fp.mode != RAYNA_MODE_PBR)  // render_px_once: the camera ray's hit coloured by the mode
             launch_shade_mode(r->dev.view, fp, r->pb, r->grid_shade, r->stream);

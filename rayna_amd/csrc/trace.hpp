@@ -20,71 +20,91 @@ constexpr int trace_waves(bool inst, bool sph, bool vol) { return inst || vol ? 
 // Fewest paths a wave claims, as EXTEND_CLAIM_LEAST (at 16 the 64x36, 2-sample sphere frame takes 417 us, not 344).
 constexpr uint32_t TRACE_CLAIM_LEAST = 4;
 
+// The arguments of k_trace and k_trace_sdf, one struct so that a kernel finds them at the start of its argument segment.
+struct TraceArgs {
+    SceneView sv;
+    FrameParams fp;
+    PathBuffers pb;
+    const int32_t *queue;
+    const uint32_t *count;
+    uint32_t first_depth;
+    int2 *overflow;
+    uint32_t *work, *segments;
+    ExtendTuning tune;
+    AdjointParams ap;
+    BatchView bv;
+};
+// The arguments again, read where they are used: some ninety words of them serve the shading and refill alone, and
+// loaded once at the kernel's start they would hold (and spill, into vector registers) scalar registers through the
+// traversal loops.  The compiler cannot move these loads out of the loop, because it does not know the pointer.
+__device__ __forceinline__ const TraceArgs &cold_args() {
+    typedef __attribute__((address_space(4))) const TraceArgs *Segment;
+    Segment p = (Segment)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return *(const TraceArgs *)p;
+}
+
 // first_depth 0: the paths are the chunk's slots, from their camera rays (computed here).  first_depth > 0: the paths
 // are queue[0 .. *count_ptr), which k_shade kept at depth 0, from their stored rays and throughputs.
 template <bool BATCH, bool INST, bool SPH, bool VOL, bool TEX, bool ADJOINT>
 __global__ __launch_bounds__(EXT_BLOCK) __attribute__((amdgpu_waves_per_eu(trace_waves(INST, SPH, VOL)))) void k_trace(
-    SceneView sv, FrameParams fp, PathBuffers pb, const int32_t *queue, const uint32_t *count_ptr,
-    uint32_t first_depth, int2 *overflow, uint32_t *work, uint32_t *segments, ExtendTuning tune, AdjointParams ap,
-    BatchView bv) {
+    TraceArgs args) {
     __shared__ unsigned long long s_entry[EXT_LDS_STACK * EXT_BLOCK];
     __shared__ float s_t[3 * EXT_BLOCK];  // the paths' throughputs
-    const uint32_t count = queue ? *count_ptr : fp.n_slots;
+    const SceneView &sv = args.sv;
+    const uint32_t count = args.queue ? *args.count : args.fp.n_slots;
     // A refill shades too, so it waits for a quarter more lanes than k_extend's (at 32, 40 and 48 lanes the four mesh
     // preview frames take 4.19, 4.03 and 4.00 ms, the 1080p mesh frame 48.5, 48.3 and 49.0).
-    const uint32_t refill_lanes = tune.refill_lanes + tune.refill_lanes / 4u < 64u
-                                      ? tune.refill_lanes + tune.refill_lanes / 4u
+    const uint32_t refill_lanes = args.tune.refill_lanes + args.tune.refill_lanes / 4u < 64u
+                                      ? args.tune.refill_lanes + args.tune.refill_lanes / 4u
                                       : 64u;
     const uint32_t gid = blockIdx.x * EXT_BLOCK + threadIdx.x;
     const uint32_t lane = __lane_id();
-    const uint32_t copy = ADJOINT ? blockIdx.x % ap.copies : 0u;
-    LaneStack st{(lds_u64 *)s_entry, overflow + gid, gridDim.x * EXT_BLOCK, 0};
+    LaneStack st{(lds_u64 *)s_entry, args.overflow + gid, gridDim.x * EXT_BLOCK, 0};
     enum : int { IDLE, TRACING, HIT };  // no path; a ray in the tree; its closest hit found
     int state = IDLE;
     uint32_t slot = 0, depth = 0, n_segments = 0;
     DRay ray{};
     Best b{FLT_MAX, -1, 0u, 0u, 0u};
-    int32_t leaf = 0;
-    int leaf_i = 0, leaf_n = 0;
-    float leaf_t = 0.0f;
-    uint32_t batch_next = 0, batch_end = 0;
-    bool exhausted = false;
-    WaveClaims claims(count, EXT_BLOCK / 64, TRACE_CLAIM_LEAST, tune.wave_batch, work);
+    LeafRange leaf;
+    TravStats stats;
+    WaveClaims claims(count, EXT_BLOCK / 64, TRACE_CLAIM_LEAST, args.tune.wave_batch, args.work);
     // the path's RNG key, pixel and sample, and in a batch its request
-    auto identify = [&](dm::Key *key, uint32_t *pixel, uint32_t *sample) -> const RequestParams * {
+    auto identify = [&](const TraceArgs &A, dm::Key *key, uint32_t *pixel, uint32_t *sample) -> const RequestParams * {
         if (BATCH) {
-            const RequestParams *R = bv.reqs + bv.slot_req[slot];
+            const RequestParams *R = A.bv.reqs + A.bv.slot_req[slot];
             const uint32_t l = slot - R->slot_base;
             *key = dm::Key{R->key0, R->key1};
             *pixel = l / R->n_spp;
             *sample = R->s0 + l % R->n_spp;
             return R;
         }
-        *key = dm::Key{fp.key0, fp.key1};
-        *pixel = slot / fp.n_spp;
-        *sample = fp.s0 + slot % fp.n_spp;
+        *key = dm::Key{A.fp.key0, A.fp.key1};
+        *pixel = slot / A.fp.n_spp;
+        *sample = A.fp.s0 + slot % A.fp.n_spp;
         return nullptr;
     };
-    dm::Key vkey{fp.key0, fp.key1};
+    dm::Key vkey{0u, 0u};
     uint32_t vpixel = 0, vsample = 0;  // VOL: kept for the free-flight draws
     for (;;) {
         unsigned long long idle = __ballot(state == IDLE);
         const unsigned long long waiting = idle | __ballot(state == HIT);
         if (waiting == ~0ull || (uint32_t)__popcll(waiting) >= refill_lanes) {
+            const TraceArgs &A = cold_args();
             bool begin = false;
             if (state == HIT) {
                 dm::Key key;
                 uint32_t pixel, sample;
-                const RequestParams *R = identify(&key, &pixel, &sample);
+                const RequestParams *R = identify(A, &key, &pixel, &sample);
                 const Col T{s_t[threadIdx.x], s_t[EXT_BLOCK + threadIdx.x], s_t[2 * EXT_BLOCK + threadIdx.x]};
                 Col L{0.0f, 0.0f, 0.0f}, add{0.0f, 0.0f, 0.0f};
-                if (ADJOINT) L = Col{pb.lr[slot], pb.lg[slot], pb.lb[slot]};
+                if (ADJOINT) L = Col{A.pb.lr[slot], A.pb.lg[slot], A.pb.lb[slot]};
                 const uint32_t at_depth = depth;
                 const Best hit = b;
                 begin = shade_vertex<ADJOINT, TEX, false, false>(
-                    sv, nullptr, ap, copy, ray, hit.ref, &hit.t, &hit.aux, &hit.sub, false, f3{0.0f, 0.0f, 0.0f}, key,
-                    pixel, sample, at_depth, BATCH ? R->ray_depth : fp.ray_depth, BATCH ? R->skybox : sv.skybox,
-                    BATCH ? R->sky_image : sv.sky_image, T, L, add, [&](const DRay &nr, const Col &t) {
+                    A.sv, nullptr, A.ap, ADJOINT ? blockIdx.x % A.ap.copies : 0u, ray, hit.ref, &hit.t, &hit.aux, &hit.sub, false, f3{0.0f, 0.0f, 0.0f}, key,
+                    pixel, sample, at_depth, BATCH ? R->ray_depth : A.fp.ray_depth, BATCH ? R->skybox : A.sv.skybox,
+                    BATCH ? R->sky_image : A.sv.sky_image, T, L, add, [&](const DRay &nr, const Col &t) {
                         ray = ray_from_dir(nr.o, nr.d);
                         s_t[threadIdx.x] = t.r;
                         s_t[EXT_BLOCK + threadIdx.x] = t.g;
@@ -92,48 +112,33 @@ __global__ __launch_bounds__(EXT_BLOCK) __attribute__((amdgpu_waves_per_eu(trace
                         ++depth;
                     });
                 const bool adds = !(add.r == 0.0f && add.g == 0.0f && add.b == 0.0f);
-                if (!ADJOINT && at_depth != 0u && adds) L = Col{pb.lr[slot], pb.lg[slot], pb.lb[slot]};
+                if (!ADJOINT && at_depth != 0u && adds) L = Col{A.pb.lr[slot], A.pb.lg[slot], A.pb.lb[slot]};
                 if (!ADJOINT) L = L + add;
                 if (ADJOINT || at_depth == 0u || adds) {
-                    pb.lr[slot] = L.r;
-                    pb.lg[slot] = L.g;
-                    pb.lb[slot] = L.b;
+                    A.pb.lr[slot] = L.r;
+                    A.pb.lg[slot] = L.g;
+                    A.pb.lb[slot] = L.b;
                 }
                 state = IDLE;
             }
             idle = __ballot(state == IDLE && !begin);
-            if (!exhausted && idle != 0ull) {
-                const uint32_t n = (uint32_t)__popcll(idle);
-                const uint32_t r = batch_end - batch_next;
-                uint32_t nb = 0, nb_end = 0;
-                if (r < n && !claims.last) claims.take(__ffsll((long long)idle) - 1, &nb, &nb_end);
-                const uint32_t idx = (uint32_t)__popcll(idle & ((1ull << lane) - 1ull));
-                uint32_t q = 0xffffffffu;
-                if (idx < r) q = batch_next + idx;
-                else if (idx - r < nb_end - nb) q = nb + (idx - r);
-                if (r >= n) {
-                    batch_next += n;
-                } else {
-                    const uint32_t from_new = (n - r < nb_end - nb) ? n - r : nb_end - nb;
-                    batch_next = nb + from_new;
-                    batch_end = nb_end;
-                }
-                if (claims.last && batch_next == batch_end) exhausted = true;
+            if (!claims.exhausted && idle != 0ull) {
+                const uint32_t q = claims.hand_out(idle);
                 if (state == IDLE && !begin && q != 0xffffffffu) {
-                    slot = queue ? (uint32_t)queue[q] : q;
-                    depth = first_depth;
+                    slot = A.queue ? (uint32_t)A.queue[q] : q;
+                    depth = A.first_depth;
                     Col T{1.0f, 1.0f, 1.0f};
-                    if (first_depth == 0u) {
+                    if (A.first_depth == 0u) {
                         dm::Key key;
                         uint32_t pixel, sample;
-                        const RequestParams *R = identify(&key, &pixel, &sample);
+                        const RequestParams *R = identify(A, &key, &pixel, &sample);
                         const DRay c = BATCH ? camera_ray(R->vp, R->width, R->height, R->sdim, key, pixel, sample)
-                                             : camera_ray(fp.vp, fp.width, fp.height, fp.sdim, key, pixel, sample);
+                                             : camera_ray(A.fp.vp, A.fp.width, A.fp.height, A.fp.sdim, key, pixel, sample);
                         ray = ray_from_dir(c.o, c.d);
                     } else {
-                        ray = ray_from_dir(f3{pb.ox[slot], pb.oy[slot], pb.oz[slot]},
-                                           f3{pb.dx[slot], pb.dy[slot], pb.dz[slot]});
-                        T = Col{pb.tr[slot], pb.tg[slot], pb.tb[slot]};
+                        ray = ray_from_dir(f3{A.pb.ox[slot], A.pb.oy[slot], A.pb.oz[slot]},
+                                           f3{A.pb.dx[slot], A.pb.dy[slot], A.pb.dz[slot]});
+                        T = Col{A.pb.tr[slot], A.pb.tg[slot], A.pb.tb[slot]};
                     }
                     s_t[threadIdx.x] = T.r;
                     s_t[EXT_BLOCK + threadIdx.x] = T.g;
@@ -142,76 +147,37 @@ __global__ __launch_bounds__(EXT_BLOCK) __attribute__((amdgpu_waves_per_eu(trace
                 }
             }
             if (begin) {
-                int32_t root = sv.root;
-                if (BATCH) root = bv.reqs[bv.slot_req[slot]].root;
-                if (VOL) (void)identify(&vkey, &vpixel, &vsample);
+                int32_t root = A.sv.root;
+                if (BATCH) root = A.bv.reqs[A.bv.slot_req[slot]].root;
+                if (VOL) (void)identify(A, &vkey, &vpixel, &vsample);
                 if (INST) {  // finish_instance reloads the world ray
-                    pb.ox[slot] = ray.o.x;
-                    pb.oy[slot] = ray.o.y;
-                    pb.oz[slot] = ray.o.z;
-                    pb.dx[slot] = ray.d.x;
-                    pb.dy[slot] = ray.d.y;
-                    pb.dz[slot] = ray.d.z;
+                    A.pb.ox[slot] = ray.o.x;
+                    A.pb.oy[slot] = ray.o.y;
+                    A.pb.oz[slot] = ray.o.z;
+                    A.pb.dx[slot] = ray.d.x;
+                    A.pb.dy[slot] = ray.d.y;
+                    A.pb.dz[slot] = ray.d.z;
                 }
                 b = Best{FLT_MAX, -1, 0u, 0u, 0u};
                 st.sp = 0;
                 st.top_valid = false;
                 if (root >= 0) st.push(root, -__builtin_inff());
-                leaf = 0;
+                leaf.code = 0;
                 state = TRACING;
                 ++n_segments;
             }
         }
         if (!__any(state == TRACING)) {
-            if (exhausted && !__any(state == HIT)) break;
+            if (claims.exhausted && !__any(state == HIT)) break;
             continue;
         }
-        if (state == TRACING) {  // k_extend's loops
-            bool stalled = leaf != 0 && ((uint32_t)leaf & LEAF_CODE_ITEMS) && leaf_i > 0;
-            for (;;) {
-                const unsigned long long searching = __ballot(leaf == 0 && st.sp > 0);
-                if (searching == 0ull) break;
-                if ((uint32_t)__popcll(searching) <= EXTEND_INNER_EXIT && __any(leaf != 0)) break;
-                if (stalled || st.sp == 0) continue;
-                int32_t code;
-                float tent;
-                st.pop(&code, &tent);
-                if (!(tent <= b.t * BOX_SLACK)) {
-                    if (INST && tent != tent) {
-                        if (leaf != 0) {
-                            st.push(code, tent);
-                            stalled = true;
-                        } else {
-                            finish_instance(sv, pb, slot, code, ray, b, st);
-                        }
-                    }
-                    continue;
-                }
-                if (code < 0) {
-                    if (leaf != 0) {
-                        st.push(code, tent);
-                        stalled = true;
-                        continue;
-                    }
-                    leaf = code;
-                    leaf_i = 0;
-                    leaf_n = (int)(((uint32_t)code >> 27) & 7u) + 1;
-                    leaf_t = tent;
-                    continue;
-                }
-                expand(sv, ray, b.t, code, st);
-            }
-            do {
-                if (leaf != 0) {
-                    if (leaf_test<INST, SPH, VOL>(sv, ray, leaf, leaf_i, leaf_t, b, st, vkey, vpixel, vsample, depth) ||
-                        ++leaf_i == leaf_n)
-                        leaf = 0;
-                }
-            } while ((uint32_t)__popcll(__ballot(leaf != 0)) > EXTEND_PRIM_EXIT);
-            if (st.sp == 0 && leaf == 0) state = HIT;
+        if (state == TRACING) {
+            traverse_pass<INST, SPH, VOL>(sv, args.pb, slot, ray, b, leaf, st, vkey, vpixel, vsample, depth, stats);
+            if (st.sp == 0 && leaf.code == 0) state = HIT;
         }
     }
+    stats.flush();
     // the wave's closest-hit queries, added to one of SEGMENT_PARTS counters a line apart
     for (int o = 32; o > 0; o >>= 1) n_segments += __shfl_xor(n_segments, o);
-    if (lane == 0u && n_segments != 0u) atomicAdd(segments + 32 * (blockIdx.x % SEGMENT_PARTS), n_segments);
+    if (lane == 0u && n_segments != 0u) atomicAdd(args.segments + 32 * (blockIdx.x % SEGMENT_PARTS), n_segments);
 }

@@ -22,21 +22,22 @@
 // rayna_traversal_stats().
 #ifdef RAYNA_TRAVERSAL_STATS
 __device__ unsigned long long g_trav_stats[4];
-#define RAYNA_STAT(name, v) (stat_##name += (v))
-#define RAYNA_STAT_DECL() unsigned long long stat_pops = 0, stat_expands = 0, stat_prims = 0, stat_iterations = 0
-#define RAYNA_STAT_FLUSH()                            \
-    do {                                              \
-        atomicAdd(&g_trav_stats[0], stat_pops);       \
-        atomicAdd(&g_trav_stats[1], stat_expands);    \
-        atomicAdd(&g_trav_stats[2], stat_prims);      \
-        atomicAdd(&g_trav_stats[3], stat_iterations); \
-    } while (0)
+struct TravStats {
+    unsigned long long pops = 0, expands = 0, prims = 0, iterations = 0;
+    __device__ void flush() const {
+        atomicAdd(&g_trav_stats[0], pops);
+        atomicAdd(&g_trav_stats[1], expands);
+        atomicAdd(&g_trav_stats[2], prims);
+        atomicAdd(&g_trav_stats[3], iterations);
+    }
+};
+#define RAYNA_STAT(name) (++stats.name)
 #else
-#define RAYNA_STAT(name, v) ((void)0)
-#define RAYNA_STAT_DECL() ((void)0)
-#define RAYNA_STAT_FLUSH() ((void)0)
+struct TravStats {
+    __device__ void flush() const {}
+};
+#define RAYNA_STAT(name) ((void)0)
 #endif
-
 
 // Traversal stack of one lane: the top EXT_LDS_STACK entries in LDS, each (code, distance) one 64-bit word (one
 // column per lane, conflict-free), deeper entries in this thread's column of a global overflow array (`stride` =
@@ -266,15 +267,7 @@ __device__ __forceinline__ bool leaf_test(const SceneView &sv, DRay &ray, int32_
     return false;
 }
 
-// Closest bounded hit of every live path (Renderer::calculate_intersection, renderer.rs:494-501); the
-// unbounded objects are marched afterwards by k_march.  BATCH: the slots belong to the requests of bv, each
-// with its own scene root and RNG key.  INST: the scene holds instances.  SPH: it intersects spheres.  VOL: it
-// holds media.  Occupancy: a 128-lane block holds 11 KiB of LDS stack, so 14 blocks fit a CU.  Without
-// instances, spheres or media the kernel runs at seven waves per SIMD (72 VGPRs, a few bytes of spills): on the
-// 1080p mesh frame 32.8 ms of k_extend with everything compiled in at six waves, 31.7 without the media code,
-// 31.1 at seven waves with 11 LDS entries (31.4 with 10).  The other forms keep six waves (80 VGPRs; at six
-// waves with a 16-entry stack against five: 8.5% faster).
-// The box loop of k_extend ends for the wave once this many lanes or fewer still search: waiting for the last
+// The box loop of a traversal pass ends for the wave once this many lanes or fewer still search: waiting for the last
 // few searching lanes left most of the wave idle (on the 1080p mesh frame a quarter of the loop's lane slots
 // belonged to lanes whose traversal had ended and a fifth to lanes stalled on a second range).  Measured there:
 // 0 (wait for every lane) 40.0 ms of k_extend per frame, 4: 34.8, 6: 34.4, 8: 34.1, 10: 34.2, 12: 34.5, 16: 35.3.
@@ -285,6 +278,78 @@ constexpr uint32_t EXTEND_INNER_EXIT = 8;
 // pass) 33.6; with EXTEND_INNER_EXIT 4 or 16 and this at 16: 32.9 and 33.1.  Holding part-tested ranges of items
 // back from speculation (below) left it at 32.6.
 constexpr uint32_t EXTEND_PRIM_EXIT = 16;
+
+// The leaf range a lane holds (code 0: none) and the next of its entries to test.
+struct LeafRange {
+    int32_t code = 0;
+    int i = 0, n = 0;
+    float t = 0.0f;
+};
+
+// One pass of a wave's traversal, for the active lanes: inner nodes, then the held ranges' primitives.  A lane's
+// traversal has ended when its stack is empty and it holds no range.
+//
+// Inner nodes until at most EXTEND_INNER_EXIT lanes still search for a leaf range while some lane holds one (or until
+// none searches).  A lane that holds a range keeps expanding inner nodes while others search (speculative traversal,
+// Aila & Laine 2009); a second leaf range, or an instance's end, goes back on the stack and the lane waits.  The lanes
+// still searching when the loop ends keep their stacks and go on in the next pass, after the ranges are tested; every
+// pass tests a range or pops an entry, so the loop ends.
+//
+// The held ranges' primitives, one per round, until at most EXTEND_PRIM_EXIT lanes still test.  A lane left holding
+// part of a range keeps it (its next entry in leaf.i) through the next pass: with a range of triangles, which push
+// nothing, it speculates there as a lane holding a range does; with a range of items it waits (stalled), because the
+// links and instance entries its items push count towards the stack bound only as a block on top of a depth-first
+// state, not interleaved with speculative expansions of the links pushed so far.  Every round tests a primitive of
+// each holder, so the loop ends.
+template <bool INST, bool SPH, bool VOL>
+__device__ __forceinline__ void traverse_pass(const SceneView &sv, const PathBuffers &pb, uint32_t slot, DRay &ray,
+                                              Best &b, LeafRange &leaf, LaneStack &st, const dm::Key &key,
+                                              uint32_t pixel, uint32_t sample, uint32_t bounce, TravStats &stats) {
+    bool stalled = leaf.code != 0 && ((uint32_t)leaf.code & LEAF_CODE_ITEMS) && leaf.i > 0;
+    for (;;) {
+        const unsigned long long searching = __ballot(leaf.code == 0 && st.sp > 0);
+        if (searching == 0ull) break;
+        if ((uint32_t)__popcll(searching) <= EXTEND_INNER_EXIT && __any(leaf.code != 0)) break;
+        if (stalled || st.sp == 0) continue;
+        int32_t code;
+        float tent;
+        st.pop(&code, &tent);
+        RAYNA_STAT(pops);
+        if (!(tent <= b.t * BOX_SLACK)) {  // culled, or an instance's marker (a NaN distance)
+            if (INST && tent != tent) {
+                if (leaf.code != 0) {
+                    st.push(code, tent);
+                    stalled = true;
+                } else {
+                    finish_instance(sv, pb, slot, code, ray, b, st);
+                }
+            }
+            continue;
+        }
+        if (code < 0) {
+            if (leaf.code != 0) {
+                st.push(code, tent);
+                stalled = true;
+                continue;
+            }
+            leaf.code = code;
+            leaf.i = 0;
+            leaf.n = (int)(((uint32_t)code >> 27) & 7u) + 1;
+            leaf.t = tent;
+            continue;
+        }
+        RAYNA_STAT(expands);
+        expand(sv, ray, b.t, code, st);
+    }
+    do {
+        if (leaf.code != 0) {
+            RAYNA_STAT(prims);
+            if (leaf_test<INST, SPH, VOL>(sv, ray, leaf.code, leaf.i, leaf.t, b, st, key, pixel, sample, bounce) ||
+                ++leaf.i == leaf.n)
+                leaf.code = 0;
+        }
+    } while ((uint32_t)__popcll(__ballot(leaf.code != 0)) > EXTEND_PRIM_EXIT);
+}
 
 // Fewest queue positions a wave claims: below 4 * 7000 paths the launch runs on fewer waves instead of on waves of one
 // or two lanes.  (Four 641x359, 1-sample mesh frames at 32, 16, 8 and 4: 5.89, 5.79, 5.62 and 5.39 ms; the 64x36,
@@ -297,6 +362,14 @@ constexpr uint32_t EXTEND_CLAIM_LEAST = 4;
 #ifndef RAYNA_EXT_WAVES_LEAN
 #define RAYNA_EXT_WAVES_LEAN 7
 #endif
+// Closest bounded hit of every live path (Renderer::calculate_intersection, renderer.rs:494-501); the
+// unbounded objects are marched afterwards by k_march.  BATCH: the slots belong to the requests of bv, each
+// with its own scene root and RNG key.  INST: the scene holds instances.  SPH: it intersects spheres.  VOL: it
+// holds media.  Occupancy: a 128-lane block holds 11 KiB of LDS stack, so 14 blocks fit a CU.  Without
+// instances, spheres or media the kernel runs at seven waves per SIMD (72 VGPRs, a few bytes of spills): on the
+// 1080p mesh frame 32.8 ms of k_extend with everything compiled in at six waves, 31.7 without the media code,
+// 31.1 at seven waves with 11 LDS entries (31.4 with 10).  The other forms keep six waves (80 VGPRs; at six
+// waves with a 16-entry stack against five: 8.5% faster).
 template <bool BATCH, bool INST, bool SPH, bool VOL>
 __global__ __launch_bounds__(EXT_BLOCK) __attribute__((amdgpu_waves_per_eu(
     (INST || SPH || VOL) ? RAYNA_EXT_WAVES : RAYNA_EXT_WAVES_LEAN))) void k_extend(
@@ -309,36 +382,17 @@ __global__ __launch_bounds__(EXT_BLOCK) __attribute__((amdgpu_waves_per_eu(
     const uint32_t gid = blockIdx.x * EXT_BLOCK + threadIdx.x;
     const uint32_t lane = __lane_id();
     LaneStack st{(lds_u64 *)s_entry, overflow + gid, gridDim.x * EXT_BLOCK, 0};
-    bool active = false, exhausted = false;
+    bool active = false;
     uint32_t slot = 0, pixel = 0, sample = 0;
     DRay ray{};
     Best b{FLT_MAX, -1, 0u, 0u};
-    int32_t leaf = 0;
-    int leaf_i = 0, leaf_n = 0;
-    float leaf_t = 0.0f;
-    // The wave's unhanded queue positions [batch_next, batch_end), handed to idle lanes without atomics; wave-uniform.
-    uint32_t batch_next = 0, batch_end = 0;
+    LeafRange leaf;
     WaveClaims claims(count, EXT_BLOCK / 64, EXTEND_CLAIM_LEAST, tune.wave_batch, work);
-    RAYNA_STAT_DECL();
+    TravStats stats;
     for (;;) {
         const unsigned long long idle = __ballot(!active);
-        if (!exhausted && (idle == ~0ull || (uint32_t)__popcll(idle) >= refill_lanes)) {
-            const uint32_t n = (uint32_t)__popcll(idle);
-            const uint32_t r = batch_end - batch_next;  // old positions, handed out first
-            uint32_t nb = 0, nb_end = 0;                // new batch [nb, nb_end)
-            if (r < n && !claims.last) claims.take(__ffsll((long long)idle) - 1, &nb, &nb_end);
-            const uint32_t idx = (uint32_t)__popcll(idle & ((1ull << lane) - 1ull));  // rank among idle lanes
-            uint32_t q = 0xffffffffu;
-            if (idx < r) q = batch_next + idx;
-            else if (idx - r < nb_end - nb) q = nb + (idx - r);
-            if (r >= n) {
-                batch_next += n;
-            } else {
-                const uint32_t from_new = (n - r < nb_end - nb) ? n - r : nb_end - nb;
-                batch_next = nb + from_new;
-                batch_end = nb_end;
-            }
-            if (claims.last && batch_next == batch_end) exhausted = true;
+        if (!claims.exhausted && (idle == ~0ull || (uint32_t)__popcll(idle) >= refill_lanes)) {
+            const uint32_t q = claims.hand_out(idle);
             if (!active) {
                 if (q != 0xffffffffu) {
                     slot = queue ? (uint32_t)queue[q] : q;
@@ -360,75 +414,19 @@ __global__ __launch_bounds__(EXT_BLOCK) __attribute__((amdgpu_waves_per_eu(
                     st.sp = 0;
                     st.top_valid = false;
                     if (root >= 0) st.push(root, -__builtin_inff());
-                    leaf = 0;
+                    leaf.code = 0;
                     active = true;
                 }
             }
         }
         if (!__any(active)) {
-            if (exhausted) break;
+            if (claims.exhausted) break;
             continue;
         }
-        RAYNA_STAT(iterations, 1);
+        RAYNA_STAT(iterations);
         if (active) {
-            // Inner nodes until at most EXTEND_INNER_EXIT lanes still search for a leaf range while some lane
-            // holds one (or until none searches).  A lane that holds a range keeps expanding inner nodes while
-            // others search (speculative traversal, Aila & Laine 2009); a second leaf range, or an instance's
-            // end, goes back on the stack and the lane waits.  The lanes still searching when the loop ends keep
-            // their stacks and go on in the next pass, after the ranges are tested; every pass tests a range or
-            // pops an entry, so the loop ends.
-            bool stalled = leaf != 0 && ((uint32_t)leaf & LEAF_CODE_ITEMS) && leaf_i > 0;
-            for (;;) {
-                const unsigned long long searching = __ballot(leaf == 0 && st.sp > 0);
-                if (searching == 0ull) break;
-                if ((uint32_t)__popcll(searching) <= EXTEND_INNER_EXIT && __any(leaf != 0)) break;
-                if (stalled || st.sp == 0) continue;
-                int32_t code;
-                float tent;
-                st.pop(&code, &tent);
-                RAYNA_STAT(pops, 1);
-                if (!(tent <= b.t * BOX_SLACK)) {  // culled, or an instance's marker (a NaN distance)
-                    if (INST && tent != tent) {
-                        if (leaf != 0) {
-                            st.push(code, tent);
-                            stalled = true;
-                        } else {
-                            finish_instance(sv, pb, slot, code, ray, b, st);
-                        }
-                    }
-                    continue;
-                }
-                if (code < 0) {
-                    if (leaf != 0) {
-                        st.push(code, tent);
-                        stalled = true;
-                        continue;
-                    }
-                    leaf = code;
-                    leaf_i = 0;
-                    leaf_n = (int)(((uint32_t)code >> 27) & 7u) + 1;
-                    leaf_t = tent;
-                    continue;
-                }
-                RAYNA_STAT(expands, 1);
-                expand(sv, ray, b.t, code, st);
-            }
-            // The held ranges' primitives, one per pass, until at most EXTEND_PRIM_EXIT lanes still test.  A lane
-            // left holding part of a range keeps it (its next entry in leaf_i) through the next box loop: with a
-            // range of triangles, which push nothing, it speculates there as a lane holding a range does; with a
-            // range of items it waits (stalled), because the links and instance entries its items push count
-            // towards the stack bound only as a block on top of a depth-first state, not interleaved with
-            // speculative expansions of the links pushed so far.  Every pass tests a primitive of each holder, so
-            // the loop ends.
-            do {
-                if (leaf != 0) {
-                    RAYNA_STAT(prims, 1);
-                    if (leaf_test<INST, SPH, VOL>(sv, ray, leaf, leaf_i, leaf_t, b, st, key, pixel, sample, depth) ||
-                        ++leaf_i == leaf_n)
-                        leaf = 0;
-                }
-            } while ((uint32_t)__popcll(__ballot(leaf != 0)) > EXTEND_PRIM_EXIT);
-            if (st.sp == 0 && leaf == 0) {
+            traverse_pass<INST, SPH, VOL>(sv, pb, slot, ray, b, leaf, st, key, pixel, sample, depth, stats);
+            if (st.sp == 0 && leaf.code == 0) {
                 pb.hit_t[slot] = b.t;
                 pb.hit_ref[slot] = b.ref;
                 pb.hit_aux[slot] = b.aux;
@@ -438,7 +436,7 @@ __global__ __launch_bounds__(EXT_BLOCK) __attribute__((amdgpu_waves_per_eu(
             }
         }
     }
-    RAYNA_STAT_FLUSH();
+    stats.flush();
 }
 
 // Rays traced as wave packets: at depth 0 of a single-request frame the 64 lanes of a wave hold neighbouring

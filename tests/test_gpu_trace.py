@@ -1,9 +1,11 @@
 """Paths traced to their ends in one launch against one launch per depth: validation keeps a frame on the latter (and
 changes no pixel), so every scene's two frames and closest-hit counts must be equal, whatever the depth limit, the
-samples per pixel (below and from 16 on, where the camera rays are packets) and the number of chunks."""
+samples per pixel (below and from 16 on, where the camera rays are packets), the number of chunks and, with unbounded
+objects, the number of paths (from 128 * 128 on the camera rays get launches of their own)."""
 import numpy as np
 import pytest
 
+import oracle
 from rayna_amd import Renderer, presets
 
 pytestmark = pytest.mark.gpu
@@ -11,13 +13,15 @@ pytestmark = pytest.mark.gpu
 SCENES = {"mesh": lambda **k: presets.triangle_mesh(subdiv=3, **k), "spheres": presets.random_spheres,
           "cornell": presets.cornell, "rttnw": lambda **k: presets.rttnw(balls=50, **k),
           "textured": presets.textured, "transformed": presets.transformed_mix,
-          "inverse": lambda **k: presets.inverse_spheres(**k)[:3]}
+          "inverse": lambda **k: presets.inverse_spheres(**k)[:3], "mixed": presets.mixed_primitives,
+          "sdf": lambda **k: presets.sdf_volume(max_iterations=64, **k)}
 
 
 @pytest.mark.parametrize("scene", sorted(SCENES))
 @pytest.mark.parametrize("width,height,samples,depth,chunk", [(1, 1, 1, 6, 0), (37, 23, 15, 0, 0), (37, 23, 16, 0, 0),
                                                              (37, 23, 17, 1, 0), (64, 64, 3, 7, 0), (33, 65, 40, 5, 0),
-                                                             (64, 33, 40, 4, 64 * 33 * 17)])
+                                                             (64, 33, 40, 4, 64 * 33 * 17),
+                                                             (128, 127, 1, 4, 0), (128, 128, 1, 4, 0)])
 def test_one_launch_equals_one_per_depth(gpu, scene, width, height, samples, depth, chunk):
     sc, cam, opts = SCENES[scene](width=width, height=height, samples=samples, ray_depth=depth)
     frames = []
@@ -31,3 +35,16 @@ def test_one_launch_equals_one_per_depth(gpu, scene, width, height, samples, dep
     for a, b in zip(frames[:2], frames[2:]):
         assert np.array_equal(a[0], b[0])
         assert a[1] == b[1]
+
+
+@pytest.mark.parametrize("scene", ["cornell", "mixed", "rttnw", "sdf", "textured"])
+@pytest.mark.parametrize("samples", [3, 16])
+def test_adjoint_equals_the_oracle(gpu, scene, samples):
+    """The replay in one launch, on scenes with instances, media, textures and unbounded objects: the oracle's gradient
+    up to the order of its float64 sums."""
+    sc, cam, opts = SCENES[scene](width=24, height=16, samples=samples, ray_depth=5)
+    d = np.random.default_rng(3).standard_normal((16, 24, 3)).astype(np.float32)
+    with Renderer(sc, cam, opts) as r:
+        g, _ = r.adjoint(d, layout="rowmajor")
+    ref, _, _ = oracle.TwinScene(sc).adjoint(cam, opts, d, precision=32)
+    assert np.linalg.norm(g - ref) <= 1e-9 * np.linalg.norm(ref)
