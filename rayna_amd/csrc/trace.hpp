@@ -54,7 +54,10 @@ __global__ __launch_bounds__(EXT_BLOCK) __attribute__((amdgpu_waves_per_eu(trace
     const SceneView &sv = args.sv;
     const uint32_t count = args.queue ? *args.count : args.fp.n_slots;
     // A refill shades too, so it waits for a quarter more lanes than k_extend's (at 32, 40 and 48 lanes the four mesh
-    // preview frames take 4.19, 4.03 and 4.00 ms, the 1080p mesh frame 48.5, 48.3 and 49.0).
+    // preview frames take 4.19, 4.03 and 4.00 ms, the 1080p mesh frame 48.5, 48.3 and 49.0).  Once no path is left to
+    // take, idle lanes say nothing: half of the wave's paths then wait (against refill_lanes waiting or idle, where a
+    // wave with few paths shaded them one by one: the preview frames 4.24 -> 3.96 ms, the inverse-rendering step 3.97 ->
+    // 3.80; at a third 4.01 and 3.77, at a twelfth 4.18 and 3.95).
     const uint32_t refill_lanes = args.tune.refill_lanes + args.tune.refill_lanes / 4u < 64u
                                       ? args.tune.refill_lanes + args.tune.refill_lanes / 4u
                                       : 64u;
@@ -89,7 +92,8 @@ __global__ __launch_bounds__(EXT_BLOCK) __attribute__((amdgpu_waves_per_eu(trace
     for (;;) {
         unsigned long long idle = __ballot(state == IDLE);
         const unsigned long long waiting = idle | __ballot(state == HIT);
-        if (waiting == ~0ull || (uint32_t)__popcll(waiting) >= refill_lanes) {
+        const uint32_t n_idle = (uint32_t)__popcll(idle), n_hit = (uint32_t)__popcll(waiting) - n_idle;
+        if (waiting == ~0ull || (claims.exhausted ? 2u * n_hit >= 64u - n_idle : n_idle + n_hit >= refill_lanes)) {
             const TraceArgs &A = cold_args();
             bool begin = false;
             if (state == HIT) {
