@@ -472,6 +472,12 @@ rayna_status rayna_scene_tree(const rayna_scene_desc *scene, int32_t *node_words
 /* Renderer drop. */
 void rayna_destroy(rayna_renderer *r);
 
+/* Pinned host memory for images: rayna_render and rayna_render_batch copy into it directly, several times faster than
+ * into ordinary memory.  Valid for every device.  Errors are reported through rayna_last_error(NULL);
+ * rayna_host_free(NULL) does nothing. */
+rayna_status rayna_host_alloc(uint64_t bytes, void **out);
+void rayna_host_free(void *p);
+
 /* Measurement hook (no engine counterpart): the fp32 VALU issue rate the current GPU sustains, the peak the
  * traversal kernels' VALU roofline is taken against.  A calibration kernel runs eight independent multiply-add
  * chains per lane (one v_mul_f32 and one v_add_f32 per link: no packed or fused forms), eight waves on every

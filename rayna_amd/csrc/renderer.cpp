@@ -1013,6 +1013,18 @@ void rayna_destroy(rayna_renderer *r) {
     delete r;
 }
 
+rayna_status rayna_host_alloc(uint64_t bytes, void **out) {
+    g_create_error.clear();
+    if (!out || bytes == 0) return fail(nullptr, RAYNA_INVALID_ARGUMENT, "null output or no bytes");
+    *out = nullptr;
+    HIP_TRY(nullptr, hipHostMalloc(out, bytes, hipHostMallocPortable));
+    return RAYNA_OK;
+}
+
+void rayna_host_free(void *p) {
+    if (p) (void)hipHostFree(p);
+}
+
 rayna_status rayna_debug_sqrt_mismatches(uint32_t first, uint64_t count, uint64_t *mismatches) {
     g_create_error.clear();
     if (!mismatches || count > (1ull << 32) - first)

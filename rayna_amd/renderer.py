@@ -19,6 +19,7 @@ from typing import Optional
 import numpy as np
 
 from . import _abi as A
+from . import host_buffers
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 # RAYNA_AMD_LIB selects another build of the library (e.g. a tuning variant); the default is the in-tree build.
@@ -31,7 +32,8 @@ EXPORTS = ("rayna_create", "rayna_set_scene", "rayna_set_camera", "rayna_set_opt
            "rayna_set_validate", "rayna_validate_counts", "rayna_adjoint_static", "rayna_batch_create",
            "rayna_batch_set_tuning", "rayna_render_batch", "rayna_batch_destroy", "rayna_batch_last_error",
            "rayna_primary_hits", "rayna_dfs_order", "rayna_tree_hash", "rayna_scene_prepare", "rayna_scene_tree", "rayna_destroy",
-           "rayna_measure_valu_peak", "rayna_debug_sqrt_mismatches", "rayna_debug_fail_launches", "rayna_last_error")
+           "rayna_host_alloc", "rayna_host_free", "rayna_measure_valu_peak", "rayna_debug_sqrt_mismatches",
+           "rayna_debug_fail_launches", "rayna_last_error")
 
 
 # RAYNA_CHECK_* of include/rayna_gpu.h, in order: the invariants of the engine's shared/validate.rs
@@ -109,6 +111,10 @@ def lib() -> C.CDLL:
                                        C.POINTER(C.c_int32)]
         L.rayna_destroy.restype = None
         L.rayna_destroy.argtypes = [vp]
+        L.rayna_host_alloc.restype = C.c_int
+        L.rayna_host_alloc.argtypes = [C.c_uint64, C.POINTER(vp)]
+        L.rayna_host_free.restype = None
+        L.rayna_host_free.argtypes = [vp]
         L.rayna_measure_valu_peak.restype = C.c_int
         L.rayna_measure_valu_peak.argtypes = [C.c_uint32, C.POINTER(C.c_double), C.POINTER(C.c_double)]
         L.rayna_debug_sqrt_mismatches.restype = C.c_int
@@ -294,7 +300,7 @@ class Renderer:
 
     def render(self, layout: str = "xmajor", to_host: bool = True) -> Render:
         o = self._options
-        img = np.zeros((o.width * o.height * 3,), np.float32) if to_host else None
+        img = host_buffers.empty(o.width * o.height * 3, np.float32) if to_host else None
         dims = (C.c_uint32 * 2)()
         st = A.RenderStats()
         lay = A.LAYOUT_XMAJOR if layout == "xmajor" else A.LAYOUT_ROWMAJOR
@@ -312,7 +318,7 @@ class Renderer:
         """render() followed by the UI's 8-bit conversion (rayna_ui/src/ext/img_ext.rs:15-45) on the GPU:
         (height, width, 4) uint8 RGBA, gamma 1/2.2."""
         o = self._options
-        img = np.zeros(o.width * o.height * 4, np.uint8)
+        img = host_buffers.empty(o.width * o.height * 4, np.uint8)
         dims = (C.c_uint32 * 2)()
         st = A.RenderStats()
         _check(lib().rayna_render_srgb8(self._h, img.ctypes.data_as(C.POINTER(C.c_uint8)), dims, C.byref(st)),

@@ -1,0 +1,98 @@
+"""The pool of pinned image buffers: its bounds, reuse and fallbacks on a stand-in allocator, and on the GPU that an
+image is never overwritten while it or a view of it is held."""
+import gc
+import threading
+
+import numpy as np
+import pytest
+
+from rayna_amd import Renderer, host_buffers, presets, renderer
+
+
+class FakeLib:
+    """rayna_host_alloc / rayna_host_free over ordinary memory."""
+
+    def __init__(self, fail=False):
+        self.fail, self.held = fail, {}
+
+    def rayna_host_alloc(self, size, out):
+        if self.fail:
+            return 1
+        a = np.zeros(size, np.uint8)
+        self.held[a.ctypes.data] = a
+        out._obj.value = a.ctypes.data
+        return 0
+
+    def rayna_host_free(self, address):
+        del self.held[address]
+
+
+@pytest.fixture
+def fake(monkeypatch):
+    lib = FakeLib()
+    monkeypatch.setattr(renderer, "lib", lambda: lib)
+    monkeypatch.setattr(host_buffers, "_pool", host_buffers._Pool())
+    return lib
+
+
+def test_reuse_only_after_the_last_view(fake):
+    a = host_buffers.empty(1000, np.float32)
+    at = a.ctypes.data
+    view = a[10:20].reshape(2, 5)
+    del a
+    gc.collect()
+    b = host_buffers.empty(1000, np.float32)
+    assert b.ctypes.data != at and b.flags.writeable and b.shape == (1000,)
+    del view
+    gc.collect()
+    assert host_buffers.empty(990, np.float32).ctypes.data == at
+
+
+def test_bounds(fake, monkeypatch):
+    monkeypatch.setattr(host_buffers, "IDLE_BYTES", 3 * 4096)
+    monkeypatch.setattr(host_buffers, "PINNED_BYTES", 5 * 4096)
+    arrays = [host_buffers.empty(4096, np.uint8) for _ in range(7)]
+    assert len(fake.held) == 5 and host_buffers._pool.used_bytes == 5 * 4096
+    del arrays
+    gc.collect()
+    assert len(fake.held) == 3 and host_buffers._pool.used_bytes == 0
+
+
+def test_without_pinned_memory_and_empty(fake):
+    fake.fail = True
+    assert host_buffers.empty(5, np.float32).shape == (5,) and host_buffers._pool.used_bytes == 0
+    assert host_buffers.empty(0, np.float32).shape == (0,)
+
+
+def test_threads(fake):
+    bad = []
+
+    def work(k):
+        for i in range(300):
+            a = host_buffers.empty(1 + (i * 37 + k) % 5000, np.uint8)
+            a[:] = k
+            b = host_buffers.empty(1 + (i * 53 + k) % 5000, np.uint8)
+            b[:] = k + 100
+            if not (a == k).all():
+                bad.append(k)
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(6)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    gc.collect()
+    assert not bad and host_buffers._pool.used_bytes == 0
+
+
+@pytest.mark.gpu
+def test_held_images_keep_their_values(gpu):
+    frames, copies = [], []
+    for seed in range(4):
+        sc, cam, opts = presets.cornell(width=65, height=43, samples=2, seed=seed)
+        with Renderer(sc, cam, opts) as r:
+            for out in (r.render(), r.render_srgb8(), r.render(layout="rowmajor")):
+                frames.append(out.img[1:])
+                copies.append(out.img[1:].copy())
+    for a, b in zip(frames, copies):
+        assert np.array_equal(a, b)
