@@ -492,7 +492,7 @@ hipError_t enqueue(rayna_batch *b, const Plan &pl, int used, bool timing) {
                          P.queue_count + 2 * (D + 2) + depth, s);
             launch_shade(cv, fp, P.pb, qin, cin, qout, cout, depth, b->grid_shade, nullptr, bv, s);
         }
-        launch_count_segments(P.queue_count, apart, apart > 0 ? fp.n_slots : 0, P.claims, P.segments, s);
+        launch_count_segments(SegmentCount{P.queue_count, apart, apart > 0 ? fp.n_slots : 0u, P.claims, P.segments, 0u}, s);
         // (a dependency on the same pipeline is kept by its stream's order)
         if (used > 1 && pl.dep[c] >= 0 && (size_t)pl.dep[c] % used != c % used)
             check(hipStreamWaitEvent(s, b->resolved[pl.dep[c]], 0));

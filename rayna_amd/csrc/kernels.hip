@@ -1215,22 +1215,23 @@ __global__ __launch_bounds__(BLOCK) void k_sum_grad(const double *grad, uint32_t
     out[i] = s;
 }
 
-// Running sums, in sample order, of the n samples (slots base + p * n + k, k < n) of each pixel p of
-// [p0, p0 + np) into sum (three planes of P floats; first: start from 0).  The whole block calls it.  The samples
-// are staged in LDS with coalesced loads (one row of n | 1 floats per pixel and channel: an odd stride keeps the
-// summing threads on distinct banks), then one thread per (pixel, channel) adds its row in order.
-__device__ void resolve_pixels(const PathBuffers &pb, uint32_t base, uint32_t p0, uint32_t np, uint32_t n, uint32_t P,
-                               float *sum, bool first) {
+// Sums, in sample order, of the n samples (slots base + p * n + k, k < n) of each pixel p of [p0, p0 + np), each on top
+// of init(channel, p), given to done(channel, p, sum).  The whole block calls it.  The samples are staged in LDS with
+// coalesced loads (one row of n | 1 floats per pixel and channel: an odd stride keeps the summing threads on distinct
+// banks), then one thread per (pixel, channel) adds its row in order.
+template <class Init, class Done>
+__device__ __forceinline__ void resolve_pixels(const PathBuffers &pb, uint32_t base, uint32_t p0, uint32_t np, uint32_t n,
+                                               Init init, Done done) {
     __shared__ float stage[3 * RESOLVE_STAGE];
     const uint32_t t = threadIdx.x;
     const float *src[3] = {pb.lr + base + (size_t)p0 * n, pb.lg + base + (size_t)p0 * n, pb.lb + base + (size_t)p0 * n};
     const uint32_t w = n | 1u;
     if (w > RESOLVE_STAGE) {  // a thread per pixel, straight from HBM
         for (uint32_t px = t; px < np; px += BLOCK)
-            for (int c = 0; c < 3; ++c) {
-                float s = first ? 0.0f : sum[c * P + p0 + px];
+            for (uint32_t c = 0; c < 3; ++c) {
+                float s = init(c, p0 + px);
                 for (uint32_t k = 0; k < n; ++k) s = s + src[c][(size_t)px * n + k];
-                sum[c * P + p0 + px] = s;
+                done(c, p0 + px, s);
             }
         return;
     }
@@ -1246,38 +1247,60 @@ __device__ void resolve_pixels(const PathBuffers &pb, uint32_t base, uint32_t p0
     for (uint32_t u = t; u < 3 * np; u += BLOCK) {
         const uint32_t c = u / np, px = u - c * np;
         const float *row = stage + c * RESOLVE_STAGE + px * w;
-        float s = first ? 0.0f : sum[c * P + p0 + px];
+        float s = init(c, p0 + px);
         for (uint32_t k = 0; k < n; ++k) s = s + row[k];
-        sum[c * P + p0 + px] = s;
+        done(c, p0 + px, s);
     }
 }
 
-// Per-pixel running sum of the chunk's samples in sample order (render_px_msaa's sum, renderer.rs:398-402).
-__global__ __launch_bounds__(BLOCK) void k_resolve(FrameParams fp, PathBuffers pb, float *sum, uint32_t chunk_samples,
-                                                   int first) {
-    const uint32_t per = resolve_pixels_per_block(chunk_samples);
-    const uint32_t p0 = blockIdx.x * per;
-    const uint32_t np = fp.n_pixels - p0 < per ? fp.n_pixels - p0 : per;
-    resolve_pixels(pb, 0u, p0, np, chunk_samples, fp.n_pixels, sum, first != 0);
+// A chunk's closest-hit queries: first_count, the lengths of queues 1 to n - 1, and what k_trace counted.  One wave.
+__device__ __forceinline__ void count_segments(const SegmentCount &sc) {
+    const uint32_t lane = __lane_id();
+    unsigned long long s = 0;
+    for (uint32_t i = 1 + lane; i < sc.n; i += 64) s += sc.queue_count[i];
+    for (uint32_t i = lane; i < SEGMENT_PARTS; i += 64) s += sc.parts[32 * i];
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+    if (lane == 0u) *sc.segments = (sc.first ? 0ull : *sc.segments) + s + sc.first_count;
 }
 
-// Sample mean, accumulation buffer update and output image (accum_buffer.rs:31-45).
-__global__ __launch_bounds__(BLOCK) void k_finalize(FrameParams fp, const float *sum, float *acc, double frames,
-                                                    float *out, int layout) {
+// Channel c of pixel p's output: the sample mean, added to the accumulation buffer (accum_buffer.rs:31-45).
+__device__ __forceinline__ void finalize_channel(const FrameParams &fp, const FrameOutput &out, uint32_t c, uint32_t p,
+                                                 float mean) {
+    const uint32_t P = fp.n_pixels, x = p % fp.width, y = p / fp.width;
+    const size_t o = out.layout == RAYNA_LAYOUT_XMAJOR ? ((size_t)x * fp.height + y) * 3 : (size_t)p * 3;
+    const float a = (out.fresh ? 0.0f : out.acc[c * P + p]) + mean;
+    out.acc[c * P + p] = a;
+    out.image[o + c] = (float)((double)a / out.frames);
+}
+
+// Per-pixel running sum of the chunk's samples in sample order (render_px_msaa's sum, renderer.rs:398-402), and the
+// chunk's closest-hit queries.  LAST: the frame's last chunk, whose sums go on to the output at once (a launch and a
+// trip of the sums through memory less than k_finalize after it).
+template <bool LAST>
+__global__ __launch_bounds__(BLOCK) void k_resolve(FrameParams fp, PathBuffers pb, float *sum, uint32_t chunk_samples,
+                                                   int first, SegmentCount sc, FrameOutput out) {
+    if (blockIdx.x == 0 && threadIdx.x < 64) count_segments(sc);
+    const uint32_t per = resolve_pixels_per_block(chunk_samples);
+    const uint32_t p0 = blockIdx.x * per, P = fp.n_pixels;
+    const uint32_t np = P - p0 < per ? P - p0 : per;
+    resolve_pixels(
+        pb, 0u, p0, np, chunk_samples, [&](uint32_t c, uint32_t p) { return first ? 0.0f : sum[c * P + p]; },
+        [&](uint32_t c, uint32_t p, float s) {
+            if (LAST) finalize_channel(fp, out, c, p, s / (float)fp.spp);
+            else sum[c * P + p] = s;
+        });
+}
+
+// The output from the frame's sums, and under validation its check of the pixels' means.
+__global__ __launch_bounds__(BLOCK) void k_finalize(FrameParams fp, const float *sum, FrameOutput out) {
     const uint32_t p = blockIdx.x * BLOCK + threadIdx.x;
     if (p >= fp.n_pixels) return;
     const uint32_t P = fp.n_pixels;
     const float n = (float)fp.spp;
     const float mean[3] = {sum[p] / n, sum[P + p] / n, sum[2 * P + p] / n};
     if (fp.checks && !colour_ok(Col{mean[0], mean[1], mean[2]})) count_check(fp.checks, RAYNA_CHECK_PIXEL);
-    const uint32_t x = p % fp.width, y = p / fp.width;
-    const size_t o = layout == RAYNA_LAYOUT_XMAJOR ? ((size_t)x * fp.height + y) * 3 : (size_t)p * 3;
 #pragma unroll
-    for (int c = 0; c < 3; ++c) {
-        const float a = acc[c * P + p] + mean[c];
-        acc[c * P + p] = a;
-        out[o + c] = (float)((double)a / frames);
-    }
+    for (uint32_t c = 0; c < 3; ++c) finalize_channel(fp, out, c, p, mean[c]);
 }
 
 // k_resolve for the requests of a batch chunk: blockIdx.y selects the request.
@@ -1287,7 +1310,12 @@ __global__ __launch_bounds__(BLOCK) void k_resolve_batch(BatchView bv, PathBuffe
     const uint32_t p0 = blockIdx.x * per;
     if (p0 >= R.n_pixels) return;  // the whole block
     const uint32_t np = R.n_pixels - p0 < per ? R.n_pixels - p0 : per;
-    resolve_pixels(pb, R.slot_base, p0, np, R.n_spp, R.n_pixels, sum + R.sum_offset, R.first_piece != 0);
+    float *su = sum + R.sum_offset;
+    const uint32_t P = R.n_pixels;
+    const bool first = R.first_piece != 0;
+    resolve_pixels(
+        pb, R.slot_base, p0, np, R.n_spp, [&](uint32_t c, uint32_t p) { return first ? 0.0f : su[c * P + p]; },
+        [&](uint32_t c, uint32_t p, float s) { su[c * P + p] = s; });
 }
 
 // The sample mean of each finished request of a batch (a first frame: the accumulation is the mean itself),
@@ -1429,16 +1457,7 @@ __global__ __launch_bounds__(BLOCK) void k_sqrt_check(uint32_t first, uint32_t c
     if (bad) atomicAdd(mismatches, (unsigned long long)bad);
 }
 
-// Adds a chunk's closest-hit queries to *segments: first_count, the lengths of queues 1 to n - 1, and what k_trace
-// counted.  One wave.
-__global__ void k_count_segments(const uint32_t *queue_count, uint32_t n, uint32_t first_count, const uint32_t *parts,
-                                 unsigned long long *segments) {
-    unsigned long long s = 0;
-    for (uint32_t i = 1 + threadIdx.x; i < n; i += 64) s += queue_count[i];
-    for (uint32_t i = threadIdx.x; i < SEGMENT_PARTS; i += 64) s += parts[32 * i];
-    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
-    if (threadIdx.x == 0) *segments += s + first_count;
-}
+__global__ void k_count_segments(SegmentCount sc) { count_segments(sc); }  // one wave
 
 inline unsigned grid_for(uint64_t n, int block) { return (unsigned)((n + block - 1) / block); }
 
@@ -1647,15 +1666,17 @@ void launch_to_srgb8(const float *img, uint32_t n_pixels, uint8_t *rgba, hipStre
 }
 
 void launch_resolve(const FrameParams &fp, const PathBuffers &pb, float *sum, uint32_t chunk_samples, int first,
-                    hipStream_t s) {
-    hipLaunchKernelGGL(k_resolve, dim3(grid_for(fp.n_pixels, (int)resolve_pixels_per_block(chunk_samples))),
-                       dim3(BLOCK), 0, s, fp, pb, sum, chunk_samples, first);
+                    const SegmentCount &sc, const FrameOutput *out, hipStream_t s) {
+    const dim3 grid(grid_for(fp.n_pixels, (int)resolve_pixels_per_block(chunk_samples)));
+    if (out)
+        hipLaunchKernelGGL(k_resolve<true>, grid, dim3(BLOCK), 0, s, fp, pb, sum, chunk_samples, first, sc, *out);
+    else
+        hipLaunchKernelGGL(k_resolve<false>, grid, dim3(BLOCK), 0, s, fp, pb, sum, chunk_samples, first, sc,
+                           FrameOutput{});
 }
 
-void launch_finalize(const FrameParams &fp, const float *sum, float *acc, double frames, float *out, int layout,
-                     hipStream_t s) {
-    hipLaunchKernelGGL(k_finalize, dim3(grid_for(fp.n_pixels, BLOCK)), dim3(BLOCK), 0, s, fp, sum, acc, frames, out,
-                       layout);
+void launch_finalize(const FrameParams &fp, const float *sum, const FrameOutput &out, hipStream_t s) {
+    hipLaunchKernelGGL(k_finalize, dim3(grid_for(fp.n_pixels, BLOCK)), dim3(BLOCK), 0, s, fp, sum, out);
 }
 
 void launch_fill_u32(uint32_t *p, uint32_t value, uint32_t n, hipStream_t s) {
@@ -1671,9 +1692,8 @@ uint64_t launch_valu_peak(float *out, uint32_t blocks, uint32_t iters, hipStream
     return (uint64_t)blocks * (BLOCK / 64) * iters * (2 * VALU_PEAK_CHAINS);
 }
 
-void launch_count_segments(const uint32_t *queue_count, uint32_t n, uint32_t first_count, const uint32_t *parts,
-                           unsigned long long *segments, hipStream_t s) {
-    hipLaunchKernelGGL(k_count_segments, dim3(1), dim3(64), 0, s, queue_count, n, first_count, parts, segments);
+void launch_count_segments(const SegmentCount &sc, hipStream_t s) {
+    hipLaunchKernelGGL(k_count_segments, dim3(1), dim3(64), 0, s, sc);
 }
 
 // ------------------------------------------------------------------------------------------ static workspace

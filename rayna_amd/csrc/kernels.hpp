@@ -164,10 +164,29 @@ void launch_sum_grad(const double *grad, uint32_t n, uint32_t copies, double *ou
 void launch_shade_mode(const SceneView &sv, const FrameParams &fp, const PathBuffers &pb, int grid, hipStream_t s);
 // The UI's 8-bit conversion of a row-major float image (width * height * 3) to RGBA.
 void launch_to_srgb8(const float *img, uint32_t n_pixels, uint8_t *rgba, hipStream_t s);
+// A chunk's closest-hit queries, added to *segments (first: set): first_count, the lengths of queues 1 to n - 1 and the
+// SEGMENT_PARTS counters of launch_trace.
+struct SegmentCount {
+    const uint32_t *queue_count;
+    uint32_t n, first_count;
+    const uint32_t *parts;
+    unsigned long long *segments;
+    uint32_t first;
+};
+// Where a frame's means go: the accumulation buffer (three planes; fresh: it holds nothing yet), and the image, the
+// accumulated sum over `frames`.
+struct FrameOutput {
+    float *acc, *image;
+    double frames;
+    int32_t layout;  // RAYNA_LAYOUT_*
+    uint32_t fresh;
+};
+// The chunk's samples added to the frame's per-pixel sums, and the chunk's queries counted.  out: the chunk is the
+// frame's last, and its sums go to the output instead (launch_finalize is then not needed; it checks the pixels under
+// validation, which this does not).
 void launch_resolve(const FrameParams &fp, const PathBuffers &pb, float *sum, uint32_t chunk_samples, int first,
-                    hipStream_t s);
-void launch_finalize(const FrameParams &fp, const float *sum, float *acc, double frames, float *out, int layout,
-                     hipStream_t s);
+                    const SegmentCount &sc, const FrameOutput *out, hipStream_t s);
+void launch_finalize(const FrameParams &fp, const float *sum, const FrameOutput &out, hipStream_t s);
 void launch_fill_u32(uint32_t *p, uint32_t value, uint32_t n, hipStream_t s);
 // Whether launch_extend traces this depth as wave packets (k_extend_packet).  At depth 0 of a single request the
 // packets compute the camera rays themselves, so only the march and the non-PBR modes need k_generate's rays.
@@ -177,8 +196,7 @@ bool extend_packets(const SceneView &sv, const FrameParams &fp, const ExtendTuni
 // the wave64 VALU instructions its chains issue (loop and set-up instructions not counted).
 uint64_t launch_valu_peak(float *out, uint32_t blocks, uint32_t iters, hipStream_t s);
 void launch_sqrt_check(uint32_t first, uint32_t count, unsigned long long *mismatches, uint32_t blocks, hipStream_t s);
-void launch_count_segments(const uint32_t *queue_count, uint32_t n, uint32_t first_count, const uint32_t *parts,
-                           unsigned long long *segments, hipStream_t s);
+void launch_count_segments(const SegmentCount &sc, hipStream_t s);
 
 // The static workspace of rayna_adjoint_static (a file-scope device array of adjoint_scratch_doubles()
 // doubles): its address on `device`, which must be the current device (taken on the first call per device).

@@ -70,7 +70,6 @@ __global__ __launch_bounds__(MARCH_BLOCK) __attribute__((amdgpu_waves_per_eu(8))
     const uint32_t n_items = count * n_sdf;
     const uint32_t refill_lanes = tune.refill_lanes;
     WaveClaims claims(n_items, MARCH_BLOCK / 64, MARCH_CLAIM_LEAST, tune.wave_batch * MARCH_CLAIM_FACTOR, work);
-    const uint32_t lane = __lane_id();
     bool active = false;
     int32_t j = 0;  // the lane's SDF
     MarchLane L{};

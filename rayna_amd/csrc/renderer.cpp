@@ -58,7 +58,7 @@ struct rayna_renderer {
     // SEGMENT_WORDS of k_trace's query counters, then claim counters: CLAIM_WORDS for k_extend (or k_trace) and for
     // k_march per depth, and for queries
     uint32_t *claims = nullptr;
-    unsigned long long *segments = nullptr;
+    unsigned long long *segments = nullptr;  // a call's closest-hit queries, in pinned host memory the kernels write to
     float *sum = nullptr, *acc = nullptr, *out_dev = nullptr;
     uint8_t *rgba_dev = nullptr;  // the 8-bit output of rayna_render_srgb8
     uint64_t rgba_cap = 0;
@@ -87,6 +87,7 @@ struct rayna_renderer {
     std::vector<hipEvent_t> events;
     // the last pass over a chunk: the event triples it recorded, and whether the first was of the camera rays alone
     size_t pass_marks = 1;
+    std::vector<size_t> marks;  // of the call so far: the event each mark stands for
     bool camera_apart = true;
     // debug validation (shared/validate.rs): RAYNA_CHECKS counters, counted in PBR frames while `validate`
     uint32_t *checks = nullptr;
@@ -230,7 +231,6 @@ void free_paths(rayna_renderer *r) {
     r->queue[0] = r->queue[1] = nullptr;
     r->queue_count = nullptr;
     r->claims = nullptr;
-    r->segments = nullptr;
     r->sum = r->acc = r->out_dev = nullptr;
     r->dimg = nullptr;
     r->primal_frame = -1;
@@ -309,12 +309,12 @@ rayna_status alloc_paths(rayna_renderer *r) {
     if ((st = alloc(slots * sizeof(uint32_t), (void **)&r->pb.hit_sub)) != RAYNA_OK) return st;
     for (int q = 0; q < 2; ++q)
         if ((st = alloc(slots * sizeof(int32_t), (void **)&r->queue[q])) != RAYNA_OK) return st;
-    if ((st = alloc(qlen * sizeof(uint32_t), (void **)&r->queue_count)) != RAYNA_OK) return st;
-    if ((st = alloc((SEGMENT_WORDS + (size_t)(o.ray_depth + 3) * 2 * CLAIM_WORDS) * sizeof(uint32_t),
-                    (void **)&r->claims)) !=
-        RAYNA_OK)
+    // the queue counters and, on the next line, the query and claim counters: one fill clears them
+    const uint32_t qpad = (qlen + 31u) / 32u * 32u;
+    if ((st = alloc((qpad + SEGMENT_WORDS + (size_t)(o.ray_depth + 3) * 2 * CLAIM_WORDS) * sizeof(uint32_t),
+                    (void **)&r->queue_count)) != RAYNA_OK)
         return st;
-    if ((st = alloc(sizeof(unsigned long long), (void **)&r->segments)) != RAYNA_OK) return st;
+    r->claims = r->queue_count + qpad;
     if ((st = alloc(3 * P * sizeof(float), (void **)&r->sum)) != RAYNA_OK) return st;
     if ((st = alloc(3 * P * sizeof(float), (void **)&r->acc)) != RAYNA_OK) return st;
     if ((st = alloc(3 * P * sizeof(float), (void **)&r->out_dev)) != RAYNA_OK) return st;
@@ -367,18 +367,23 @@ FrameParams frame_params(const rayna_renderer *r, uint64_t frame_index) {
 }
 
 // Trace the samples [s0, s0 + n) of every pixel: extend and shade per depth, from launched_depths on whole paths.  With `adjoint`, the
-// replay of path replay backpropagation: the radiance field must hold the chunk's primal radiance.
-void trace_chunk(rayna_renderer *r, FrameParams &fp, uint32_t s0, uint32_t n, std::vector<hipEvent_t> *ev, size_t *evi,
-                 uint64_t *extend_launches, const AdjointParams *adjoint = nullptr) {
+// replay of path replay backpropagation: the radiance field must hold the chunk's primal radiance.  Returns the count of
+// the chunk's queries, to be launched after it (first: the call's first chunk).
+SegmentCount trace_chunk(rayna_renderer *r, FrameParams &fp, uint32_t s0, uint32_t n, std::vector<hipEvent_t> *ev, size_t *evi,
+                 uint64_t *extend_launches, bool first, const AdjointParams *adjoint = nullptr) {
     fp.s0 = s0;
     fp.n_spp = n;
     fp.n_slots = fp.n_pixels * n;
     const uint32_t D2 = r->opts.ray_depth + 2;
-    launch_fill_u32(r->queue_count, 0u, 3 * D2, r->stream);
-    launch_fill_u32(r->claims, 0u, SEGMENT_WORDS + D2 * 2 * CLAIM_WORDS, r->stream);
+    launch_fill_u32(r->queue_count, 0u, (uint32_t)(r->claims - r->queue_count) + SEGMENT_WORDS + D2 * 2 * CLAIM_WORDS,
+                    r->stream);
     uint32_t *claims = r->claims + SEGMENT_WORDS;
+    bool launched = true;  // since the last event
     auto mark = [&] {
-        if (ev) (void)hipEventRecord((*ev)[(*evi)++], r->stream);
+        if (!ev) return;
+        if (launched) (void)hipEventRecord((*ev)[(*evi)++], r->stream);
+        r->marks.push_back(*evi - 1);
+        launched = false;
     };
     const uint32_t depths = r->opts.ray_depth + 1;
     const uint32_t apart = std::min(depths, launched_depths(r->dev.view, fp, r->tune, BatchView{}));
@@ -399,6 +404,7 @@ void trace_chunk(rayna_renderer *r, FrameParams &fp, uint32_t s0, uint32_t n, st
         const bool rest = depth >= apart;  // this launch takes every path to its end
         mark();
         ++r->pass_marks;
+        launched = true;
         if (rest) {
             launch_trace(r->dev.view, fp, r->pb, qin, cin, depth, r->grid_extend, r->dev.overflow, work, r->claims,
                          r->tune, adjoint, BatchView{}, r->stream);
@@ -410,6 +416,7 @@ void trace_chunk(rayna_renderer *r, FrameParams &fp, uint32_t s0, uint32_t n, st
                          r->queue_count + 2 * D2 + depth, r->stream);
         }
         mark();
+        launched = fp.mode != RAYNA_MODE_PBR || !rest;
         if (fp.mode != RAYNA_MODE_PBR)  // render_px_once: the camera ray's hit coloured by the mode
             launch_shade_mode(r->dev.view, fp, r->pb, r->grid_shade, r->stream);
         else if (!rest)
@@ -418,7 +425,7 @@ void trace_chunk(rayna_renderer *r, FrameParams &fp, uint32_t s0, uint32_t n, st
         mark();
         if (rest || fp.mode != RAYNA_MODE_PBR) break;
     }
-    launch_count_segments(r->queue_count, apart, apart > 0 ? fp.n_slots : 0, r->claims, r->segments, r->stream);
+    return SegmentCount{r->queue_count, apart, apart > 0 ? fp.n_slots : 0u, r->claims, r->segments, first ? 1u : 0u};
 }
 
 rayna_status ensure_events(rayna_renderer *r, size_t n) {
@@ -430,17 +437,18 @@ rayna_status ensure_events(rayna_renderer *r, size_t n) {
     return RAYNA_OK;
 }
 
-// Device times from the events of one call: events[0] before the first kernel, events[evi - 1] after the
-// last, and pass_marks triples [before extend, after extend, after shade] per pass over a chunk in between.
+// Device times from the events of one call: events[0] before the first kernel, events[evi - 1] after the last, and in
+// marks the events of the triples [before extend, after extend, after shade], pass_marks per pass over a chunk.
 rayna_status event_times(rayna_renderer *r, size_t evi, rayna_render_stats *st) {
     float ms = 0;
     HIP_TRY(r, hipEventElapsedTime(&ms, r->events[0], r->events[evi - 1]));
     st->kernel_ms = ms;
     double ext = 0, sh = 0, ext0 = 0;
-    for (size_t i = 1, k = 0; i + 2 < evi; i += 3, ++k) {
+    for (size_t k = 0; 3 * k + 2 < r->marks.size(); ++k) {
+        const size_t *m = &r->marks[3 * k];
         float a = 0, b = 0;
-        HIP_TRY(r, hipEventElapsedTime(&a, r->events[i], r->events[i + 1]));
-        HIP_TRY(r, hipEventElapsedTime(&b, r->events[i + 1], r->events[i + 2]));
+        HIP_TRY(r, hipEventElapsedTime(&a, r->events[m[0]], r->events[m[1]]));
+        if (m[2] != m[1]) HIP_TRY(r, hipEventElapsedTime(&b, r->events[m[1]], r->events[m[2]]));
         ext += a;
         sh += b;
         if (r->camera_apart && k % r->pass_marks == 0) ext0 += a;
@@ -466,6 +474,109 @@ uint32_t ilog2(uint32_t v) {
     uint32_t r = 0;
     while (v >>= 1) ++r;
     return r;
+}
+
+// rayna_render and, with out_rgba, rayna_render_srgb8: one frame, its image to out_rgb or converted to out_rgba.
+rayna_status render_frame(rayna_renderer *r, float *out_rgb, uint8_t *out_rgba, int32_t layout, uint32_t out_dims[2],
+                          rayna_render_stats *stats) {
+    if (!r) return fail(r, RAYNA_INVALID_ARGUMENT, "null renderer");
+    REQUIRE_LIVE(r);
+    if (layout != RAYNA_LAYOUT_XMAJOR && layout != RAYNA_LAYOUT_ROWMAJOR)
+        return fail(r, RAYNA_INVALID_ARGUMENT, "unknown layout");
+    const auto t0 = std::chrono::steady_clock::now();
+    HIP_TRY(r, hipSetDevice(r->device));
+    {
+        const rayna_status ms = ensure_mt(r);
+        if (ms != RAYNA_OK) return ms;
+    }
+    rayna_render_stats st{};
+    const uint32_t W = r->opts.width, H = r->opts.height;
+    if (!r->cam_valid) {
+        const uint32_t w2 = ilog2(W), h2 = ilog2(H);
+        if (out_rgb) write_checkerboard(w2, h2, out_rgb, layout);
+        if (out_rgba) {  // channels of exactly 0 and 1 map to 0 and 255
+            const uint64_t P = (uint64_t)w2 * h2;
+            std::vector<float> chk(3 * P);
+            write_checkerboard(w2, h2, chk.data(), RAYNA_LAYOUT_ROWMAJOR);
+            for (uint64_t p = 0; p < P; ++p) {
+                for (int c = 0; c < 3; ++c) out_rgba[4 * p + c] = chk[3 * p + c] >= 1.0f ? 255 : 0;
+                out_rgba[4 * p + 3] = 255;
+            }
+        }
+        if (out_dims) {
+            out_dims[0] = w2;
+            out_dims[1] = h2;
+        }
+        st.accum_frames = r->frames;
+    } else {
+        if (out_dims) {
+            out_dims[0] = W;
+            out_dims[1] = H;
+        }
+        const uint64_t P = (uint64_t)W * H;
+        if (out_rgba && r->rgba_cap < 4 * P) {
+            if (r->rgba_dev) (void)hipFree(r->rgba_dev);
+            r->rgba_dev = nullptr;
+            r->rgba_cap = 0;
+            HIP_TRY(r, hipMalloc((void **)&r->rgba_dev, 4 * P));
+            r->rgba_cap = 4 * P;
+        }
+        FrameParams fp = frame_params(r, r->frames);
+        if (r->validate && r->opts.mode == RAYNA_MODE_PBR) fp.checks = r->checks;
+        const uint32_t spp = r->opts.samples;
+        const uint32_t n_chunks = (spp + r->chunk_samples - 1) / r->chunk_samples;
+        std::vector<hipEvent_t> *ev = nullptr;
+        const size_t n_events = (size_t)n_chunks * (r->opts.ray_depth + 1) * 3 + 2;
+        if (stats) ev = &r->events;
+        if (ev) {
+            const rayna_status es = ensure_events(r, n_events);
+            if (es != RAYNA_OK) return es;
+        }
+        const int64_t frame_index = (int64_t)r->frames;
+        r->frames += 1;
+        const FrameOutput out{r->acc, r->out_dev, (double)r->frames, layout, r->acc_dirty ? 1u : 0u};
+        r->acc_dirty = false;
+        r->marks.clear();
+        size_t evi = 0;
+        if (ev) HIP_TRY(r, hipEventRecord((*ev)[evi++], r->stream));
+        uint64_t launches = 0;
+        for (uint32_t c = 0; c < n_chunks; ++c) {
+            const uint32_t s0 = c * r->chunk_samples;
+            const uint32_t n = std::min(r->chunk_samples, spp - s0);
+            const SegmentCount sc = trace_chunk(r, fp, s0, n, ev, &evi, &launches, c == 0);
+            fp.n_slots = fp.n_pixels * n;
+            launch_resolve(fp, r->pb, r->sum, n, c == 0 ? 1 : 0, sc, c + 1 == n_chunks && !fp.checks ? &out : nullptr,
+                           r->stream);
+        }
+        if (fp.checks) launch_finalize(fp, r->sum, out, r->stream);
+        r->primal_frame = n_chunks == 1 ? frame_index : -1;
+        if (ev) HIP_TRY(r, hipEventRecord((*ev)[evi++], r->stream));
+        {
+            const rayna_status ls = launch_status(r, "render");
+            if (ls != RAYNA_OK) return ls;
+        }
+        if (out_rgb)
+            HIP_TRY_LAUNCHED(
+                r, hipMemcpyAsync(out_rgb, r->out_dev, 3 * P * sizeof(float), hipMemcpyDeviceToHost, r->stream));
+        if (out_rgba) {
+            launch_to_srgb8(r->out_dev, (uint32_t)P, r->rgba_dev, r->stream);
+            const rayna_status ls = launch_status(r, "render_srgb8");
+            if (ls != RAYNA_OK) return ls;
+            HIP_TRY_LAUNCHED(r, hipMemcpyAsync(out_rgba, r->rgba_dev, 4 * P, hipMemcpyDeviceToHost, r->stream));
+        }
+        HIP_TRY_LAUNCHED(r, hipStreamSynchronize(r->stream));
+        st.accum_frames = r->frames;
+        st.samples = P * spp;
+        st.segments = *r->segments;
+        st.extend_launches = launches;
+        if (ev) {
+            const rayna_status ts = event_times(r, evi, &st);
+            if (ts != RAYNA_OK) return ts;
+        }
+    }
+    st.duration_s = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
+    if (stats) *stats = st;
+    return RAYNA_OK;
 }
 
 }  // namespace
@@ -494,6 +605,11 @@ rayna_status rayna_create(const rayna_scene_desc *scene, const rayna_camera *cam
         return bail(RAYNA_DEVICE_ERROR);
     }
     if ((st = set_grid(r)) != RAYNA_OK) return bail(st);
+    if (hipHostMalloc((void **)&r->segments, sizeof(unsigned long long), hipHostMallocPortable | hipHostMallocMapped) !=
+        hipSuccess) {
+        r->error = "no pinned host memory";
+        return bail(RAYNA_OUT_OF_MEMORY);
+    }
     r->opts = *opts;
     r->cam = *camera;
     r->cam_valid = viewport(r->cam, r->vp);
@@ -547,121 +663,12 @@ rayna_status rayna_clear_accumulation(rayna_renderer *r) {
 
 rayna_status rayna_render(rayna_renderer *r, float *out_rgb, int32_t layout, uint32_t out_dims[2],
                           rayna_render_stats *stats) {
-    if (!r) return fail(r, RAYNA_INVALID_ARGUMENT, "null renderer");
-    REQUIRE_LIVE(r);
-    if (layout != RAYNA_LAYOUT_XMAJOR && layout != RAYNA_LAYOUT_ROWMAJOR)
-        return fail(r, RAYNA_INVALID_ARGUMENT, "unknown layout");
-    const auto t0 = std::chrono::steady_clock::now();
-    HIP_TRY(r, hipSetDevice(r->device));
-    {
-        const rayna_status ms = ensure_mt(r);
-        if (ms != RAYNA_OK) return ms;
-    }
-    rayna_render_stats st{};
-    const uint32_t W = r->opts.width, H = r->opts.height;
-    if (!r->cam_valid) {
-        const uint32_t w2 = ilog2(W), h2 = ilog2(H);
-        if (out_rgb) write_checkerboard(w2, h2, out_rgb, layout);
-        if (out_dims) {
-            out_dims[0] = w2;
-            out_dims[1] = h2;
-        }
-        st.accum_frames = r->frames;
-    } else {
-        if (out_dims) {
-            out_dims[0] = W;
-            out_dims[1] = H;
-        }
-        const uint64_t P = (uint64_t)W * H;
-        if (r->acc_dirty) {
-            HIP_TRY(r, hipMemsetAsync(r->acc, 0, 3 * P * sizeof(float), r->stream));
-            r->acc_dirty = false;
-        }
-        FrameParams fp = frame_params(r, r->frames);
-        if (r->validate && r->opts.mode == RAYNA_MODE_PBR) fp.checks = r->checks;
-        const int64_t frame_index = (int64_t)r->frames;
-        r->frames += 1;
-        HIP_TRY(r, hipMemsetAsync(r->segments, 0, sizeof(unsigned long long), r->stream));
-        const uint32_t spp = r->opts.samples;
-        const uint32_t n_chunks = (spp + r->chunk_samples - 1) / r->chunk_samples;
-        std::vector<hipEvent_t> *ev = nullptr;
-        const size_t n_events = (size_t)n_chunks * (r->opts.ray_depth + 1) * 3 + 2;
-        if (stats) ev = &r->events;
-        if (ev) {
-            const rayna_status es = ensure_events(r, n_events);
-            if (es != RAYNA_OK) return es;
-        }
-        size_t evi = 0;
-        if (ev) HIP_TRY(r, hipEventRecord((*ev)[evi++], r->stream));
-        uint64_t launches = 0;
-        for (uint32_t c = 0; c < n_chunks; ++c) {
-            const uint32_t s0 = c * r->chunk_samples;
-            const uint32_t n = std::min(r->chunk_samples, spp - s0);
-            trace_chunk(r, fp, s0, n, ev, &evi, &launches);
-            fp.n_slots = fp.n_pixels * n;
-            launch_resolve(fp, r->pb, r->sum, n, c == 0 ? 1 : 0, r->stream);
-        }
-        launch_finalize(fp, r->sum, r->acc, (double)r->frames, r->out_dev, layout, r->stream);
-        r->primal_frame = n_chunks == 1 ? frame_index : -1;
-        if (ev) HIP_TRY(r, hipEventRecord((*ev)[evi++], r->stream));
-        {
-            const rayna_status ls = launch_status(r, "render");
-            if (ls != RAYNA_OK) return ls;
-        }
-        if (out_rgb)
-            HIP_TRY_LAUNCHED(
-                r, hipMemcpyAsync(out_rgb, r->out_dev, 3 * P * sizeof(float), hipMemcpyDeviceToHost, r->stream));
-        unsigned long long segs = 0;
-        HIP_TRY_LAUNCHED(r, hipMemcpyAsync(&segs, r->segments, sizeof(segs), hipMemcpyDeviceToHost, r->stream));
-        HIP_TRY_LAUNCHED(r, hipStreamSynchronize(r->stream));
-        st.accum_frames = r->frames;
-        st.samples = P * spp;
-        st.segments = segs;
-        st.extend_launches = launches;
-        if (ev) {
-            const rayna_status ts = event_times(r, evi, &st);
-            if (ts != RAYNA_OK) return ts;
-        }
-    }
-    st.duration_s = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
-    if (stats) *stats = st;
-    return RAYNA_OK;
+    return render_frame(r, out_rgb, nullptr, layout, out_dims, stats);
 }
 
 rayna_status rayna_render_srgb8(rayna_renderer *r, uint8_t *out_rgba, uint32_t out_dims[2], rayna_render_stats *stats) {
     if (!r || !out_rgba) return fail(r, RAYNA_INVALID_ARGUMENT, "null argument");
-    uint32_t dims[2] = {0, 0};
-    const rayna_status st = rayna_render(r, nullptr, RAYNA_LAYOUT_ROWMAJOR, dims, stats);
-    if (st != RAYNA_OK) return st;
-    if (out_dims) {
-        out_dims[0] = dims[0];
-        out_dims[1] = dims[1];
-    }
-    const uint64_t P = (uint64_t)dims[0] * dims[1];
-    if (!r->cam_valid) {  // the checkerboard: channels of exactly 0 and 1 map to 0 and 255
-        std::vector<float> chk(3 * P);
-        write_checkerboard(dims[0], dims[1], chk.data(), RAYNA_LAYOUT_ROWMAJOR);
-        for (uint64_t p = 0; p < P; ++p) {
-            for (int c = 0; c < 3; ++c) out_rgba[4 * p + c] = chk[3 * p + c] >= 1.0f ? 255 : 0;
-            out_rgba[4 * p + 3] = 255;
-        }
-        return RAYNA_OK;
-    }
-    if (r->rgba_cap < 4 * P) {
-        if (r->rgba_dev) (void)hipFree(r->rgba_dev);
-        r->rgba_dev = nullptr;
-        r->rgba_cap = 0;
-        HIP_TRY(r, hipMalloc((void **)&r->rgba_dev, 4 * P));
-        r->rgba_cap = 4 * P;
-    }
-    launch_to_srgb8(r->out_dev, (uint32_t)P, r->rgba_dev, r->stream);
-    {
-        const rayna_status ls = launch_status(r, "render_srgb8");
-        if (ls != RAYNA_OK) return ls;
-    }
-    HIP_TRY_LAUNCHED(r, hipMemcpyAsync(out_rgba, r->rgba_dev, 4 * P, hipMemcpyDeviceToHost, r->stream));
-    HIP_TRY_LAUNCHED(r, hipStreamSynchronize(r->stream));
-    return RAYNA_OK;
+    return render_frame(r, nullptr, out_rgba, RAYNA_LAYOUT_ROWMAJOR, out_dims, stats);
 }
 
 rayna_status rayna_set_tuning(rayna_renderer *r, const rayna_tuning *t) {
@@ -782,7 +789,6 @@ rayna_status rayna_adjoint(rayna_renderer *r, uint32_t frame, const float *d_ima
         }
     HIP_TRY(r, hipMemcpyAsync(r->dimg, d.data(), d.size() * sizeof(float), hipMemcpyHostToDevice, r->stream));
     HIP_TRY(r, hipMemsetAsync(r->grad, 0, per_copy * copies, r->stream));
-    HIP_TRY(r, hipMemsetAsync(r->segments, 0, sizeof(unsigned long long), r->stream));
 
     const uint32_t spp = r->opts.samples;
     const uint32_t n_chunks = (spp + r->chunk_samples - 1) / r->chunk_samples;
@@ -796,13 +802,16 @@ rayna_status rayna_adjoint(rayna_renderer *r, uint32_t frame, const float *d_ima
     }
     std::vector<hipEvent_t> *ev = stats ? &r->events : nullptr;
     size_t evi = 0;
+    r->marks.clear();
     if (ev) HIP_TRY(r, hipEventRecord((*ev)[evi++], r->stream));
     uint64_t launches = 0;
     for (uint32_t c = 0; c < n_chunks; ++c) {
         const uint32_t s0 = c * r->chunk_samples;
         const uint32_t n = std::min(r->chunk_samples, spp - s0);
-        if (!reuse) trace_chunk(r, fp, s0, n, ev, &evi, &launches);  // primal pass: the chunk's radiance
-        trace_chunk(r, fp, s0, n, ev, &evi, &launches, &ap);         // adjoint replay
+        if (!reuse)  // primal pass: the chunk's radiance
+            launch_count_segments(trace_chunk(r, fp, s0, n, ev, &evi, &launches, c == 0), r->stream);
+        // adjoint replay
+        launch_count_segments(trace_chunk(r, fp, s0, n, ev, &evi, &launches, c == 0 && reuse, &ap), r->stream);
     }
     launch_sum_grad(r->grad, 3 * n_materials, copies, r->grad_sum, r->stream);
     if (ev) HIP_TRY(r, hipEventRecord((*ev)[evi++], r->stream));
@@ -811,8 +820,6 @@ rayna_status rayna_adjoint(rayna_renderer *r, uint32_t frame, const float *d_ima
         if (ls != RAYNA_OK) return ls;
     }
     HIP_TRY_LAUNCHED(r, hipMemcpyAsync(grad_rgb, r->grad_sum, per_copy, hipMemcpyDeviceToHost, r->stream));
-    unsigned long long segs = 0;
-    HIP_TRY_LAUNCHED(r, hipMemcpyAsync(&segs, r->segments, sizeof(segs), hipMemcpyDeviceToHost, r->stream));
     HIP_TRY_LAUNCHED(r, hipStreamSynchronize(r->stream));
     // the radiance field now holds what the replay left of it
     r->primal_frame = -1;
@@ -822,7 +829,7 @@ rayna_status rayna_adjoint(rayna_renderer *r, uint32_t frame, const float *d_ima
         if (ts != RAYNA_OK) return ts;
         st.accum_frames = r->frames;
         st.samples = P * spp;
-        st.segments = segs;
+        st.segments = *r->segments;
         st.extend_launches = launches;
         st.duration_s = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
         *stats = st;
@@ -852,9 +859,8 @@ rayna_status rayna_adjoint_static(rayna_renderer *r, uint32_t frame, const float
     double *ws = nullptr;
     HIP_TRY(r, adjoint_scratch(r->device, &ws));
     const uint32_t copies = (uint32_t)std::min<uint64_t>(64, cap / per_copy);
-    // the workspace keeps the last call's contents: clear the copies (a fill kernel, no memset) and the counter
+    // the workspace keeps the last call's contents: clear the copies (a fill kernel, no memset)
     launch_fill_u32(reinterpret_cast<uint32_t *>(ws), 0u, (uint32_t)(2 * per_copy * copies), r->stream);
-    launch_fill_u32(reinterpret_cast<uint32_t *>(r->segments), 0u, 2, r->stream);
     const uint32_t spp = r->opts.samples;
     const uint32_t n_chunks = (spp + r->chunk_samples - 1) / r->chunk_samples;
     const bool reuse = n_chunks == 1 && r->primal_frame == (int64_t)frame;
@@ -864,8 +870,8 @@ rayna_status rayna_adjoint_static(rayna_renderer *r, uint32_t frame, const float
     for (uint32_t c = 0; c < n_chunks; ++c) {
         const uint32_t s0 = c * r->chunk_samples;
         const uint32_t n = std::min(r->chunk_samples, spp - s0);
-        if (!reuse) trace_chunk(r, fp, s0, n, nullptr, nullptr, &launches);
-        trace_chunk(r, fp, s0, n, nullptr, nullptr, &launches, &ap);
+        if (!reuse) (void)trace_chunk(r, fp, s0, n, nullptr, nullptr, &launches, c == 0);
+        (void)trace_chunk(r, fp, s0, n, nullptr, nullptr, &launches, false, &ap);
     }
     launch_sum_grad(ws, 3 * n_materials, copies, grad_dev, r->stream);
     {
@@ -1008,6 +1014,7 @@ void rayna_destroy(rayna_renderer *r) {
     if (r->sdf_buf) (void)hipFree(r->sdf_buf);
     if (r->rgba_dev) (void)hipFree(r->rgba_dev);
     if (r->checks) (void)hipFree(r->checks);
+    if (r->segments) (void)hipHostFree(r->segments);
     for (hipEvent_t e : r->events) (void)hipEventDestroy(e);
     if (r->stream) (void)hipStreamDestroy(r->stream);
     delete r;

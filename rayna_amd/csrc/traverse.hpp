@@ -380,7 +380,6 @@ __global__ __launch_bounds__(EXT_BLOCK) __attribute__((amdgpu_waves_per_eu(
     const uint32_t refill_lanes = tune.refill_lanes;
     dm::Key key{fp.key0, fp.key1};
     const uint32_t gid = blockIdx.x * EXT_BLOCK + threadIdx.x;
-    const uint32_t lane = __lane_id();
     LaneStack st{(lds_u64 *)s_entry, overflow + gid, gridDim.x * EXT_BLOCK, 0};
     bool active = false;
     uint32_t slot = 0, pixel = 0, sample = 0;
