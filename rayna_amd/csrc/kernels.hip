@@ -591,6 +591,7 @@ __device__ __forceinline__ void append_strip(const uint32_t *mine, uint32_t n_ke
 }
 
 #include "traverse.hpp"
+#include "quad.hpp"
 #include "march.hpp"
 
 // ------------------------------------------------------------------------------------------ shading
@@ -1464,14 +1465,19 @@ inline unsigned grid_for(uint64_t n, int block) { return (unsigned)((n + block -
 }  // namespace
 
 using TraceKernel = void (*)(TraceArgs);
-// The k_trace instantiations, [batch, adjoint, neither][textures][instances][form], forms as EXTEND_KERNELS'.
-#define RAYNA_TRACE_FORMS(B, T, I, A)                                                                   \
-    {k_trace<B, I, false, false, T, A>, k_trace<B, I, true, false, T, A>, k_trace<B, I, true, true, T, A>}
-#define RAYNA_TRACE_SET(B, A)                                                                            \
-    {{RAYNA_TRACE_FORMS(B, false, false, A), RAYNA_TRACE_FORMS(B, false, true, A)},                      \
-     {RAYNA_TRACE_FORMS(B, true, false, A), RAYNA_TRACE_FORMS(B, true, true, A)}}
+// The k_trace instantiations, [batch, adjoint, neither][textures][instances][form], forms as EXTEND_KERNELS'; and with
+// four lanes to a path, [batch, adjoint, neither][textures][form].
+#define RAYNA_TRACE_FORMS(Q, B, T, I, A)                                                                         \
+    {k_trace<Q, B, I, false, false, T, A>, k_trace<Q, B, I, true, false, T, A>, k_trace<Q, B, I, true, true, T, A>}
+#define RAYNA_TRACE_SET(B, A)                                                                                    \
+    {{RAYNA_TRACE_FORMS(false, B, false, false, A), RAYNA_TRACE_FORMS(false, B, false, true, A)},                \
+     {RAYNA_TRACE_FORMS(false, B, true, false, A), RAYNA_TRACE_FORMS(false, B, true, true, A)}}
+#define RAYNA_QUAD_SET(B, A) {RAYNA_TRACE_FORMS(true, B, false, false, A), RAYNA_TRACE_FORMS(true, B, true, false, A)}
 const TraceKernel TRACE_KERNELS[3][2][2][3] = {RAYNA_TRACE_SET(false, false), RAYNA_TRACE_SET(true, false),
                                                RAYNA_TRACE_SET(false, true)};
+const TraceKernel QUAD_KERNELS[3][2][3] = {RAYNA_QUAD_SET(false, false), RAYNA_QUAD_SET(true, false),
+                                           RAYNA_QUAD_SET(false, true)};
+#undef RAYNA_QUAD_SET
 #undef RAYNA_TRACE_SET
 #undef RAYNA_TRACE_FORMS
 
@@ -1501,6 +1507,7 @@ struct ExtendOccupancy {
     int n[2][2][3];
     int trace[3][2][2][3];
     int trace_sdf[3][3];
+    int quad[3][2][3];
     int most;
 };
 template <class Kernel>
@@ -1521,6 +1528,10 @@ const ExtendOccupancy &extend_occupancy() {
                 if (i == 0)
                     for (int k = 0; k < 3; ++k)
                         o.most = std::max(o.most, o.trace_sdf[k][f] = resident_blocks(TRACE_SDF_KERNELS[k][f]));
+                if (i == 0)
+                    for (int k = 0; k < 3; ++k)
+                        for (int t = 0; t < 2; ++t)
+                            o.most = std::max(o.most, o.quad[k][t][f] = resident_blocks(QUAD_KERNELS[k][t][f]));
                 for (int k = 0; k < 3; ++k)
                     for (int t = 0; t < 2; ++t)
                         o.most = std::max(o.most, o.trace[k][t][i][f] = resident_blocks(TRACE_KERNELS[k][t][i][f]));
@@ -1598,8 +1609,17 @@ void launch_trace(const SceneView &sv, const FrameParams &fp, const PathBuffers 
     const int k = bv.reqs ? 1 : adjoint ? 2 : 0, t = sv.textured ? 1 : 0, i = sv.instances ? 1 : 0;
     const int f = extend_form(sv), fs = i || t ? 2 : f ? 1 : 0;
     const ExtendOccupancy &o = extend_occupancy();
-    const TraceKernel kernel = sv.n_sdfs > 0 ? TRACE_SDF_KERNELS[k][fs] : TRACE_KERNELS[k][t][i][f];
-    const int resident = sv.n_sdfs > 0 ? o.trace_sdf[k][fs] : o.trace[k][t][i][f];
+    // Four lanes to a path where the launch is too small to be bound by anything but its longest paths; the larger the
+    // tree, the longer that holds.  (One launch per frame, a lane and four lanes to a path: 64x36x1 over 82 K triangles
+    // 0.49 and 0.27 ms, 480 spheres 0.27 and 0.16, Cornell 0.17 and 0.11; 640x360x1 1.02 and 0.77, 0.62 and 0.41, 0.25
+    // and 0.29; 1280x720x1 1.79 and 1.53, 0.85 and 0.90, 0.52 and 0.71; 1280x720x4 3.0 and 4.4, 1.5 and 2.7, 1.1 and
+    // 2.1.)
+    const uint64_t quad_slots = std::min<uint64_t>(1u << 20, std::max<uint64_t>(1u << 17, 4096ull * sv.n_nodes));
+    const bool quad = !i && fp.n_slots <= quad_slots;
+    const TraceKernel kernel = sv.n_sdfs > 0 ? TRACE_SDF_KERNELS[k][fs]
+                               : quad        ? QUAD_KERNELS[k][t][f]
+                                             : TRACE_KERNELS[k][t][i][f];
+    const int resident = sv.n_sdfs > 0 ? o.trace_sdf[k][fs] : quad ? o.quad[k][t][f] : o.trace[k][t][i][f];
     const int g = std::max(1, std::min(grid, grid / o.most * resident));
     const TraceArgs args{sv,   fp,   pb,       queue, count,    first_depth,
                          overflow, work, segments, tune,  adjoint ? *adjoint : AdjointParams{}, bv};

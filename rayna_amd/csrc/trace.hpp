@@ -19,6 +19,9 @@ constexpr int trace_waves(bool inst, bool sph, bool vol) { return inst || vol ? 
 
 // Fewest paths a wave claims, as EXTEND_CLAIM_LEAST (at 16 the 64x36, 2-sample sphere frame takes 417 us, not 344).
 constexpr uint32_t TRACE_CLAIM_LEAST = 4;
+// With four lanes to a path a wave holds sixteen: more at a time would leave the others idle (the four mesh preview
+// frames at most 8, 16 and 32: 2.74, 2.73 and 3.18 ms; the sphere thumbnail at least 1, 2 and 4: 161, 171 and 170 us).
+constexpr uint32_t QUAD_CLAIM_LEAST = 1, QUAD_CLAIM_MOST = 16;
 
 // The arguments of k_trace and k_trace_sdf, one struct so that a kernel finds them at the start of its argument segment.
 struct TraceArgs {
@@ -46,7 +49,10 @@ __device__ __forceinline__ const TraceArgs &cold_args() {
 
 // first_depth 0: the paths are the chunk's slots, from their camera rays (computed here).  first_depth > 0: the paths
 // are queue[0 .. *count_ptr), which k_shade kept at depth 0, from their stored rays and throughputs.
-template <bool BATCH, bool INST, bool SPH, bool VOL, bool TEX, bool ADJOINT>
+//
+// QUAD: four lanes to a path (quad.hpp): all of them hold it, the first one shades and takes new paths.  Without
+// instances.
+template <bool QUAD, bool BATCH, bool INST, bool SPH, bool VOL, bool TEX, bool ADJOINT>
 __global__ __launch_bounds__(EXT_BLOCK) __attribute__((amdgpu_waves_per_eu(trace_waves(INST, SPH, VOL)))) void k_trace(
     TraceArgs args) {
     __shared__ unsigned long long s_entry[EXT_LDS_STACK * EXT_BLOCK];
@@ -63,7 +69,9 @@ __global__ __launch_bounds__(EXT_BLOCK) __attribute__((amdgpu_waves_per_eu(trace
                                       : 64u;
     const uint32_t gid = blockIdx.x * EXT_BLOCK + threadIdx.x;
     const uint32_t lane = __lane_id();
+    const bool lead = !QUAD || (lane & 3u) == 0u;
     LaneStack st{(lds_u64 *)s_entry, args.overflow + gid, gridDim.x * EXT_BLOCK, 0};
+    QuadStack qst{(lds_u64 *)s_entry, args.overflow + (gid & ~3u), gridDim.x * EXT_BLOCK};
     enum : int { IDLE, TRACING, HIT };  // no path; a ray in the tree; its closest hit found
     int state = IDLE;
     uint32_t slot = 0, depth = 0, n_segments = 0;
@@ -71,7 +79,8 @@ __global__ __launch_bounds__(EXT_BLOCK) __attribute__((amdgpu_waves_per_eu(trace
     Best b{FLT_MAX, -1, 0u, 0u, 0u};
     LeafRange leaf;
     TravStats stats;
-    WaveClaims claims(count, EXT_BLOCK / 64, TRACE_CLAIM_LEAST, args.tune.wave_batch, args.work);
+    WaveClaims claims(count, EXT_BLOCK / 64, QUAD ? QUAD_CLAIM_LEAST : TRACE_CLAIM_LEAST,
+                      QUAD ? QUAD_CLAIM_MOST : args.tune.wave_batch, args.work);
     // the path's RNG key, pixel and sample, and in a batch its request
     auto identify = [&](const TraceArgs &A, dm::Key *key, uint32_t *pixel, uint32_t *sample) -> const RequestParams * {
         if (BATCH) {
@@ -96,7 +105,7 @@ __global__ __launch_bounds__(EXT_BLOCK) __attribute__((amdgpu_waves_per_eu(trace
         if (waiting == ~0ull || (claims.exhausted ? 2u * n_hit >= 64u - n_idle : n_idle + n_hit >= refill_lanes)) {
             const TraceArgs &A = cold_args();
             bool begin = false;
-            if (state == HIT) {
+            if (state == HIT && lead) {
                 dm::Key key;
                 uint32_t pixel, sample;
                 const RequestParams *R = identify(A, &key, &pixel, &sample);
@@ -125,10 +134,10 @@ __global__ __launch_bounds__(EXT_BLOCK) __attribute__((amdgpu_waves_per_eu(trace
                 }
                 state = IDLE;
             }
-            idle = __ballot(state == IDLE && !begin);
+            idle = __ballot(state == IDLE && !begin && lead);
             if (!claims.exhausted && idle != 0ull) {
                 const uint32_t q = claims.hand_out(idle);
-                if (state == IDLE && !begin && q != 0xffffffffu) {
+                if (state == IDLE && !begin && lead && q != 0xffffffffu) {
                     slot = A.queue ? (uint32_t)A.queue[q] : q;
                     depth = A.first_depth;
                     Col T{1.0f, 1.0f, 1.0f};
@@ -150,6 +159,20 @@ __global__ __launch_bounds__(EXT_BLOCK) __attribute__((amdgpu_waves_per_eu(trace
                     begin = true;
                 }
             }
+            if (QUAD) {  // the first lane's path to all four
+                state = (int)quad_perm<QUAD_FIRST>((uint32_t)state);
+                begin = quad_perm<QUAD_FIRST>(begin ? 1u : 0u) != 0u;
+                if (begin) {
+                    slot = quad_perm<QUAD_FIRST>(slot);
+                    depth = quad_perm<QUAD_FIRST>(depth);
+                    ray.o = f3{quad_perm<QUAD_FIRST>(ray.o.x), quad_perm<QUAD_FIRST>(ray.o.y),
+                               quad_perm<QUAD_FIRST>(ray.o.z)};
+                    ray.d = f3{quad_perm<QUAD_FIRST>(ray.d.x), quad_perm<QUAD_FIRST>(ray.d.y),
+                               quad_perm<QUAD_FIRST>(ray.d.z)};
+                    ray.inv = f3{quad_perm<QUAD_FIRST>(ray.inv.x), quad_perm<QUAD_FIRST>(ray.inv.y),
+                                 quad_perm<QUAD_FIRST>(ray.inv.z)};
+                }
+            }
             if (begin) {
                 int32_t root = A.sv.root;
                 if (BATCH) root = A.bv.reqs[A.bv.slot_req[slot]].root;
@@ -163,12 +186,19 @@ __global__ __launch_bounds__(EXT_BLOCK) __attribute__((amdgpu_waves_per_eu(trace
                     A.pb.dz[slot] = ray.d.z;
                 }
                 b = Best{FLT_MAX, -1, 0u, 0u, 0u};
-                st.sp = 0;
-                st.top_valid = false;
-                if (root >= 0) st.push(root, -__builtin_inff());
-                leaf.code = 0;
+                if (QUAD) {
+                    qst.sp = 0;
+                    qst.has = root >= 0;
+                    qst.code = root;
+                    qst.t = 0.0f;
+                } else {
+                    st.sp = 0;
+                    st.top_valid = false;
+                    if (root >= 0) st.push(root, -__builtin_inff());
+                    leaf.code = 0;
+                }
                 state = TRACING;
-                ++n_segments;
+                if (lead) ++n_segments;
             }
         }
         if (!__any(state == TRACING)) {
@@ -176,8 +206,13 @@ __global__ __launch_bounds__(EXT_BLOCK) __attribute__((amdgpu_waves_per_eu(trace
             continue;
         }
         if (state == TRACING) {
-            traverse_pass<INST, SPH, VOL>(sv, args.pb, slot, ray, b, leaf, st, vkey, vpixel, vsample, depth, stats);
-            if (st.sp == 0 && leaf.code == 0) state = HIT;
+            if (QUAD) {
+                traverse_quad_pass<SPH, VOL>(sv, ray, b, qst, vkey, vpixel, vsample, depth);
+                if (!qst.has && qst.sp == 0) state = HIT;
+            } else {
+                traverse_pass<INST, SPH, VOL>(sv, args.pb, slot, ray, b, leaf, st, vkey, vpixel, vsample, depth, stats);
+                if (st.sp == 0 && leaf.code == 0) state = HIT;
+            }
         }
     }
     stats.flush();

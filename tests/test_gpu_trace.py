@@ -1,7 +1,8 @@
 """Paths traced to their ends in one launch against one launch per depth: validation keeps a frame on the latter (and
 changes no pixel), so every scene's two frames and closest-hit counts must be equal, whatever the depth limit, the
 samples per pixel (below and from 16 on, where the camera rays are packets), the number of chunks and, with unbounded
-objects, the number of paths (from 128 * 128 on the camera rays get launches of their own)."""
+objects, the number of paths (from 128 * 128 on the camera rays get launches of their own).  Up to 2^17 paths, for the
+largest trees 2^20, a path has four lanes, beyond that one."""
 import numpy as np
 import pytest
 
@@ -21,7 +22,9 @@ SCENES = {"mesh": lambda **k: presets.triangle_mesh(subdiv=3, **k), "spheres": p
 @pytest.mark.parametrize("width,height,samples,depth,chunk", [(1, 1, 1, 6, 0), (37, 23, 15, 0, 0), (37, 23, 16, 0, 0),
                                                              (37, 23, 17, 1, 0), (64, 64, 3, 7, 0), (33, 65, 40, 5, 0),
                                                              (64, 33, 40, 4, 64 * 33 * 17),
-                                                             (128, 127, 1, 4, 0), (128, 128, 1, 4, 0)])
+                                                             (128, 127, 1, 4, 0), (128, 128, 1, 4, 0),
+                                                             (363, 361, 1, 5, 0), (1025, 1024, 1, 3, 0),
+                                                             (257, 256, 16, 4, 0)])
 def test_one_launch_equals_one_per_depth(gpu, scene, width, height, samples, depth, chunk):
     sc, cam, opts = SCENES[scene](width=width, height=height, samples=samples, ray_depth=depth)
     frames = []
