@@ -8,6 +8,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -24,6 +25,30 @@ std::string g_create_error;
 
 // rayna_debug_fail_launches: < 0 off, else the number of launch checks still to pass before one fails
 std::atomic<int32_t> g_fail_launches{-1};
+
+// Words of pinned host memory that kernels write to, one per renderer.  They come in pages of 512 and are handed out
+// again when their renderer is destroyed (pinning memory for each renderer cost its creation 0.1-0.2 ms).
+std::mutex g_host_words_lock;
+std::vector<unsigned long long *> g_host_words;
+
+unsigned long long *take_host_word() {
+    std::lock_guard<std::mutex> lock(g_host_words_lock);
+    if (g_host_words.empty()) {
+        constexpr size_t WORDS = 512;
+        void *p = nullptr;
+        if (hipHostMalloc(&p, WORDS * sizeof(unsigned long long), hipHostMallocPortable | hipHostMallocMapped) != hipSuccess)
+            return nullptr;
+        for (size_t i = 0; i < WORDS; ++i) g_host_words.push_back(static_cast<unsigned long long *>(p) + i);
+    }
+    unsigned long long *w = g_host_words.back();
+    g_host_words.pop_back();
+    return w;
+}
+
+void give_host_word(unsigned long long *w) {
+    std::lock_guard<std::mutex> lock(g_host_words_lock);
+    g_host_words.push_back(w);
+}
 
 // Paths in flight per chunk: 2^27 (a 1080p frame of 64 samples in one chunk; ~10 GB of path state, sized for
 // the 288 GB of HBM of one MI355X).  Whole-frame chunks keep every depth's launch full: at 2^23 paths the
@@ -605,8 +630,7 @@ rayna_status rayna_create(const rayna_scene_desc *scene, const rayna_camera *cam
         return bail(RAYNA_DEVICE_ERROR);
     }
     if ((st = set_grid(r)) != RAYNA_OK) return bail(st);
-    if (hipHostMalloc((void **)&r->segments, sizeof(unsigned long long), hipHostMallocPortable | hipHostMallocMapped) !=
-        hipSuccess) {
+    if (!(r->segments = take_host_word())) {
         r->error = "no pinned host memory";
         return bail(RAYNA_OUT_OF_MEMORY);
     }
@@ -1014,7 +1038,7 @@ void rayna_destroy(rayna_renderer *r) {
     if (r->sdf_buf) (void)hipFree(r->sdf_buf);
     if (r->rgba_dev) (void)hipFree(r->rgba_dev);
     if (r->checks) (void)hipFree(r->checks);
-    if (r->segments) (void)hipHostFree(r->segments);
+    if (r->segments) give_host_word(r->segments);
     for (hipEvent_t e : r->events) (void)hipEventDestroy(e);
     if (r->stream) (void)hipStreamDestroy(r->stream);
     delete r;
