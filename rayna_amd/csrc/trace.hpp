@@ -105,6 +105,7 @@ __global__ __launch_bounds__(EXT_BLOCK) __attribute__((amdgpu_waves_per_eu(trace
         if (waiting == ~0ull || (claims.exhausted ? 2u * n_hit >= 64u - n_idle : n_idle + n_hit >= refill_lanes)) {
             const TraceArgs &A = cold_args();
             bool begin = false;
+            VertexGrad grad;
             if (state == HIT && lead) {
                 dm::Key key;
                 uint32_t pixel, sample;
@@ -115,7 +116,7 @@ __global__ __launch_bounds__(EXT_BLOCK) __attribute__((amdgpu_waves_per_eu(trace
                 const uint32_t at_depth = depth;
                 const Best hit = b;
                 begin = shade_vertex<ADJOINT, TEX, false, false>(
-                    A.sv, nullptr, A.ap, ADJOINT ? blockIdx.x % A.ap.copies : 0u, ray, hit.ref, &hit.t, &hit.aux, &hit.sub, false, f3{0.0f, 0.0f, 0.0f}, key,
+                    A.sv, nullptr, A.ap, grad, ray, hit.ref, &hit.t, &hit.aux, &hit.sub, false, f3{0.0f, 0.0f, 0.0f}, key,
                     pixel, sample, at_depth, BATCH ? R->ray_depth : A.fp.ray_depth, BATCH ? R->skybox : A.sv.skybox,
                     BATCH ? R->sky_image : A.sv.sky_image, T, L, add, [&](const DRay &nr, const Col &t) {
                         ray = ray_from_dir(nr.o, nr.d);
@@ -134,6 +135,7 @@ __global__ __launch_bounds__(EXT_BLOCK) __attribute__((amdgpu_waves_per_eu(trace
                 }
                 state = IDLE;
             }
+            if (ADJOINT) add_grads(A.ap, blockIdx.x % A.ap.copies, grad);
             idle = __ballot(state == IDLE && !begin && lead);
             if (!claims.exhausted && idle != 0ull) {
                 const uint32_t q = claims.hand_out(idle);

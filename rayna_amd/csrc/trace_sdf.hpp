@@ -67,6 +67,7 @@ __global__ __launch_bounds__(EXT_BLOCK) __attribute__((amdgpu_waves_per_eu(SDF_T
             (claims.exhausted ? 4u * n_hit >= 64u - n_idle : n_idle + n_hit >= SDF_REFILL_LANES)) {
             const TraceArgs &A = cold_args();
             bool begin = false;
+            VertexGrad grad;
             if (state == HIT) {
                 dm::Key key;
                 uint32_t pixel, sample;
@@ -77,7 +78,7 @@ __global__ __launch_bounds__(EXT_BLOCK) __attribute__((amdgpu_waves_per_eu(SDF_T
                 const uint32_t at_depth = depth;
                 const Best hit = b;
                 begin = shade_vertex<ADJOINT, TEX, false, false>(
-                    A.sv, nullptr, A.ap, ADJOINT ? blockIdx.x % A.ap.copies : 0u, ray, hit.ref, &hit.t, &hit.aux, &hit.sub, true, g, key, pixel, sample,
+                    A.sv, nullptr, A.ap, grad, ray, hit.ref, &hit.t, &hit.aux, &hit.sub, true, g, key, pixel, sample,
                     at_depth, BATCH ? R->ray_depth : A.fp.ray_depth, BATCH ? R->skybox : A.sv.skybox,
                     BATCH ? R->sky_image : A.sv.sky_image, T, L, add, [&](const DRay &nr, const Col &t) {
                         ray.o = nr.o;
@@ -97,6 +98,7 @@ __global__ __launch_bounds__(EXT_BLOCK) __attribute__((amdgpu_waves_per_eu(SDF_T
                 }
                 state = IDLE;
             }
+            if (ADJOINT) add_grads(A.ap, blockIdx.x % A.ap.copies, grad);
             const unsigned long long idle = __ballot(state == IDLE && !begin);
             if (!claims.exhausted && idle != 0ull) {
                 const uint32_t q = claims.hand_out(idle);
