@@ -24,7 +24,8 @@ HBM_PEAK_GBPS = 8000.0
 # Algorithmic bytes of one closest-hit query in the extend kernel: queue entry 4 B + ray origin and direction
 # 24 B read, hit distance, reference and flags 12 B written.
 EXTEND_BYTES_PER_SEGMENT = 40
-# Algorithmic bytes of the whole frame per segment (extend + shade) and per sample (generate + resolve):
+# Algorithmic bytes of the whole frame, as if every vertex went through memory between two launches (k_trace keeps the
+# later ones in registers), per segment (extend + shade) and per sample (generate + resolve):
 # extend 40 B; shade reads queue 4, ray 24, hit 12, throughput 12, radiance 12 and writes ray 24,
 # throughput 12, radiance 12, queue entry 4 -> 116 B; generate writes the 24 B camera ray per sample, resolve
 # reads 12 B.
@@ -32,17 +33,18 @@ FRAME_BYTES_PER_SEGMENT = 40 + 116
 FRAME_BYTES_PER_SAMPLE = 24 + 12
 # Counter-derived figures of the extend stage on the 1080p triangle-mesh frame, from rocprofv3 passes over two
 # frames of 263,040,107 closest-hit queries each (132,710,400 of them camera rays) at the commit that added them;
-# the times they are divided by are measured live.  Traffic (both extend kernels): what leaves L2 for the
-# fabric, FETCH_SIZE 4.1536e7 KiB read as 64-byte units (x2.0: a 256 MiB copy reads 131,087 KiB) plus WRITE_SIZE
-# 1.4767e7 KiB (x1.0: the copy writes 262,143 KiB); it counts hits in the Infinity Cache as well as HBM, so it
-# bounds the HBM bytes from above.  VALU (k_extend, depths 1-8): SQ_INSTS_VALU 3.3124e10 wave64 instructions over
-# 2 x 130,329,707 queries; lanes active SQ_THREAD_CYCLES_VALU / (64 SQ_ACTIVE_INST_VALU) = 7.9352e11 / (64 x
-# 3.3368e10); 0.878 instructions per CU per cycle (GRBM_GUI_ACTIVE 1.1794e9 over 8 XCDs, 256 CUs).
+# the times they are divided by are measured live.  The stage is k_extend_packet (camera rays), k_extend (the first
+# bounce) and k_trace (every later vertex, traversed and shaded).  Traffic: what leaves L2 for the fabric, FETCH_SIZE
+# 3.9936e7 KiB read as 64-byte units (x2.0: a 256 MiB copy reads 131,087 KiB) plus WRITE_SIZE 1.0291e7 KiB (x1.0: the
+# copy writes 262,143 KiB); it counts hits in the Infinity Cache as well as HBM, so it bounds the HBM bytes from above.
+# VALU (k_extend and k_trace, depths 1-8): SQ_INSTS_VALU 2.3102e10 + 1.4481e10 wave64 instructions over 2 x 130,329,707
+# queries; lanes active SQ_THREAD_CYCLES_VALU / (64 SQ_ACTIVE_INST_VALU) = (6.4028e11 + 3.0339e11) / (64 x 3.7870e10);
+# instructions per CU per cycle from GRBM_GUI_ACTIVE 6.9357e8 + 4.9982e8 over 8 XCDs, 256 CUs.
 EXTEND_COUNTER_FRAMES = 2 * 263040107
-EXTEND_FABRIC_BYTES_PER_SEGMENT = {"triangle_mesh": (4.1536e7 * 2.0 + 1.4767e7) * 1024 / EXTEND_COUNTER_FRAMES}
-K_EXTEND_VALU_PER_QUERY = {"triangle_mesh": 3.3124e10 / (2 * 130329707)}
-K_EXTEND_LANES_ACTIVE = {"triangle_mesh": 7.9352e11 / (64 * 3.3368e10)}
-K_EXTEND_VALU_PER_CU_CYCLE = {"triangle_mesh": 3.3124e10 / (1.1794e9 / 8 * 256)}
+EXTEND_FABRIC_BYTES_PER_SEGMENT = {"triangle_mesh": (3.9936e7 * 2.0 + 1.0291e7) * 1024 / EXTEND_COUNTER_FRAMES}
+K_EXTEND_VALU_PER_QUERY = {"triangle_mesh": 3.7583e10 / (2 * 130329707)}
+K_EXTEND_LANES_ACTIVE = {"triangle_mesh": 9.4367e11 / (64 * 3.7870e10)}
+K_EXTEND_VALU_PER_CU_CYCLE = {"triangle_mesh": 3.7583e10 / (1.19339e9 / 8 * 256)}
 # VALU issue peak: one wave64 instruction per CU per cycle -- the rate the calibration kernel
 # (rayna_measure_valu_peak: independent fp32 multiply-add chains, no packed or fused forms) reaches per active
 # cycle (0.977 by the same counters) -- at MI355X's published 256 CUs and 2.4 GHz.
@@ -59,9 +61,9 @@ def _progress(msg: str):
 
 
 def valu_roofline(workload: str, camera_rays: int, segs: int, ext_ms: float, cam_ms: float):
-    """k_extend (depths 1-8) against the VALU issue peak: its wave64 VALU instructions per closest-hit query
-    (counted by rocprofv3 on this workload) times this run's queries at those depths, over this run's k_extend
-    time (the extend launches' HIP events less the camera rays')."""
+    """k_extend and k_trace (depths 1-8, k_trace's shading included) against the VALU issue peak: their wave64 VALU
+    instructions per closest-hit query (counted by rocprofv3 on this workload) times this run's queries at those
+    depths, over this run's time in them (the extend launches' HIP events less the camera rays')."""
     per_q = K_EXTEND_VALU_PER_QUERY.get(workload)
     t = (ext_ms - cam_ms) * 1e-3
     if not per_q or t <= 0:
@@ -70,7 +72,8 @@ def valu_roofline(workload: str, camera_rays: int, segs: int, ext_ms: float, cam
     calib, _ = measure_valu_peak()
     achieved = per_q * (segs - camera_rays) / t / 1e9
     lanes = K_EXTEND_LANES_ACTIVE[workload]
-    return {"kernel": "k_extend (depths 1-8)", "achieved": achieved, "peak": VALU_PEAK_G,
+    return {"kernel": "k_extend (depth 1) and k_trace (depths 2-8, shading included)", "achieved": achieved,
+            "peak": VALU_PEAK_G,
             "unit": "G wave64 VALU instructions/s", "frac": achieved / VALU_PEAK_G, "insts_per_query": per_q,
             "lanes_active": lanes, "useful_frac": achieved / VALU_PEAK_G * lanes,
             "insts_per_cu_cycle_profiled": K_EXTEND_VALU_PER_CU_CYCLE[workload],
@@ -490,9 +493,10 @@ def main(argv=None):
         "scene_build_s": t_build,
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBPS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBPS, "traffic": traffic,
-                     "traffic_kind": "L2-miss (fabric) bytes per launch: rocprofv3 FETCH_SIZE + WRITE_SIZE, "
+                     "traffic_kind": "L2-miss (fabric) bytes per depth: rocprofv3 FETCH_SIZE + WRITE_SIZE, "
                                      "calibrated on a 256 MiB copy; Infinity Cache hits included",
-                     "kernel": "extend: k_extend_packet (camera rays) + k_extend (later depths)",
+                     "kernel": "extend: k_extend_packet (camera rays) + k_extend (first bounce) + k_trace (later "
+                               "vertices, shading included)",
                      "bytes_per_segment": EXTEND_BYTES_PER_SEGMENT},
     }
     valu = valu_roofline(a.workload, samples_per_frame * a.steps, segs, ext_ms, cam_ms)
