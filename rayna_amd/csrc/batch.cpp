@@ -35,6 +35,7 @@ enum : uint32_t {
     SCENE_MEDIA = 4u,
     SCENE_SDFS = 8u,
     SCENE_TEXTURED = 16u,
+    SCENE_MANDELBULBS = 32u,
 };
 
 // One request's share of a chunk: samples [s0, s0 + n) of request `req`.
@@ -421,6 +422,7 @@ SceneView chunk_view(const SceneView &merged, uint32_t features) {
     v.media = (features & SCENE_MEDIA) ? merged.media : 0;
     v.textured = (features & SCENE_TEXTURED) ? merged.textured : 0;
     v.n_sdfs = (features & SCENE_SDFS) ? merged.n_sdfs : 0;
+    v.mandelbulbs = (features & SCENE_MANDELBULBS) ? merged.mandelbulbs : 0;
     return v;
 }
 
@@ -574,6 +576,7 @@ rayna_status rayna_batch_create(const rayna_scene_desc *scenes, int32_t n_scenes
         if (has_spheres(p)) f |= SCENE_SPHERES;
         if (!p.volumes.empty()) f |= SCENE_MEDIA;
         if (!p.sdfs.empty()) f |= SCENE_SDFS;
+        if (has_mandelbulbs(p)) f |= SCENE_MANDELBULBS;
         if (has_textures(p) || p.skybox == RAYNA_SKY_HDRI) f |= SCENE_TEXTURED;
         b->scene_features[i] = f;
     }
@@ -612,6 +615,7 @@ rayna_status rayna_batch_create(const rayna_scene_desc *scenes, int32_t n_scenes
     v.root = -1;  // per request
     v.n_nodes = (int32_t)merged.nodes.size();
     v.n_sdfs = (int32_t)merged.sdfs.size();
+    v.mandelbulbs = has_mandelbulbs(merged) ? 1 : 0;
     v.skybox = RAYNA_SKY_NONE;
     v.stack_need = merged.stack_need;
     v.packet_need = merged.packet_need;

@@ -221,6 +221,7 @@ rayna_status load_scene(rayna_renderer *r, const rayna_scene_desc *d) {
     v.root = ps.root;
     v.n_nodes = (int32_t)ps.nodes.size();
     v.n_sdfs = (int32_t)ps.sdfs.size();
+    v.mandelbulbs = has_mandelbulbs(ps) ? 1 : 0;
     v.skybox = ps.skybox;
     v.stack_need = ps.stack_need;
     v.packet_need = ps.packet_need;

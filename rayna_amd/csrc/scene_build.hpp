@@ -67,6 +67,13 @@ inline bool has_instances(const PackedScene &p) {
     return false;
 }
 
+// True if some unbounded object of the packed scene is a Mandelbulb.
+inline bool has_mandelbulbs(const PackedScene &p) {
+    for (const GSdf &f : p.sdfs)
+        if (f.kind == RAYNA_SDF_MANDELBULB) return true;
+    return false;
+}
+
 // True if traversal of the packed scene intersects spheres: a sphere item (also inside a BVH mesh), a medium
 // bounded by a sphere, or a transformed sphere or sphere-bounded medium.
 inline bool has_spheres(const PackedScene &p) {

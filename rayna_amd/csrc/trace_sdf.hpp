@@ -17,11 +17,15 @@
 // one 76.1 -> 71.9 (launched_depths says which depths stay apart), the batch of 16 requests 29.1 -> 20.3.
 
 // Waves per SIMD (the 161x91, 9-sample SDF frame at 4, 5 and 6: 4.6, 4.5 and 4.2 ms, the 64x36, 2-sample one at 5 and
-// 6: 3.2 and 3.4, the 720p, 128-sample one 83 and 82), and the lanes that wait before a wave shades and takes new
-// paths (16, 24 and 32 within 2%); once there are none left to take, a quarter of its paths (the 161x91, 9-sample frame
-// at half, a quarter, an eighth and a sixty-fourth: 4.31, 4.19, 4.20 and 4.28 ms).
+// 6: 3.2 and 3.4, the 720p, 128-sample one 83 and 82), and the lanes that wait before a wave shades, takes new
+// paths and traces their rays through the tree: fewer where that is cheap beside a pass of estimates, as it is beside a
+// Mandelbulb's iterations, more where it is the work and estimates are cheap.  (At 16, 32 and 48: the Mandelbulb scene
+// at 1280x720x128 71.8, 76.0 and above 81 ms, at 640x360x64 17.2, 17.9 and 19.5; a scene of 60 bounded objects and one
+// sphere SDF at 1280x720x64 19.0, 14.2 and 13.5 ms, at 333x217x30 3.20, 2.72 and 2.64.)  Once there are no paths left to
+// take, a quarter of its paths (the 161x91, 9-sample frame at half, a quarter, an eighth and a sixty-fourth: 4.31, 4.19,
+// 4.20 and 4.28 ms).
 constexpr int SDF_TRACE_WAVES = 5;
-constexpr uint32_t SDF_REFILL_LANES = 32;
+constexpr uint32_t SDF_REFILL_LANES = 48, BULB_REFILL_LANES = 16;
 
 template <bool BATCH, bool INST, bool SPH, bool VOL, bool TEX, bool ADJOINT>
 __global__ __launch_bounds__(EXT_BLOCK) __attribute__((amdgpu_waves_per_eu(SDF_TRACE_WAVES))) void k_trace_sdf(
@@ -44,6 +48,7 @@ __global__ __launch_bounds__(EXT_BLOCK) __attribute__((amdgpu_waves_per_eu(SDF_T
     int step = 0;                     // the march's step; the normal's estimate (0..5: +x -x +y -y +z -z)
     f3 g{0.0f, 0.0f, 0.0f};           // the estimate's differences, then the normal
     WaveClaims claims(count, EXT_BLOCK / 64, TRACE_CLAIM_LEAST, args.tune.wave_batch, args.work);
+    const uint32_t refill_lanes = args.sv.mandelbulbs ? BULB_REFILL_LANES : SDF_REFILL_LANES;
     TravStats stats;
     // the path's RNG key, pixel and sample, and in a batch its request
     auto identify = [&](const TraceArgs &A, dm::Key *key, uint32_t *pixel, uint32_t *sample) -> const RequestParams * {
@@ -64,7 +69,7 @@ __global__ __launch_bounds__(EXT_BLOCK) __attribute__((amdgpu_waves_per_eu(SDF_T
         const unsigned long long paths = __ballot(state != IDLE), waiting = __ballot(state == HIT) | ~paths;
         const uint32_t n_idle = 64u - (uint32_t)__popcll(paths), n_hit = (uint32_t)__popcll(waiting) - n_idle;
         if (waiting == ~0ull ||
-            (claims.exhausted ? 4u * n_hit >= 64u - n_idle : n_idle + n_hit >= SDF_REFILL_LANES)) {
+            (claims.exhausted ? 4u * n_hit >= 64u - n_idle : n_idle + n_hit >= refill_lanes)) {
             const TraceArgs &A = cold_args();
             bool begin = false;
             VertexGrad grad;
