@@ -36,8 +36,11 @@ unsigned long long *take_host_word() {
     if (g_host_words.empty()) {
         constexpr size_t WORDS = 512;
         void *p = nullptr;
-        if (hipHostMalloc(&p, WORDS * sizeof(unsigned long long), hipHostMallocPortable | hipHostMallocMapped) != hipSuccess)
+        if (hipHostMalloc(&p, WORDS * sizeof(unsigned long long), hipHostMallocPortable | hipHostMallocMapped) !=
+            hipSuccess) {
+            (void)hipGetLastError();  // taken here: the thread's next launch check would read it as its own
             return nullptr;
+        }
         for (size_t i = 0; i < WORDS; ++i) g_host_words.push_back(static_cast<unsigned long long *>(p) + i);
     }
     unsigned long long *w = g_host_words.back();
@@ -1049,7 +1052,13 @@ rayna_status rayna_host_alloc(uint64_t bytes, void **out) {
     g_create_error.clear();
     if (!out || bytes == 0) return fail(nullptr, RAYNA_INVALID_ARGUMENT, "null output or no bytes");
     *out = nullptr;
-    HIP_TRY(nullptr, hipHostMalloc(out, bytes, hipHostMallocPortable));
+    const hipError_t e = hipHostMalloc(out, bytes, hipHostMallocPortable);
+    if (e != hipSuccess) {
+        // taken here: the thread's next launch check would read it as its own (callers go on with ordinary memory)
+        (void)hipGetLastError();
+        *out = nullptr;
+    }
+    HIP_TRY(nullptr, e);
     return RAYNA_OK;
 }
 

@@ -1,5 +1,6 @@
 """The pool of pinned image buffers: its bounds, reuse and fallbacks on a stand-in allocator, and on the GPU that an
 image is never overwritten while it or a view of it is held."""
+import ctypes as C
 import gc
 import threading
 
@@ -7,6 +8,8 @@ import numpy as np
 import pytest
 
 from rayna_amd import Renderer, host_buffers, presets, renderer
+from rayna_amd import _abi as A
+from rayna_amd.batch import BatchRenderer, Request
 
 
 class FakeLib:
@@ -96,3 +99,19 @@ def test_held_images_keep_their_values(gpu):
                 copies.append(out.img[1:].copy())
     for a, b in zip(frames, copies):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.gpu
+def test_failed_pinned_allocation_leaves_no_error_behind(gpu):
+    """More bytes than any machine has, refused through the real library: the frames and batches that follow on the
+    same thread take no notice, whichever entry point reads the runtime's last error next."""
+    sc, cam, opts = presets.cornell(width=33, height=21, samples=2)
+    with Renderer(sc, cam, opts) as r, BatchRenderer([sc]) as b:
+        ref = r.render(layout="rowmajor").img.copy()
+        p = C.c_void_p()
+        for _ in range(2):
+            assert renderer.lib().rayna_host_alloc(1 << 60, C.byref(p)) == A.RAYNA_OUT_OF_MEMORY and not p.value
+            r.clear_accumulation()
+            assert np.array_equal(r.render(layout="rowmajor").img, ref)
+            assert renderer.lib().rayna_host_alloc(1 << 60, C.byref(p)) == A.RAYNA_OUT_OF_MEMORY
+            assert np.array_equal(b.render([Request(0, cam, opts)])[0][0], ref)
