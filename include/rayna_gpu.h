@@ -473,8 +473,8 @@ rayna_status rayna_scene_tree(const rayna_scene_desc *scene, int32_t *node_words
 void rayna_destroy(rayna_renderer *r);
 
 /* Pinned host memory for images: rayna_render and rayna_render_batch copy into it directly, several times faster than
- * into ordinary memory.  Valid for every device.  Errors are reported through rayna_last_error(NULL);
- * rayna_host_free(NULL) does nothing. */
+ * into ordinary memory.  Valid for every device.  Any thread may call both at any time: a failure is the status alone
+ * (rayna_last_error(NULL), one text for the whole process, is left as it is).  rayna_host_free(NULL) does nothing. */
 rayna_status rayna_host_alloc(uint64_t bytes, void **out);
 void rayna_host_free(void *p);
 

@@ -1049,17 +1049,14 @@ void rayna_destroy(rayna_renderer *r) {
 }
 
 rayna_status rayna_host_alloc(uint64_t bytes, void **out) {
-    g_create_error.clear();
-    if (!out || bytes == 0) return fail(nullptr, RAYNA_INVALID_ARGUMENT, "null output or no bytes");
+    if (!out || bytes == 0) return RAYNA_INVALID_ARGUMENT;
     *out = nullptr;
     const hipError_t e = hipHostMalloc(out, bytes, hipHostMallocPortable);
-    if (e != hipSuccess) {
-        // taken here: the thread's next launch check would read it as its own (callers go on with ordinary memory)
-        (void)hipGetLastError();
-        *out = nullptr;
-    }
-    HIP_TRY(nullptr, e);
-    return RAYNA_OK;
+    if (e == hipSuccess) return RAYNA_OK;
+    // taken here: the thread's next launch check would read it as its own (callers go on with ordinary memory)
+    (void)hipGetLastError();
+    *out = nullptr;
+    return e == hipErrorOutOfMemory ? RAYNA_OUT_OF_MEMORY : RAYNA_DEVICE_ERROR;
 }
 
 void rayna_host_free(void *p) {

@@ -115,3 +115,19 @@ def test_failed_pinned_allocation_leaves_no_error_behind(gpu):
             assert np.array_equal(r.render(layout="rowmajor").img, ref)
             assert renderer.lib().rayna_host_alloc(1 << 60, C.byref(p)) == A.RAYNA_OUT_OF_MEMORY
             assert np.array_equal(b.render([Request(0, cam, opts)])[0][0], ref)
+
+
+def test_allocations_do_not_touch_the_last_creation_error():
+    """Any thread may allocate (images do, with the GIL released), so the process-wide text that rayna_last_error(NULL)
+    reports for another thread's rayna_create stays as it is, after failures and successes alike."""
+    L = renderer.lib()
+    out = C.c_void_p()
+    assert L.rayna_create(None, None, None, C.byref(out)) == A.RAYNA_INVALID_ARGUMENT
+    text = L.rayna_last_error(None)
+    assert b"null" in text
+    assert L.rayna_host_alloc(0, C.byref(out)) == A.RAYNA_INVALID_ARGUMENT
+    assert L.rayna_host_alloc(64, None) == A.RAYNA_INVALID_ARGUMENT
+    assert L.rayna_last_error(None) == text
+    if L.rayna_host_alloc(4096, C.byref(out)) == A.RAYNA_OK:  # (no device here: refused)
+        L.rayna_host_free(out)
+    assert L.rayna_last_error(None) == text
