@@ -3,14 +3,16 @@
 A copy into ordinary memory goes through the runtime's staging buffer and, for a new array, faults every page in:
 450 us for 1 MB, 4.7 ms for a 1080p image's 25 MB, against 27 and 444 us into pinned memory (copies alone).  The
 memory of an array comes back to a pool when the array and every view of it are gone.  The pool keeps at most
-IDLE_BYTES for reuse and frees the rest; arrays beyond PINNED_BYTES in use, or for which no pinned memory can be had,
-are ordinary ones.  Any thread may ask for arrays and drop them.
+IDLE_BYTES for reuse, the longest unused making room for what comes back.  Arrays larger than that, arrays beyond
+PINNED_BYTES in use and arrays for which no pinned memory can be had are ordinary ones.  Any thread may ask for arrays
+and drop them.
 """
 from __future__ import annotations
 
 import ctypes as C
 import threading
 import weakref
+from collections import OrderedDict, deque
 
 import numpy as np
 
@@ -20,9 +22,13 @@ PINNED_BYTES = 1 << 30
 
 class _Pool:
     def __init__(self):
-        # reentrant: a collection inside a critical section may drop arrays, whose finalizers come back here
+        # reentrant: a collection inside a critical section may drop arrays, whose finalizers come back here; they
+        # leave their buffers in _returned for later (_busy)
         self._lock = threading.RLock()
-        self._idle = {}  # size -> addresses
+        self._busy = False
+        self._returned = deque()  # (address, size) given back and not yet counted
+        self._idle = OrderedDict()  # address -> size, the longest unused first
+        self._by_size = {}  # size -> the idle addresses, likewise
         self.idle_bytes = 0
         self.used_bytes = 0
 
@@ -32,16 +38,53 @@ class _Pool:
         step = max(4096, 1 << max(0, n.bit_length() - 4))
         return -(-n // step) * step
 
+    def _collect(self) -> list:
+        """Makes what was given back idle; the addresses that had to go for it, to be freed."""
+        gone = []
+        while self._returned:
+            address, size = self._returned.popleft()
+            self.used_bytes -= size
+            self.idle_bytes += size
+            self._idle[address] = size
+            self._by_size.setdefault(size, deque()).append(address)
+            while self.idle_bytes > IDLE_BYTES:
+                oldest, oldest_size = self._idle.popitem(last=False)
+                self._by_size[oldest_size].popleft()
+                self.idle_bytes -= oldest_size
+                gone.append(oldest)
+        return gone
+
+    @staticmethod
+    def _free(addresses: list):
+        if addresses:
+            from .renderer import lib
+            for a in addresses:
+                lib().rayna_host_free(a)
+
     def take(self, n: int):
         """(address, size) of a buffer of at least n bytes, or None."""
         size = self._size(n)
+        got = None
         with self._lock:
-            if self.used_bytes + size > PINNED_BYTES:
+            if self._busy or size > IDLE_BYTES:
                 return None
-            self.used_bytes += size
-            if self._idle.get(size):
-                self.idle_bytes -= size
-                return self._idle[size].pop(), size
+            self._busy = True
+            try:
+                gone = self._collect()
+                fits = self.used_bytes + size <= PINNED_BYTES
+                if fits:
+                    self.used_bytes += size
+                    if self._by_size.get(size):
+                        got = self._by_size[size].pop()
+                        del self._idle[got]
+                        self.idle_bytes -= size
+            finally:
+                self._busy = False
+        self._free(gone)
+        if got is not None:
+            return got, size
+        if not fits:
+            return None
         from .renderer import lib
         p = C.c_void_p()
         if lib().rayna_host_alloc(size, C.byref(p)) != 0:
@@ -51,14 +94,16 @@ class _Pool:
         return p.value, size
 
     def give_back(self, address: int, size: int):
+        self._returned.append((address, size))
         with self._lock:
-            self.used_bytes -= size
-            if self.idle_bytes + size <= IDLE_BYTES:
-                self.idle_bytes += size
-                self._idle.setdefault(size, []).append(address)
+            if self._busy:
                 return
-        from .renderer import lib
-        lib().rayna_host_free(address)
+            self._busy = True
+            try:
+                gone = self._collect()
+            finally:
+                self._busy = False
+        self._free(gone)
 
 
 _pool = _Pool()

@@ -131,3 +131,44 @@ def test_allocations_do_not_touch_the_last_creation_error():
     if L.rayna_host_alloc(4096, C.byref(out)) == A.RAYNA_OK:  # (no device here: refused)
         L.rayna_host_free(out)
     assert L.rayna_last_error(None) == text
+
+
+def test_a_new_size_takes_the_place_of_one_no_longer_asked_for(fake, monkeypatch):
+    """A window resized, a server's mixed requests: after a few images of the new size, no allocation and no free."""
+    monkeypatch.setattr(host_buffers, "IDLE_BYTES", 8 * 4096)
+    calls = []
+    for name in ("rayna_host_alloc", "rayna_host_free"):
+        f = getattr(fake, name)
+        monkeypatch.setattr(fake, name, lambda *a, f=f, name=name: (calls.append(name), f(*a))[1])
+    old = [host_buffers.empty(3 * 4096, np.uint8) for _ in range(2)] + [host_buffers.empty(4096, np.uint8)]
+    del old
+    gc.collect()
+    for n in (2 * 4096, 5 * 4096):
+        for k in range(50):
+            host_buffers.empty(n, np.uint8)
+            gc.collect()
+            if k == 2:
+                del calls[:]
+        assert not calls
+    assert host_buffers._pool.idle_bytes <= 8 * 4096
+    assert sum(a.size for a in fake.held.values()) == host_buffers._pool.idle_bytes
+
+
+def test_the_longest_unused_buffer_goes_first(fake, monkeypatch):
+    monkeypatch.setattr(host_buffers, "IDLE_BYTES", 3 * 4096)
+    a, b, c = (host_buffers.empty(4096, np.uint8) for _ in range(3))
+    at = {k: v.ctypes.data for k, v in (("a", a), ("b", b), ("c", c))}
+    del b  # each given back here
+    del c
+    del a
+    two = host_buffers.empty(2 * 4096, np.uint8)
+    del two
+    gc.collect()
+    assert at["b"] not in fake.held and at["c"] not in fake.held and at["a"] in fake.held
+    assert host_buffers.empty(4096, np.uint8).ctypes.data == at["a"]
+
+
+def test_images_larger_than_the_pool_keeps_are_ordinary(fake, monkeypatch):
+    monkeypatch.setattr(host_buffers, "IDLE_BYTES", 3 * 4096)
+    a = host_buffers.empty(4 * 4096, np.uint8)
+    assert not fake.held and a.shape == (4 * 4096,) and host_buffers._pool.used_bytes == 0
