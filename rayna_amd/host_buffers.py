@@ -6,10 +6,15 @@ memory of an array comes back to a pool when the array and every view of it are 
 IDLE_BYTES for reuse, the longest unused making room for what comes back.  Arrays larger than that, arrays beyond
 PINNED_BYTES in use and arrays for which no pinned memory can be had are ordinary ones.  Any thread may ask for arrays
 and drop them.
+
+A forked child does not have the parent's pinned memory (the driver keeps it out of forks), so the images alive at a
+fork are copied before it, and the child gets the copies as ordinary memory at the same addresses.
 """
 from __future__ import annotations
 
 import ctypes as C
+import mmap
+import os
 import threading
 import weakref
 from collections import OrderedDict, deque
@@ -29,6 +34,9 @@ class _Pool:
         self._returned = deque()  # (address, size) given back and not yet counted
         self._idle = OrderedDict()  # address -> size, the longest unused first
         self._by_size = {}  # size -> the idle addresses, likewise
+        self._live = {}  # address -> (bytes asked for, size)
+        self._inherited = set()  # in a forked child: the addresses of the parent's arrays
+        self._copies = []
         self.idle_bytes = 0
         self.used_bytes = 0
 
@@ -43,6 +51,9 @@ class _Pool:
         gone = []
         while self._returned:
             address, size = self._returned.popleft()
+            if address in self._inherited:  # ordinary memory here, which stays in place
+                continue
+            del self._live[address]
             self.used_bytes -= size
             self.idle_bytes += size
             self._idle[address] = size
@@ -78,6 +89,7 @@ class _Pool:
                         got = self._by_size[size].pop()
                         del self._idle[got]
                         self.idle_bytes -= size
+                        self._live[got] = n, size
             finally:
                 self._busy = False
         self._free(gone)
@@ -91,6 +103,8 @@ class _Pool:
             with self._lock:
                 self.used_bytes -= size
             return None
+        with self._lock:
+            self._live[p.value] = n, size
         return p.value, size
 
     def give_back(self, address: int, size: int):
@@ -105,8 +119,34 @@ class _Pool:
                 self._busy = False
         self._free(gone)
 
+    def before_fork(self):
+        self._lock.acquire()
+        self._copies = []
+        self._copies = [(a, size, C.string_at(a, n)) for a, (n, size) in self._live.items()]
+
+    def after_fork_in_parent(self):
+        self._copies = []
+        self._lock.release()
+
+    def after_fork_in_child(self):
+        copies, inherited = self._copies, self._inherited
+        self.__init__()
+        self._inherited = inherited
+        libc = C.CDLL(None)
+        libc.mmap.restype = C.c_void_p
+        libc.mmap.argtypes = [C.c_void_p, C.c_size_t, C.c_int, C.c_int, C.c_int, C.c_long]
+        fixed = 0x10  # MAP_FIXED
+        for address, size, data in copies:
+            at = libc.mmap(address, size, mmap.PROT_READ | mmap.PROT_WRITE,
+                           mmap.MAP_PRIVATE | mmap.MAP_ANONYMOUS | fixed, -1, 0)
+            if at == address:
+                C.memmove(address, data, len(data))
+            inherited.add(address)
+
 
 _pool = _Pool()
+os.register_at_fork(before=lambda: _pool.before_fork(), after_in_parent=lambda: _pool.after_fork_in_parent(),
+                    after_in_child=lambda: _pool.after_fork_in_child())
 
 
 def empty(count: int, dtype) -> np.ndarray:

@@ -2,6 +2,8 @@
 image is never overwritten while it or a view of it is held."""
 import ctypes as C
 import gc
+import mmap
+import os
 import threading
 
 import numpy as np
@@ -172,3 +174,73 @@ def test_images_larger_than_the_pool_keeps_are_ordinary(fake, monkeypatch):
     monkeypatch.setattr(host_buffers, "IDLE_BYTES", 3 * 4096)
     a = host_buffers.empty(4 * 4096, np.uint8)
     assert not fake.held and a.shape == (4 * 4096,) and host_buffers._pool.used_bytes == 0
+
+
+def _exit_of_forked_child(work):
+    """The exit code of a forked child that runs work(), or minus the signal that ended it."""
+    pid = os.fork()
+    if pid == 0:
+        code = 1
+        try:
+            code = 0 if work() else 2
+        finally:
+            os._exit(code)
+    return os.waitstatus_to_exitcode(os.waitpid(pid, 0)[1])
+
+
+class ForkLib:
+    """rayna_host_alloc / rayna_host_free over memory that a forked child does not have, as pinned memory."""
+
+    def __init__(self):
+        self.maps, self.freed = {}, []
+
+    def rayna_host_alloc(self, size, out):
+        m = mmap.mmap(-1, size)
+        m.madvise(mmap.MADV_DONTFORK)
+        out._obj.value = C.addressof(C.c_char.from_buffer(m))
+        self.maps[out._obj.value] = m
+        return 0
+
+    def rayna_host_free(self, address):
+        self.freed.append(address)
+
+
+def test_forked_children_have_the_images(monkeypatch):
+    """A child forked with an image in hand (a worker process that saves it) reads the image's values, in its own
+    memory; what the parent does with the buffer later is not seen, and the child gives nothing back."""
+    lib = ForkLib()
+    monkeypatch.setattr(renderer, "lib", lambda: lib)
+    monkeypatch.setattr(host_buffers, "_pool", host_buffers._Pool())
+    idle = host_buffers.empty(3000, np.uint8)
+    del idle
+    gc.collect()
+    images = [host_buffers.empty(n, np.float32) for n in (5, 1024, 70001)]
+    for k, a in enumerate(images):
+        a[:] = np.arange(a.size) + k
+    views = [a[1:] for a in images]
+
+    def child():
+        ok = all(np.array_equal(views[k], np.arange(1, images[k].size) + k) for k in range(3))
+        views[1][3] = 77.0  # writable, and its own
+        ok = ok and images[1][4] == 77.0
+        new = host_buffers.empty(3000, np.uint8)  # not the idle buffer, which the child does not have
+        new[:] = 9
+        del images[:], views[:]
+        gc.collect()
+        return ok and not lib.freed and (new == 9).all()
+
+    del a
+    assert _exit_of_forked_child(child) == 0
+    assert images[1][4] == 5.0 and host_buffers._pool.used_bytes > 0
+    assert host_buffers.empty(3000, np.uint8).size == 3000  # the pool goes on
+
+
+@pytest.mark.gpu
+def test_forked_children_have_rendered_images(gpu):
+    sc, cam, opts = presets.cornell(width=65, height=43, samples=2)
+    with Renderer(sc, cam, opts) as r:
+        img = r.render().img
+        copy = img.copy()
+        assert _exit_of_forked_child(lambda: np.array_equal(img, copy)) == 0
+        r.clear_accumulation()
+        assert np.array_equal(r.render().img, copy) and np.array_equal(img, copy)
