@@ -26,6 +26,14 @@ std::string g_create_error;
 // rayna_debug_fail_launches: < 0 off, else the number of launch checks still to pass before one fails
 std::atomic<int32_t> g_fail_launches{-1};
 
+// Lets this thread allocate and free while some stream is being captured: by default such a call is refused and
+// invalidates the capture, whichever thread makes either.
+struct RelaxedCapture {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+    ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
 // Words of pinned host memory that kernels write to, one per renderer.  They come in pages of 512 and are handed out
 // again when their renderer is destroyed (pinning memory for each renderer cost its creation 0.1-0.2 ms).
 std::mutex g_host_words_lock;
@@ -1051,6 +1059,7 @@ void rayna_destroy(rayna_renderer *r) {
 rayna_status rayna_host_alloc(uint64_t bytes, void **out) {
     if (!out || bytes == 0) return RAYNA_INVALID_ARGUMENT;
     *out = nullptr;
+    const RelaxedCapture relaxed;
     const hipError_t e = hipHostMalloc(out, bytes, hipHostMallocPortable);
     if (e == hipSuccess) return RAYNA_OK;
     // taken here: the thread's next launch check would read it as its own (callers go on with ordinary memory)
@@ -1060,7 +1069,9 @@ rayna_status rayna_host_alloc(uint64_t bytes, void **out) {
 }
 
 void rayna_host_free(void *p) {
-    if (p) (void)hipHostFree(p);
+    if (!p) return;
+    const RelaxedCapture relaxed;
+    (void)hipHostFree(p);
 }
 
 rayna_status rayna_debug_sqrt_mismatches(uint32_t first, uint64_t count, uint64_t *mismatches) {

@@ -244,3 +244,34 @@ def test_forked_children_have_rendered_images(gpu):
         assert _exit_of_forked_child(lambda: np.array_equal(img, copy)) == 0
         r.clear_accumulation()
         assert np.array_equal(r.render().img, copy) and np.array_equal(img, copy)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mode", ["global", "thread_local", "relaxed"])
+@pytest.mark.parametrize("thread", [False, True])
+def test_images_may_be_dropped_while_a_graph_is_captured(gpu, monkeypatch, mode, thread):
+    """A collection may come at any time, also between the launches of a capture, on its thread or another: the memory
+    that the pool then frees does not break the capture."""
+    import torch
+    monkeypatch.setattr(host_buffers, "_pool", host_buffers._Pool())
+    monkeypatch.setattr(host_buffers, "IDLE_BYTES", 5 << 20)
+    images = [host_buffers.empty(4 << 20, np.uint8) for _ in range(3)]
+    x = torch.zeros(64, device="cuda")
+    y = torch.zeros(64, device="cuda")
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, capture_error_mode=mode):
+        x.add_(1)
+        drop = threading.Thread(target=images.clear) if thread else None
+        if thread:
+            drop.start()
+            drop.join()
+        else:
+            images.clear()
+        y.copy_(x)
+    assert host_buffers._pool.used_bytes == 0 and host_buffers._pool.idle_bytes == 4 << 20
+    for k in range(4):
+        g.replay()
+        torch.cuda.synchronize()
+        assert (y == k + 1).all()
+        (x * 2).sum().item()  # the program's own work between replays
