@@ -477,6 +477,9 @@ void rayna_destroy(rayna_renderer *r);
  * (rayna_last_error(NULL), one text for the whole process, is left as it is).  rayna_host_free(NULL) does nothing. */
 rayna_status rayna_host_alloc(uint64_t bytes, void **out);
 void rayna_host_free(void *p);
+/* Waits for everything that the process has submitted to `device`, on any stream, before memory that copies may still
+ * read or write is used again.  Allowed while a stream is being captured (hipDeviceSynchronize is not). */
+rayna_status rayna_host_settle(int32_t device);
 
 /* Measurement hook (no engine counterpart): the fp32 VALU issue rate the current GPU sustains, the peak the
  * traversal kernels' VALU roofline is taken against.  A calibration kernel runs eight independent multiply-add

@@ -5,7 +5,8 @@ A copy into ordinary memory goes through the runtime's staging buffer and, for a
 memory of an array comes back to a pool when the array and every view of it are gone.  The pool keeps at most
 IDLE_BYTES for reuse, the longest unused making room for what comes back.  Arrays larger than that, arrays beyond
 PINNED_BYTES in use and arrays for which no pinned memory can be had are ordinary ones.  Any thread may ask for arrays
-and drop them.
+and drop them.  torch's non-blocking copies of such an array run on after the call: the array may be dropped at once,
+but not written to before they end, as with any pinned tensor.
 
 A forked child does not have the parent's pinned memory (the driver keeps it out of forks), so the images alive at a
 fork are copied before it, and the child gets the copies as ordinary memory at the same addresses.
@@ -15,6 +16,7 @@ from __future__ import annotations
 import ctypes as C
 import mmap
 import os
+import sys
 import threading
 import weakref
 from collections import OrderedDict, deque
@@ -23,6 +25,17 @@ import numpy as np
 
 IDLE_BYTES = 256 << 20
 PINNED_BYTES = 1 << 30
+
+
+def _settled() -> bool:
+    """Waits for the copies that the program may have had torch make from or to dropped arrays: from and to pinned
+    memory they run on when asked not to block, so a buffer is in use until they end.  False if that is not known."""
+    torch = sys.modules.get("torch")
+    if torch is None or not hasattr(torch, "cuda") or not torch.cuda.is_initialized():
+        return True
+    from .renderer import lib
+    devices = [d for d in range(torch.cuda.device_count()) if torch._C._cuda_hasPrimaryContext(d)]
+    return all(lib().rayna_host_settle(d) == 0 for d in devices)
 
 
 class _Pool:
@@ -94,7 +107,10 @@ class _Pool:
                 self._busy = False
         self._free(gone)
         if got is not None:
-            return got, size
+            if _settled():
+                return got, size
+            self.give_back(got, size)
+            return None
         if not fits:
             return None
         from .renderer import lib

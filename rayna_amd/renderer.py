@@ -32,7 +32,7 @@ EXPORTS = ("rayna_create", "rayna_set_scene", "rayna_set_camera", "rayna_set_opt
            "rayna_set_validate", "rayna_validate_counts", "rayna_adjoint_static", "rayna_batch_create",
            "rayna_batch_set_tuning", "rayna_render_batch", "rayna_batch_destroy", "rayna_batch_last_error",
            "rayna_primary_hits", "rayna_dfs_order", "rayna_tree_hash", "rayna_scene_prepare", "rayna_scene_tree", "rayna_destroy",
-           "rayna_host_alloc", "rayna_host_free", "rayna_measure_valu_peak", "rayna_debug_sqrt_mismatches",
+           "rayna_host_alloc", "rayna_host_free", "rayna_host_settle", "rayna_measure_valu_peak", "rayna_debug_sqrt_mismatches",
            "rayna_debug_fail_launches", "rayna_last_error")
 
 
@@ -115,6 +115,8 @@ def lib() -> C.CDLL:
         L.rayna_host_alloc.argtypes = [C.c_uint64, C.POINTER(vp)]
         L.rayna_host_free.restype = None
         L.rayna_host_free.argtypes = [vp]
+        L.rayna_host_settle.restype = C.c_int
+        L.rayna_host_settle.argtypes = [C.c_int32]
         L.rayna_measure_valu_peak.restype = C.c_int
         L.rayna_measure_valu_peak.argtypes = [C.c_uint32, C.POINTER(C.c_double), C.POINTER(C.c_double)]
         L.rayna_debug_sqrt_mismatches.restype = C.c_int

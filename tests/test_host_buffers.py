@@ -251,7 +251,7 @@ def test_forked_children_have_rendered_images(gpu):
 @pytest.mark.parametrize("thread", [False, True])
 def test_images_may_be_dropped_while_a_graph_is_captured(gpu, monkeypatch, mode, thread):
     """A collection may come at any time, also between the launches of a capture, on its thread or another: the memory
-    that the pool then frees does not break the capture."""
+    that the pool then frees, or hands out again, does not break the capture."""
     import torch
     monkeypatch.setattr(host_buffers, "_pool", host_buffers._Pool())
     monkeypatch.setattr(host_buffers, "IDLE_BYTES", 5 << 20)
@@ -259,19 +259,70 @@ def test_images_may_be_dropped_while_a_graph_is_captured(gpu, monkeypatch, mode,
     x = torch.zeros(64, device="cuda")
     y = torch.zeros(64, device="cuda")
     torch.cuda.synchronize()
+
+    def drop_and_take():
+        images.clear()
+        images.append(host_buffers.empty(4 << 20, np.uint8))  # one that was kept, once its copies have ended
+
     g = torch.cuda.CUDAGraph()
     with torch.cuda.graph(g, capture_error_mode=mode):
         x.add_(1)
-        drop = threading.Thread(target=images.clear) if thread else None
         if thread:
-            drop.start()
-            drop.join()
+            t = threading.Thread(target=drop_and_take)
+            t.start()
+            t.join()
         else:
-            images.clear()
+            drop_and_take()
         y.copy_(x)
-    assert host_buffers._pool.used_bytes == 0 and host_buffers._pool.idle_bytes == 4 << 20
+    assert host_buffers._pool.used_bytes == 4 << 20 and host_buffers._pool.idle_bytes == 0
     for k in range(4):
         g.replay()
         torch.cuda.synchronize()
         assert (y == k + 1).all()
         (x * 2).sum().item()  # the program's own work between replays
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("to_device", [True, False])
+@pytest.mark.parametrize("side", [False, True])
+def test_copies_in_flight_have_ended_before_a_buffer_is_used_again(gpu, monkeypatch, to_device, side):
+    """torch copies from and to pinned memory without waiting when asked not to block (with ordinary memory it waits):
+    a program that drops a frame after such a copy, while the device is busy, has that frame on the device, and the
+    next image keeps what is written to it."""
+    import torch
+    monkeypatch.setattr(host_buffers, "_pool", host_buffers._Pool())
+    a = torch.randn(8192, 8192, device="cuda", dtype=torch.bfloat16)
+    dev = torch.full((1 << 18,), 3.0, device="cuda")
+    stream = torch.cuda.Stream() if side else torch.cuda.current_stream()
+    torch.cuda.synchronize()
+    img = host_buffers.empty(1 << 18, np.float32)
+    img[:] = 7.0
+    at = img.ctypes.data
+    with torch.cuda.stream(stream):
+        for _ in range(60):  # tens of milliseconds of work before the copy
+            b = a @ a
+        if to_device:
+            dev.copy_(torch.from_numpy(img), non_blocking=True)
+        else:
+            torch.from_numpy(img).copy_(dev, non_blocking=True)
+    del img
+    gc.collect()
+    new = host_buffers.empty(1 << 18, np.float32)
+    assert new.ctypes.data == at
+    new[:] = -1.0
+    torch.cuda.synchronize()
+    assert (dev == (7.0 if to_device else 3.0)).all() and (new == -1.0).all()
+    del b
+
+
+def test_a_buffer_that_may_be_in_use_is_not_handed_out(fake, monkeypatch):
+    """Where it cannot be known that the copies have ended, the array is an ordinary one."""
+    a = host_buffers.empty(1000, np.uint8)
+    at = a.ctypes.data
+    del a
+    gc.collect()
+    with monkeypatch.context() as m:
+        m.setattr(host_buffers, "_settled", lambda: False)
+        b = host_buffers.empty(1000, np.uint8)
+        assert b.ctypes.data != at and host_buffers._pool.used_bytes == 0 and len(fake.held) == 1
+    assert host_buffers.empty(1000, np.uint8).ctypes.data == at
