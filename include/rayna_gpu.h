@@ -414,7 +414,8 @@ typedef struct rayna_request {
     rayna_camera camera;
     rayna_render_opts opts;   /* mode RAYNA_MODE_PBR, ray_branching 1 */
     float *out_rgb;           /* host buffer of width*height*3 floats, or NULL to leave the image on the device
-                               * (an invalid camera gives the engine's checkerboard, as rayna_render) */
+                               * (an invalid camera gives the engine's checkerboard, as rayna_render, at its
+                               * start and zeros behind it) */
 } rayna_request;
 
 typedef struct rayna_batch_stats {

@@ -42,16 +42,6 @@ class BatchStats:
     request_ms: np.ndarray  # per request: device time from the batch start until its image was final (eager)
 
 
-def _image(q: Request) -> np.ndarray:
-    """The array of a request's image.  A camera without a viewport (Camera::calculate_viewport failing) gets the
-    checkerboard, which covers only its first values: any camera that might be one gets zeros."""
-    n = q.opts.width * q.opts.height * 3
-    f = np.asarray(q.camera.fwd, np.float64)
-    sideways = f[0] * f[0] + f[2] * f[2]
-    usual = q.camera.v_fov != 0.0 and q.camera.focus_dist != 0.0 and sideways > 1e-9 * f[1] * f[1] + 1e-30
-    return host_buffers.empty(n, np.float32) if usual and np.isfinite(f).all() else np.zeros(n, np.float32)
-
-
 class BatchRenderer:
     def __init__(self, scenes: Sequence):
         self.scenes = list(scenes)
@@ -86,7 +76,7 @@ class BatchRenderer:
         for i, q in enumerate(requests):
             o = q.opts
             lay = A.LAYOUT_XMAJOR if q.layout == "xmajor" else A.LAYOUT_ROWMAJOR
-            img = _image(q) if to_host else None
+            img = host_buffers.empty(o.width * o.height * 3, np.float32) if to_host else None
             imgs.append(img)
             reqs[i] = A.Request(q.scene, lay, q.camera.desc(), o.desc(),
                                 img.ctypes.data_as(C.POINTER(C.c_float)) if to_host else None)

@@ -747,6 +747,7 @@ rayna_status rayna_render_batch(rayna_batch *b, const rayna_request *reqs, int32
     for (int p = 0; p < used; ++p) segs += seg[p];
     for (int i = 0; i < n; ++i) {
         if (valid[i] || !reqs[i].out_rgb) continue;
+        std::fill_n(reqs[i].out_rgb, 3 * (size_t)reqs[i].opts.width * reqs[i].opts.height, 0.0f);
         write_checkerboard(ilog2(reqs[i].opts.width), ilog2(reqs[i].opts.height), reqs[i].out_rgb, reqs[i].layout);
     }
     if (stats) {

@@ -8,7 +8,7 @@ import numpy as np
 import pytest
 
 import oracle
-from rayna_amd import Renderer, presets
+from rayna_amd import Renderer, host_buffers, presets
 from rayna_amd.batch import BatchRenderer, Request
 from rayna_amd.scene import Camera
 
@@ -97,3 +97,21 @@ def test_batch_latency_order(gpu):
     work = np.array([q.opts.width * q.opts.height * q.opts.samples for q in reqs])
     assert st.request_ms[np.argmin(work)] <= st.request_ms.min() + 1e-9
     assert (st.request_ms > 0).all() and st.request_ms.max() <= st.kernel_ms + 1e-6
+
+
+@pytest.mark.parametrize("fwd,fov,focus", [((1e200, 0, 0), 40.0, 1.0), ((0, 0, 0), 40.0, 1.0), ((0, 1, 0), 40.0, 1.0),
+                                           ((1e-200, 0, 0), 40.0, 1.0), ((float("nan"), 0, 1), 40.0, 1.0),
+                                           ((0, 0, 1), 0.0, 1.0), ((0, 0, 1), 40.0, 0.0)])
+def test_no_viewport_leaves_nothing_of_earlier_images(gpu, monkeypatch, fwd, fov, focus):
+    """Cameras for which calculate_viewport fails, whatever the reason: the checkerboard, then zeros, also where the
+    image's memory held another image before."""
+    scenes, reqs = _requests(n=2)
+    q = reqs[0]
+    monkeypatch.setattr(host_buffers, "empty", lambda n, dtype: np.full(n, 15.0, dtype))
+    with BatchRenderer(scenes) as b:
+        imgs, _ = b.render([q, Request(q.scene, Camera(pos=(0, 0, 0), fwd=fwd, v_fov=fov, focus_dist=focus), q.opts)])
+    monkeypatch.undo()
+    n = 3 * int(np.log2(q.opts.width)) * int(np.log2(q.opts.height))
+    flat = imgs[1].reshape(-1)
+    assert np.isin(flat[:n], (0.0, 1.0)).all() and flat[:n].any() and not flat[n:].any()
+    assert np.array_equal(imgs[0], _single(scenes, q)[0])
