@@ -121,10 +121,8 @@ struct rayna_renderer {
     uint64_t chunk_target = TARGET_SLOTS;
     ExtendTuning tune;
     std::vector<hipEvent_t> events;
-    // the last pass over a chunk: the event triples it recorded, and whether the first was of the camera rays alone
-    size_t pass_marks = 1;
-    std::vector<size_t> marks;  // of the call so far: the event each mark stands for
-    bool camera_apart = true;
+    std::vector<size_t> marks;   // of the call so far: the event each mark stands for, in triples (event_times)
+    std::vector<char> camera_at;  // per triple: whether it is the launch for a chunk's camera rays alone
     // debug validation (shared/validate.rs): RAYNA_CHECKS counters, counted in PBR frames while `validate`
     uint32_t *checks = nullptr;
     // non-empty once a launch on this renderer failed (the failure's text): every later call is refused
@@ -430,8 +428,6 @@ SegmentCount trace_chunk(rayna_renderer *r, FrameParams &fp, uint32_t s0, uint32
     fp.rays_stored = apart > 0 && (fp.mode != RAYNA_MODE_PBR || r->dev.view.n_sdfs > 0 ||
                                    !extend_packets(r->dev.view, fp, r->tune, BatchView{}, 0));
     if (fp.rays_stored) launch_generate(fp, r->pb, BatchView{}, r->stream);
-    r->camera_apart = apart > 0;
-    r->pass_marks = 0;
     for (uint32_t depth = 0; depth < depths; ++depth) {
         const int32_t *qin = depth == 0 ? nullptr : r->queue[depth & 1];
         const uint32_t *cin = depth == 0 ? nullptr : r->queue_count + depth;
@@ -440,7 +436,7 @@ SegmentCount trace_chunk(rayna_renderer *r, FrameParams &fp, uint32_t s0, uint32
         uint32_t *work = claims + (size_t)depth * 2 * CLAIM_WORDS;
         const bool rest = depth >= apart;  // this launch takes every path to its end
         mark();
-        ++r->pass_marks;
+        if (ev) r->camera_at.push_back(depth == 0 && !rest);
         launched = true;
         if (rest) {
             launch_trace(r->dev.view, fp, r->pb, qin, cin, depth, r->grid_extend, r->dev.overflow, work, r->claims,
@@ -475,7 +471,8 @@ rayna_status ensure_events(rayna_renderer *r, size_t n) {
 }
 
 // Device times from the events of one call: events[0] before the first kernel, events[evi - 1] after the last, and in
-// marks the events of the triples [before extend, after extend, after shade], pass_marks per pass over a chunk.
+// marks the events of the triples [before extend, after extend, after shade], as many per pass over a chunk as
+// launched_depths made of it (the last chunk of a frame is often smaller and has fewer).
 rayna_status event_times(rayna_renderer *r, size_t evi, rayna_render_stats *st) {
     float ms = 0;
     HIP_TRY(r, hipEventElapsedTime(&ms, r->events[0], r->events[evi - 1]));
@@ -488,7 +485,7 @@ rayna_status event_times(rayna_renderer *r, size_t evi, rayna_render_stats *st) 
         if (m[2] != m[1]) HIP_TRY(r, hipEventElapsedTime(&b, r->events[m[1]], r->events[m[2]]));
         ext += a;
         sh += b;
-        if (r->camera_apart && k % r->pass_marks == 0) ext0 += a;
+        if (r->camera_at[k]) ext0 += a;
     }
     st->extend_ms = ext;
     st->shade_ms = sh;
@@ -574,6 +571,7 @@ rayna_status render_frame(rayna_renderer *r, float *out_rgb, uint8_t *out_rgba, 
         const FrameOutput out{r->acc, r->out_dev, (double)r->frames, layout, r->acc_dirty ? 1u : 0u};
         r->acc_dirty = false;
         r->marks.clear();
+        r->camera_at.clear();
         size_t evi = 0;
         if (ev) HIP_TRY(r, hipEventRecord((*ev)[evi++], r->stream));
         uint64_t launches = 0;
@@ -839,6 +837,7 @@ rayna_status rayna_adjoint(rayna_renderer *r, uint32_t frame, const float *d_ima
     std::vector<hipEvent_t> *ev = stats ? &r->events : nullptr;
     size_t evi = 0;
     r->marks.clear();
+    r->camera_at.clear();
     if (ev) HIP_TRY(r, hipEventRecord((*ev)[evi++], r->stream));
     uint64_t launches = 0;
     for (uint32_t c = 0; c < n_chunks; ++c) {

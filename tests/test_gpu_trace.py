@@ -51,3 +51,19 @@ def test_adjoint_equals_the_oracle(gpu, scene, samples):
         g, _ = r.adjoint(d, layout="rowmajor")
     ref, _, _ = oracle.TwinScene(sc).adjoint(cam, opts, d, precision=32)
     assert np.linalg.norm(g - ref) <= 1e-9 * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("first,last", [(64, 1), (40, 25), (64, 17)])
+def test_camera_ray_time_of_unequal_chunks(gpu, first, last):
+    """A frame's chunks may differ in the depths that get launches of their own (here 2 and 0, 2 and 1, 2 and 1): the
+    time of the camera rays is the sum of their own launches.  They are about a sixth of the time here, alone as in chunks
+    (0 and two thirds were reported)."""
+    sc, cam, opts = presets.triangle_mesh(subdiv=5, width=960, height=540, samples=first + last)
+    with Renderer(sc, cam, opts) as r:
+        r.set_tuning(chunk_slots=960 * 540 * first)
+        shares = []
+        for _ in range(3):
+            s = r.render(to_host=False).stats
+            shares.append(s.extend_camera_ms / s.extend_ms)
+        assert s.extend_launches == 2 * (opts.ray_depth + 1)
+    assert 0.02 < np.median(shares) < 0.4
