@@ -55,6 +55,7 @@ struct Plan {
     std::vector<uint32_t> depth;               // per chunk: deepest ray_depth of its requests
     std::vector<uint32_t> n_sdf;               // per chunk: most unbounded objects of its requests' scenes
     std::vector<uint32_t> features;            // per chunk: SCENE_* bits of any of its requests' scenes
+    std::vector<int32_t> n_nodes;              // per chunk: the largest tree of its requests' scenes
     std::vector<uint32_t> slots;               // per chunk
     std::vector<int32_t> dep;                  // per chunk: the last earlier chunk holding a piece of one of its
                                                // requests (its resolve must come first), or -1
@@ -95,6 +96,7 @@ struct rayna_batch {
     SceneView view{};
     std::vector<SceneSlot> slots;
     std::vector<uint32_t> scene_features;  // per scene: SCENE_* bits
+    std::vector<int32_t> scene_nodes;      // per scene: the nodes of its tree
     size_t overflow_entries = 0;  // per pipeline: extend grid * block * stack entries beyond the LDS part
     int cus = 1, grid_extend = 1024, grid_shade = 1024, grid_march = 1024;
     uint32_t n_sdf_max = 0;  // most unbounded objects of one scene
@@ -363,6 +365,7 @@ void make_plan(rayna_batch *b, const rayna_request *reqs, int n, const std::vect
         pl.first_entry.push_back((uint32_t)pl.table.size());
         pl.first_final.push_back((uint32_t)pl.finals.size());
         uint32_t slot = 0, maxp = 0, depth = 0, nsdf = 0, rblocks = 1, feat = 0;
+        int32_t nodes = 0;
         for (size_t e = 0; e < pl.chunks[c].size(); ++e) {
             const Piece &pc = pl.chunks[c][e];
             const rayna_request &q = reqs[pc.req];
@@ -399,12 +402,14 @@ void make_plan(rayna_batch *b, const rayna_request *reqs, int n, const std::vect
             depth = std::max(depth, q.opts.ray_depth);
             nsdf = std::max(nsdf, (uint32_t)sc.n_sdfs);
             feat |= b->scene_features[q.scene];
+            nodes = std::max(nodes, b->scene_nodes[q.scene]);
         }
         pl.max_pixels.push_back(maxp);
         pl.resolve_blocks.push_back(rblocks);
         pl.depth.push_back(depth);
         pl.n_sdf.push_back(nsdf);
         pl.features.push_back(feat);
+        pl.n_nodes.push_back(nodes);
         pl.slots.push_back(slot);
         pl.max_depth = std::max(pl.max_depth, depth);
     }
@@ -414,9 +419,11 @@ void make_plan(rayna_batch *b, const rayna_request *reqs, int n, const std::vect
 // The merged scene set's view as one chunk sees it: the kernels compile out the sphere test, media, instance
 // and texture code and, without SDFs, the SDF normal code (k_shade's eight-wave form), so a chunk whose requests'
 // scenes hold none of these runs the forms a single render of those scenes would.  A request's rays only reach
-// its own scene's tree, so the other scenes' items never meet the compiled-out code.
-SceneView chunk_view(const SceneView &merged, uint32_t features) {
+// its own scene's tree, so the other scenes' items never meet the compiled-out code.  n_nodes: the rules on the size of
+// a tree (launched_depths, launch_trace) go by the largest that rays of the chunk enter.
+SceneView chunk_view(const SceneView &merged, uint32_t features, int32_t n_nodes) {
     SceneView v = merged;
+    v.n_nodes = n_nodes;
     v.instances = (features & SCENE_INSTANCES) ? merged.instances : 0;
     v.sphere_tests = (features & SCENE_SPHERES) ? merged.sphere_tests : 0;
     v.media = (features & SCENE_MEDIA) ? merged.media : 0;
@@ -430,7 +437,7 @@ SceneView chunk_view(const SceneView &merged, uint32_t features) {
 uint32_t plan_launches(const rayna_batch *b, const Plan &pl, int used) {
     uint32_t n = (uint32_t)used;  // segment counters
     for (size_t c = 0; c < pl.chunks.size(); ++c) {
-        const SceneView cv = chunk_view(b->view, pl.features[c]);
+        const SceneView cv = chunk_view(b->view, pl.features[c], pl.n_nodes[c]);
         const BatchView bv{b->table, (uint32_t)pl.chunks[c].size(), nullptr};
         FrameParams fp{};
         fp.n_slots = pl.slots[c];
@@ -468,7 +475,7 @@ hipError_t enqueue(rayna_batch *b, const Plan &pl, int used, bool timing) {
         fp.n_slots = pl.slots[c];
         fp.ray_depth = pl.depth[c];
         const uint32_t D = pl.depth[c];
-        const SceneView cv = chunk_view(b->view, pl.features[c]);
+        const SceneView cv = chunk_view(b->view, pl.features[c], pl.n_nodes[c]);
         launch_fill_u32(P.queue_count, 0u, 3 * (D + 2), s);
         launch_fill_u32(P.claims, 0u, SEGMENT_WORDS + (D + 1) * 2 * CLAIM_WORDS, s);
         uint32_t *claims = P.claims + SEGMENT_WORDS;
@@ -561,6 +568,7 @@ rayna_status rayna_batch_create(const rayna_scene_desc *scenes, int32_t n_scenes
     b->grid_shade = b->cus * SHADE_BLOCKS_PER_CU;
     std::vector<PackedScene> packed(n_scenes);
     b->scene_features.assign(n_scenes, 0u);
+    b->scene_nodes.assign(n_scenes, 0);
     for (int i = 0; i < n_scenes; ++i) {
         std::string err;
         const rayna_status st = pack_scene(scenes[i], packed[i], err);
@@ -579,6 +587,7 @@ rayna_status rayna_batch_create(const rayna_scene_desc *scenes, int32_t n_scenes
         if (has_mandelbulbs(p)) f |= SCENE_MANDELBULBS;
         if (has_textures(p) || p.skybox == RAYNA_SKY_HDRI) f |= SCENE_TEXTURED;
         b->scene_features[i] = f;
+        b->scene_nodes[i] = (int32_t)p.nodes.size();
     }
     PackedScene merged;
     if (!merge_scenes(packed, merged, b->slots)) {

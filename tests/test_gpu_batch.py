@@ -115,3 +115,16 @@ def test_no_viewport_leaves_nothing_of_earlier_images(gpu, monkeypatch, fwd, fov
     flat = imgs[1].reshape(-1)
     assert np.isin(flat[:n], (0.0, 1.0)).all() and flat[:n].any() and not flat[n:].any()
     assert np.array_equal(imgs[0], _single(scenes, q)[0])
+
+
+def test_a_chunk_is_launched_as_its_own_scenes_ask(gpu):
+    """The size of a tree decides how many depths get launches of their own: a batch's other scenes do not count."""
+    _, cam, opts = presets.cornell(width=1024, height=1024, samples=16, ray_depth=2)
+    launches, images = [], []
+    for others in ([], [presets.triangle_mesh(subdiv=4)[0]]):
+        with BatchRenderer([presets.cornell()[0]] + others) as b:
+            imgs, st = b.render([Request(0, cam, opts)])
+            launches.append(st.launches)
+            images.append(imgs[0])
+    assert launches[0] == launches[1]
+    assert np.array_equal(*images)
