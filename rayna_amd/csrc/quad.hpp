@@ -33,6 +33,15 @@ __device__ __forceinline__ uint32_t quad_bits(unsigned long long mask) {
     return (uint32_t)(mask >> (__lane_id() & 60u)) & 15u;
 }
 
+// Between one lane's store of a stack entry and another lane's load of it, and between loads and a store that takes
+// their place: keeps the compiler from moving either across (the wave's own accesses to LDS and memory stay in order,
+// so this costs no instruction).
+__device__ __forceinline__ void quad_stack_order() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // A quad's traversal: the entry it holds (code, entry distance) and the stack below it.
 struct QuadStack {
     lds_u64 *s_entry;
@@ -84,7 +93,9 @@ __device__ __forceinline__ void expand_quad(const SceneView &sv, const DRay &ray
                       (quad_perm<QUAD_ROT3>(key) > key ? 1 : 0);  // children farther than this lane's
     const bool nearest = hit && below == n - 1;
     const float t = __uint_as_float(key & ~3u);
+    quad_stack_order();
     if (hit && !nearest) st.store(st.sp + below, code, t);
+    quad_stack_order();
     st.has = n > 0;
     st.sp += n > 0 ? n - 1 : 0;
     st.code = (int32_t)quad_or(nearest ? (uint32_t)code : 0u);
@@ -127,7 +138,9 @@ __device__ __forceinline__ void traverse_quad_pass(const SceneView &sv, DRay &ra
             }
             if (items) {
                 const uint32_t links = quad_bits(__ballot(link));
+                quad_stack_order();
                 if (link) st.store(st.sp + __popc(links & ((1u << c) - 1u)), sv.items[start + i].index, st.t);
+                quad_stack_order();
                 st.sp += __popc(links);
             }
         }

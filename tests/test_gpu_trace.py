@@ -7,7 +7,8 @@ import numpy as np
 import pytest
 
 import oracle
-from rayna_amd import Renderer, presets
+from rayna_amd import Camera, Renderer, RenderOpts, presets
+from tests.test_stack_bound import deep_scene
 
 pytestmark = pytest.mark.gpu
 
@@ -67,3 +68,18 @@ def test_camera_ray_time_of_unequal_chunks(gpu, first, last):
             shares.append(s.extend_camera_ms / s.extend_ms)
         assert s.extend_launches == 2 * (opts.ray_depth + 1)
     assert 0.02 < np.median(shares) < 0.4
+
+
+@pytest.mark.parametrize("width,height,samples", [(1, 1, 1), (37, 23, 3), (150, 120, 7)])
+def test_quad_stacks_past_their_lds_share(gpu, width, height, samples):
+    """Four lanes to a path (up to 2^17 of them) on a tree that takes 55 stack entries, 44 of them in LDS; and with 16
+    samples to a pixel the first bounce from the camera-ray packets' hits."""
+    scene = deep_scene()
+    cam = Camera(pos=(0.2, 0.0, 0.0), fwd=(1.0, 0.0, 0.0), v_fov=60.0, focus_dist=1.0)
+    for spp in (samples, 16):
+        opts = RenderOpts(width, height, spp, 4)
+        with Renderer(scene, cam, opts) as r:
+            out = r.render(layout="rowmajor")
+        ref, segments, _, _ = oracle.TwinScene(scene).render(cam, opts, precision=32, box_mode=oracle.BOX_TIGHT)
+        assert np.array_equal(out.img, ref)
+        assert out.stats.segments == segments

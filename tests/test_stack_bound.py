@@ -195,3 +195,60 @@ def test_speculation_can_exceed_the_depth_first_bound():
     rng = np.random.default_rng(9)
     peak = max(lane_peak(tree, rng, 1.0, 1.0) for _ in range(200))
     assert tree.packet_need < peak <= tree.stack_need, (tree.packet_need, peak, tree.stack_need)
+
+
+def quad_peak(tree, rng, p_hit):
+    """Peak of a quad's stack (four lanes to a path): the quad holds one entry beside it; of a node's children that its
+    ray hits it holds the nearest and stores the others; a range's mesh-BVH links are stored when its primitives have
+    been tested."""
+    held, stack, peak = ("node", tree.root), [], 0
+    while held is not None or stack:
+        if held is None:
+            held = stack.pop()
+            if rng.random() > p_hit:  # culled against the closest hit so far
+                held = None
+                continue
+        if held[0] == "node":
+            kids = [c for c in tree.children(held[1]) if rng.random() < p_hit]
+            rng.shuffle(kids)
+            held = kids.pop() if kids else None
+            stack.extend(kids)
+        else:
+            _, start, count, kind = held
+            if kind == LEAF_ITEMS:
+                stack.extend(("node", int(tree.items[start + i, 1])) for i in range(count)
+                             if int(tree.items[start + i, 0]) == ITEM_LINK)
+            held = None
+        peak = max(peak, len(stack))
+    return peak
+
+
+@pytest.mark.parametrize("name", sorted(n for n in SCENES if "instances" not in n and n not in ("adversarial_all", "rttnw")))
+def test_quad_stack_stays_within_packet_need(name):
+    """Quads trace scenes without instances; entry i of a quad's stack lies in LDS or, past that, in the overflow
+    column of its first lane, which has room for stack_need entries less a lane's LDS share."""
+    tree = Tree(SCENES[name]())
+    rng = np.random.default_rng(10)
+    peak = max(quad_peak(tree, rng, p) for p in (1.0, 0.9, 0.6) for _ in range(60))
+    assert peak <= tree.packet_need <= tree.stack_need, (peak, tree.packet_need, tree.stack_need)
+
+
+def deep_scene():
+    """Pairs of triangles across the x axis at distances 1, 2, 4, ..., each as wide as it is far: the tree is a chain,
+    and a ray from the origin along x meets every box of it, the rest of the chain nearest."""
+    x = np.array([2.0 ** k * f for k in range(60) for f in (1.0, 1.05)])
+    v = np.array([[[a, -0.5 * a, -0.5 * a], [a, 0.5 * a, -0.5 * a], [a, 0.0, 0.5 * a]] for a in x])
+    mesh = TriangleListMesh(v, np.tile((-1.0, 0.0, 0.0), (len(v), 3, 1)))
+    return Scene([SimpleObject(mesh, LambertianMaterial((0.7, 0.6, 0.5)))], SimpleSkybox)
+
+
+def test_deep_scene_outgrows_the_quads_lds_stack():
+    """On deep_scene a quad holds the chain's next node and stores its siblings: 55 entries on the way to the nearest
+    triangles, of which 44 fit its LDS share (tests/test_gpu_trace.py traces it)."""
+    tree = Tree(deep_scene())
+    stored, e = 0, ("node", tree.root)
+    while e[0] == "node" or e[3] == LEAF_ITEMS:
+        kids = tree.children(e[1]) if e[0] == "node" else [("node", int(tree.items[e[1] + i, 1])) for i in range(e[2])]
+        e = next((k for k in kids if k[0] == "node"), kids[0])
+        stored += len(kids) - 1
+    assert 44 < stored < tree.packet_need <= PACKET_STACK
