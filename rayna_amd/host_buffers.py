@@ -25,16 +25,24 @@ import numpy as np
 
 IDLE_BYTES = 256 << 20
 PINNED_BYTES = 1 << 30
+# Waiting for a device that has just worked takes 8-13 us, of the 145 us that a 64x36 frame takes, but one wait does for
+# all that was given back before it: so SPARE buffers of up to SPARE_BYTES take turns where torch uses a GPU.
+SPARE = 8
+SPARE_BYTES = 8 << 20
 
 
-def _settled() -> bool:
-    """Waits for the copies that the program may have had torch make from or to dropped arrays: from and to pinned
-    memory they run on when asked not to block, so a buffer is in use until they end.  False if that is not known."""
+def _devices_elsewhere_in_use() -> list:
+    """The devices on which torch may still be copying from or to dropped arrays: copies from and to pinned memory run on
+    after the call when asked not to block."""
     torch = sys.modules.get("torch")
     if torch is None or not hasattr(torch, "cuda") or not torch.cuda.is_initialized():
-        return True
+        return []
+    return [d for d in range(torch.cuda.device_count()) if torch._C._cuda_hasPrimaryContext(d)]
+
+
+def _settle(devices: list) -> bool:
+    """Waits for those copies.  False if that cannot be done."""
     from .renderer import lib
-    devices = [d for d in range(torch.cuda.device_count()) if torch._C._cuda_hasPrimaryContext(d)]
     return all(lib().rayna_host_settle(d) == 0 for d in devices)
 
 
@@ -45,8 +53,10 @@ class _Pool:
         self._lock = threading.RLock()
         self._busy = False
         self._returned = deque()  # (address, size) given back and not yet counted
-        self._idle = OrderedDict()  # address -> size, the longest unused first
+        self._idle = OrderedDict()  # address -> (size, the how many-th to be given back), the longest unused first
         self._by_size = {}  # size -> the idle addresses, likewise
+        self._given = 0  # buffers given back so far
+        self._settled = 0  # no copy is under way in those of them up to here
         self._live = {}  # address -> (bytes asked for, size)
         self._inherited = set()  # in a forked child: the addresses of the parent's arrays
         self._copies = []
@@ -69,10 +79,11 @@ class _Pool:
             del self._live[address]
             self.used_bytes -= size
             self.idle_bytes += size
-            self._idle[address] = size
+            self._given += 1
+            self._idle[address] = size, self._given
             self._by_size.setdefault(size, deque()).append(address)
             while self.idle_bytes > IDLE_BYTES:
-                oldest, oldest_size = self._idle.popitem(last=False)
+                oldest, (oldest_size, _) = self._idle.popitem(last=False)
                 self._by_size[oldest_size].popleft()
                 self.idle_bytes -= oldest_size
                 gone.append(oldest)
@@ -88,7 +99,7 @@ class _Pool:
     def take(self, n: int):
         """(address, size) of a buffer of at least n bytes, or None."""
         size = self._size(n)
-        got = None
+        got, devices, upto = None, [], 0
         with self._lock:
             if self._busy or size > IDLE_BYTES:
                 return None
@@ -98,8 +109,16 @@ class _Pool:
                 fits = self.used_bytes + size <= PINNED_BYTES
                 if fits:
                     self.used_bytes += size
-                    if self._by_size.get(size):
-                        got = self._by_size[size].pop()
+                    same = self._by_size.get(size)
+                    if same and self._idle[same[0]][1] <= self._settled:
+                        got = same.popleft()
+                    elif same:
+                        devices = _devices_elsewhere_in_use()
+                        if not devices:
+                            got = same.pop()
+                        elif len(same) >= SPARE or size > SPARE_BYTES:
+                            got, upto = same.popleft(), self._given
+                    if got is not None:
                         del self._idle[got]
                         self.idle_bytes -= size
                         self._live[got] = n, size
@@ -107,10 +126,13 @@ class _Pool:
                 self._busy = False
         self._free(gone)
         if got is not None:
-            if _settled():
-                return got, size
-            self.give_back(got, size)
-            return None
+            if upto:
+                if not _settle(devices):
+                    self.give_back(got, size)
+                    return None
+                with self._lock:
+                    self._settled = max(self._settled, upto)
+            return got, size
         if not fits:
             return None
         from .renderer import lib

@@ -255,6 +255,7 @@ def test_images_may_be_dropped_while_a_graph_is_captured(gpu, monkeypatch, mode,
     import torch
     monkeypatch.setattr(host_buffers, "_pool", host_buffers._Pool())
     monkeypatch.setattr(host_buffers, "IDLE_BYTES", 5 << 20)
+    monkeypatch.setattr(host_buffers, "SPARE_BYTES", 0)
     images = [host_buffers.empty(4 << 20, np.uint8) for _ in range(3)]
     x = torch.zeros(64, device="cuda")
     y = torch.zeros(64, device="cuda")
@@ -291,6 +292,7 @@ def test_copies_in_flight_have_ended_before_a_buffer_is_used_again(gpu, monkeypa
     next image keeps what is written to it."""
     import torch
     monkeypatch.setattr(host_buffers, "_pool", host_buffers._Pool())
+    monkeypatch.setattr(host_buffers, "SPARE_BYTES", 0)
     a = torch.randn(8192, 8192, device="cuda", dtype=torch.bfloat16)
     dev = torch.full((1 << 18,), 3.0, device="cuda")
     stream = torch.cuda.Stream() if side else torch.cuda.current_stream()
@@ -307,22 +309,43 @@ def test_copies_in_flight_have_ended_before_a_buffer_is_used_again(gpu, monkeypa
             torch.from_numpy(img).copy_(dev, non_blocking=True)
     del img
     gc.collect()
-    new = host_buffers.empty(1 << 18, np.float32)
-    assert new.ctypes.data == at
-    new[:] = -1.0
+    new = []
+    while not new or new[-1].ctypes.data != at:
+        new.append(host_buffers.empty(1 << 18, np.float32))
+        new[-1][:] = -1.0
     torch.cuda.synchronize()
-    assert (dev == (7.0 if to_device else 3.0)).all() and (new == -1.0).all()
+    assert (dev == (7.0 if to_device else 3.0)).all() and all((a == -1.0).all() for a in new)
     del b
 
 
+@pytest.fixture(autouse=True)
+def only_this_library_uses_a_device(request, monkeypatch):
+    """For the tests on a stand-in library, whatever ran in the process before."""
+    if "fake" in request.fixturenames:
+        monkeypatch.setattr(host_buffers, "_devices_elsewhere_in_use", lambda: [])
+
+
 def test_a_buffer_that_may_be_in_use_is_not_handed_out(fake, monkeypatch):
-    """Where it cannot be known that the copies have ended, the array is an ordinary one."""
-    a = host_buffers.empty(1000, np.uint8)
-    at = a.ctypes.data
-    del a
-    gc.collect()
-    with monkeypatch.context() as m:
-        m.setattr(host_buffers, "_settled", lambda: False)
-        b = host_buffers.empty(1000, np.uint8)
-        assert b.ctypes.data != at and host_buffers._pool.used_bytes == 0 and len(fake.held) == 1
-    assert host_buffers.empty(1000, np.uint8).ctypes.data == at
+    """Where torch uses a device, a buffer is handed out again after a wait for the device that began after it was given
+    back, one wait for all of these; small ones take turns; and where the wait fails, the array is an ordinary one."""
+    waits, ok = [], True
+    monkeypatch.setattr(host_buffers, "_devices_elsewhere_in_use", lambda: [0, 1])
+    monkeypatch.setattr(host_buffers, "_settle", lambda devices: (waits.append(devices), ok)[1])
+    monkeypatch.setattr(host_buffers, "SPARE_BYTES", 4096)
+
+    def use(n):
+        a = host_buffers.empty(n, np.uint8)
+        return a.ctypes.data
+
+    at = [use(1000) for _ in range(100)]
+    assert len(fake.held) == len(set(at)) == host_buffers.SPARE
+    assert 100 / host_buffers.SPARE - 2 <= len(waits) <= 100 / host_buffers.SPARE and waits[0] == [0, 1]
+    del waits[:]
+    assert len({use(5000) for _ in range(10)}) == 1 and len(waits) == 9  # larger: a wait each time
+    a = host_buffers.empty(5000, np.uint8)
+    del a, waits[:]
+    ok = False
+    b = host_buffers.empty(5000, np.uint8)
+    assert len(waits) == 1 and b.ctypes.data not in fake.held and host_buffers._pool.used_bytes == 0
+    ok = True
+    assert use(5000) in fake.held
