@@ -742,16 +742,22 @@ rayna_status rayna_render_batch(rayna_batch *b, const rayna_request *reqs, int32
         BHIP(b, enqueue(b, pl, used, true));
     }
     BHIP(b, hipGetLastError());
-    for (int i = 0; i < n; ++i) {
+    // Copies into pinned memory run on after these calls: whatever fails, the images are the caller's again only when
+    // the copies under way have ended.
+    hipError_t copied = hipSuccess;
+    for (int i = 0; i < n && copied == hipSuccess; ++i) {
         if (!reqs[i].out_rgb || !valid[i]) continue;
-        BHIP(b, hipMemcpyAsync(reqs[i].out_rgb, b->out + pl.out_offset[i],
-                               3 * (size_t)reqs[i].opts.width * reqs[i].opts.height * sizeof(float),
-                               hipMemcpyDeviceToHost, b->stream));
+        copied = hipMemcpyAsync(reqs[i].out_rgb, b->out + pl.out_offset[i],
+                                3 * (size_t)reqs[i].opts.width * reqs[i].opts.height * sizeof(float),
+                                hipMemcpyDeviceToHost, b->stream);
     }
     unsigned long long seg[MAX_PIPELINES] = {};
-    for (int p = 0; p < used; ++p)
-        BHIP(b, hipMemcpyAsync(&seg[p], b->pipes[p].segments, sizeof(seg[p]), hipMemcpyDeviceToHost, b->stream));
-    BHIP(b, hipStreamSynchronize(b->stream));
+    for (int p = 0; p < used && copied == hipSuccess; ++p)
+        copied = hipMemcpyAsync(&seg[p], b->pipes[p].segments, sizeof(seg[p]), hipMemcpyDeviceToHost, b->stream);
+    const hipError_t waited = hipStreamSynchronize(b->stream);
+    if (waited != hipSuccess) (void)rayna_host_settle(b->device);
+    BHIP(b, copied);
+    BHIP(b, waited);
     unsigned long long segs = 0;
     for (int p = 0; p < used; ++p) segs += seg[p];
     for (int i = 0; i < n; ++i) {

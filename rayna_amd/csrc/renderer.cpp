@@ -599,7 +599,10 @@ rayna_status render_frame(rayna_renderer *r, float *out_rgb, uint8_t *out_rgba, 
             if (ls != RAYNA_OK) return ls;
             HIP_TRY_LAUNCHED(r, hipMemcpyAsync(out_rgba, r->rgba_dev, 4 * P, hipMemcpyDeviceToHost, r->stream));
         }
-        HIP_TRY_LAUNCHED(r, hipStreamSynchronize(r->stream));
+        const hipError_t waited = hipStreamSynchronize(r->stream);
+        // a copy into pinned memory may be under way: the image is the caller's again when it has ended
+        if (waited != hipSuccess) (void)rayna_host_settle(r->device);
+        HIP_TRY_LAUNCHED(r, waited);
         st.accum_frames = r->frames;
         st.samples = P * spp;
         st.segments = *r->segments;
@@ -1040,7 +1043,8 @@ rayna_status rayna_scene_tree(const rayna_scene_desc *scene, int32_t *node_words
 void rayna_destroy(rayna_renderer *r) {
     if (!r) return;
     (void)hipSetDevice(r->device);
-    if (r->stream) (void)hipStreamSynchronize(r->stream);
+    // nothing of this renderer may still write its host word when another has it
+    if (r->stream && hipStreamSynchronize(r->stream) != hipSuccess) (void)rayna_host_settle(r->device);
     free_paths(r);
     free_scene(r->dev);
     if (r->grad) (void)hipFree(r->grad);

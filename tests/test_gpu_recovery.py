@@ -5,13 +5,17 @@ worker (rayna_ui/src/integration/mod.rs:100-125) and builds a new one from the s
 keeps (rayna_ui/src/app.rs:483-495).  Here the failed call reports RAYNA_DEVICE_ERROR, every later call on that
 renderer RAYNA_RENDERER_LOST, and Renderer.recreated() is the caller's restart: its frames are bit-identical to
 a fresh renderer's and to the oracle's."""
+import ctypes as C
+import threading
+
 import numpy as np
 import pytest
 
 import oracle
-from rayna_amd import Renderer, RayError, presets
+from rayna_amd import Renderer, RayError, host_buffers, presets
 from rayna_amd import _abi as A
-from rayna_amd.renderer import debug_fail_launches
+from rayna_amd.batch import BatchRenderer
+from rayna_amd.renderer import debug_fail_launches, lib
 
 pytestmark = pytest.mark.gpu
 
@@ -94,3 +98,41 @@ def test_failed_adjoint_and_srgb8_lose_the_renderer(gpu, injection):
         assert np.array_equal(r.render_srgb8().img, rgba_ref)
     finally:
         r.close()
+
+
+@pytest.mark.parametrize("call", ["render", "render_srgb8", "batch"])
+def test_a_refused_wait_leaves_no_copy_in_flight(gpu, call):
+    """While another thread captures a graph in the global mode the runtime refuses to wait for a stream, so a call fails
+    after its frame and the copy of its image are under way.  It returns only when they have ended: pinned image memory
+    goes back to a pool and to the next image."""
+    sc, cam, opts = presets.triangle_mesh(subdiv=4, width=1920, height=1080, samples=64)
+    n = opts.width * opts.height
+    hip = C.CDLL(next(line.split()[-1] for line in open("/proc/self/maps") if "libamdhip64" in line))
+    stream, graph = C.c_void_p(), C.c_void_p()
+    assert hip.hipStreamCreateWithFlags(C.byref(stream), 1) == 0
+    L = lib()
+    img = host_buffers.empty(3 * n, np.float32)
+    out = img.ctypes.data_as(C.POINTER(C.c_float))
+    statuses = []
+    with Renderer(sc, cam, opts) as r, BatchRenderer([sc]) as b:
+        q = (A.Request * 1)(A.Request(0, A.LAYOUT_ROWMAJOR, cam.desc(), opts.desc(), out))
+        calls = {"render": lambda: L.rayna_render(r._h, out, A.LAYOUT_ROWMAJOR, None, None),
+                 "render_srgb8": lambda: L.rayna_render_srgb8(r._h, C.cast(out, C.POINTER(C.c_uint8)), None, None),
+                 "batch": lambda: L.rayna_render_batch(b._h, q, 1, None)}
+
+        def refused():
+            statuses.append(calls[call]())
+            img[:] = -1.0
+
+        assert calls[call]() == A.RAYNA_OK
+        img[:] = 5.0
+        assert hip.hipStreamBeginCapture(stream, 0) == 0
+        t = threading.Thread(target=refused)
+        t.start()
+        t.join()
+        hip.hipStreamEndCapture(stream, C.byref(graph))
+        hip.hipGetLastError()
+        assert hip.hipDeviceSynchronize() == 0
+        assert statuses == [A.RAYNA_DEVICE_ERROR]
+        assert (img == -1.0).all()
+    hip.hipStreamDestroy(stream)
