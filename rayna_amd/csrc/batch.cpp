@@ -261,7 +261,7 @@ rayna_status validate(rayna_batch *b, const rayna_request &q, int i) {
         return bfail(b, RAYNA_INVALID_ARGUMENT, at + "zero width, height, samples or branching");
     if (o.ray_branching != 1) return bfail(b, RAYNA_UNSUPPORTED, at + "ray_branching > 1");
     if (o.mode != RAYNA_MODE_PBR) return bfail(b, RAYNA_UNSUPPORTED, at + "only RenderMode::PBR");
-    if (o.ray_depth > 1000) return bfail(b, RAYNA_UNSUPPORTED, at + "ray_depth above 1000");
+    if (o.ray_depth > MAX_RAY_DEPTH) return bfail(b, RAYNA_UNSUPPORTED, at + "ray_depth above 1000");
     if ((uint64_t)o.width * o.height > b->chunk_slots)
         return bfail(b, RAYNA_UNSUPPORTED, at + "more pixels than paths per chunk");
     return RAYNA_OK;
@@ -478,6 +478,7 @@ hipError_t enqueue(rayna_batch *b, const Plan &pl, int used, bool timing) {
         const SceneView cv = chunk_view(b->view, pl.features[c], pl.n_nodes[c]);
         launch_fill_u32(P.queue_count, 0u, 3 * (D + 2), s);
         launch_fill_u32(P.claims, 0u, SEGMENT_WORDS + (D + 1) * 2 * CLAIM_WORDS, s);
+        SegmentCounter *queries = reinterpret_cast<SegmentCounter *>(P.claims);
         uint32_t *claims = P.claims + SEGMENT_WORDS;
         const uint32_t apart = std::min(D + 1, launched_depths(cv, fp, b->tune, bv));
         // the camera rays are stored only where a kernel loads them: k_extend and k_march at depth 0 (the camera-ray
@@ -491,7 +492,7 @@ hipError_t enqueue(rayna_batch *b, const Plan &pl, int used, bool timing) {
             uint32_t *cout = P.queue_count + depth + 1;
             uint32_t *work = claims + (size_t)depth * 2 * CLAIM_WORDS;
             if (depth >= apart) {  // every path to its end
-                launch_trace(cv, fp, P.pb, qin, cin, depth, b->grid_extend, P.overflow, work, P.claims, b->tune,
+                launch_trace(cv, fp, P.pb, qin, cin, depth, b->grid_extend, P.overflow, work, queries, b->tune,
                              nullptr, bv, s);
                 break;
             }
@@ -501,7 +502,7 @@ hipError_t enqueue(rayna_batch *b, const Plan &pl, int used, bool timing) {
                          P.queue_count + 2 * (D + 2) + depth, s);
             launch_shade(cv, fp, P.pb, qin, cin, qout, cout, depth, b->grid_shade, nullptr, bv, s);
         }
-        launch_count_segments(SegmentCount{P.queue_count, apart, apart > 0 ? fp.n_slots : 0u, P.claims, P.segments, 0u}, s);
+        launch_count_segments(SegmentCount{P.queue_count, apart, apart > 0 ? fp.n_slots : 0u, queries, P.segments, 0u}, s);
         // (a dependency on the same pipeline is kept by its stream's order)
         if (used > 1 && pl.dep[c] >= 0 && (size_t)pl.dep[c] % used != c % used)
             check(hipStreamWaitEvent(s, b->resolved[pl.dep[c]], 0));

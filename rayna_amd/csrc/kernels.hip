@@ -1293,7 +1293,7 @@ __device__ __forceinline__ void count_segments(const SegmentCount &sc) {
     const uint32_t lane = __lane_id();
     unsigned long long s = 0;
     for (uint32_t i = 1 + lane; i < sc.n; i += 64) s += sc.queue_count[i];
-    for (uint32_t i = lane; i < SEGMENT_PARTS; i += 64) s += sc.parts[32 * i];
+    for (uint32_t i = lane; i < SEGMENT_PARTS; i += 64) s += sc.parts[SEGMENT_STRIDE * i];
     for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
     if (lane == 0u) *sc.segments = (sc.first ? 0ull : *sc.segments) + s + sc.first_count;
 }
@@ -1638,7 +1638,7 @@ uint32_t launched_depths(const SceneView &sv, const FrameParams &fp, const Exten
 
 void launch_trace(const SceneView &sv, const FrameParams &fp, const PathBuffers &pb, const int32_t *queue,
                   const uint32_t *count, uint32_t first_depth, int grid, int2 *overflow, uint32_t *work,
-                  uint32_t *segments, const ExtendTuning &tune, const AdjointParams *adjoint, const BatchView &bv,
+                  SegmentCounter *segments, const ExtendTuning &tune, const AdjointParams *adjoint, const BatchView &bv,
                   hipStream_t s) {
     const int k = bv.reqs ? 1 : adjoint ? 2 : 0, t = sv.textured ? 1 : 0, i = sv.instances ? 1 : 0;
     const int f = extend_form(sv), fs = i || t ? 2 : f ? 1 : 0;

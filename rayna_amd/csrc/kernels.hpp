@@ -95,9 +95,16 @@ void launch_generate(const FrameParams &fp, const PathBuffers &pb, const BatchVi
 constexpr uint32_t CLAIM_PARTS = RAYNA_CLAIM_PARTS;
 constexpr uint32_t CLAIM_WORDS = CLAIM_PARTS * 32;
 
-// k_trace's counters of closest-hit queries, one 128-byte line apart.
+// Deepest ray_depth that options may ask for.
+constexpr uint32_t MAX_RAY_DEPTH = 1000;
+
+// k_trace's counters of closest-hit queries, one 128-byte line apart (SEGMENT_WORDS words of 32 bits in all).  A wave
+// adds to the counter of its block, so each holds what a whole chunk may come to: 2^32 paths to the depth limit.
+using SegmentCounter = unsigned long long;
 constexpr uint32_t SEGMENT_PARTS = 64;
+constexpr uint32_t SEGMENT_STRIDE = 128 / sizeof(SegmentCounter);
 constexpr uint32_t SEGMENT_WORDS = SEGMENT_PARTS * 32;
+static_assert((SegmentCounter)-1 >> 32 >= MAX_RAY_DEPTH + 1, "a query counter may overflow");
 
 // queue == nullptr: identity queue of fp.n_slots entries; else queue[0 .. *count)
 // overflow: traversal stack entries beyond the LDS part, extend_block() * grid * (stack_need - extend_lds_stack());
@@ -130,7 +137,7 @@ uint32_t launched_depths(const SceneView &sv, const FrameParams &fp, const Exten
 // SEGMENT_WORDS zeroed words, the closest-hit queries (launch_count_segments).
 void launch_trace(const SceneView &sv, const FrameParams &fp, const PathBuffers &pb, const int32_t *queue,
                   const uint32_t *count, uint32_t first_depth, int grid, int2 *overflow, uint32_t *work,
-                  uint32_t *segments, const ExtendTuning &tune, const AdjointParams *adjoint, const BatchView &bv,
+                  SegmentCounter *segments, const ExtendTuning &tune, const AdjointParams *adjoint, const BatchView &bv,
                   hipStream_t s);
 void launch_shade(const SceneView &sv, const FrameParams &fp, const PathBuffers &pb, const int32_t *queue_in,
                   const uint32_t *count_in, int32_t *queue_out, uint32_t *count_out, uint32_t depth, int grid,
@@ -169,7 +176,7 @@ void launch_to_srgb8(const float *img, uint32_t n_pixels, uint8_t *rgba, hipStre
 struct SegmentCount {
     const uint32_t *queue_count;
     uint32_t n, first_count;
-    const uint32_t *parts;
+    const SegmentCounter *parts;
     unsigned long long *segments;
     uint32_t first;
 };

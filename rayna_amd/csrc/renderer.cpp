@@ -368,7 +368,7 @@ rayna_status check_opts(rayna_renderer *r, const rayna_render_opts *o) {
         return fail(r, RAYNA_INVALID_ARGUMENT, "render options must have non-zero width, height, samples, branching");
     if (o->ray_branching != 1) return fail(r, RAYNA_UNSUPPORTED, "ray_branching > 1 is not supported on the GPU");
     if (o->mode < RAYNA_MODE_PBR || o->mode > RAYNA_MODE_SIDE) return fail(r, RAYNA_INVALID_ARGUMENT, "unknown render mode");
-    if (o->ray_depth > 1000) return fail(r, RAYNA_UNSUPPORTED, "ray_depth above 1000");
+    if (o->ray_depth > MAX_RAY_DEPTH) return fail(r, RAYNA_UNSUPPORTED, "ray_depth above 1000");
     return RAYNA_OK;
 }
 
@@ -412,6 +412,7 @@ SegmentCount trace_chunk(rayna_renderer *r, FrameParams &fp, uint32_t s0, uint32
     const uint32_t D2 = r->opts.ray_depth + 2;
     launch_fill_u32(r->queue_count, 0u, (uint32_t)(r->claims - r->queue_count) + SEGMENT_WORDS + D2 * 2 * CLAIM_WORDS,
                     r->stream);
+    SegmentCounter *queries = reinterpret_cast<SegmentCounter *>(r->claims);
     uint32_t *claims = r->claims + SEGMENT_WORDS;
     bool launched = true;  // since the last event
     auto mark = [&] {
@@ -439,8 +440,8 @@ SegmentCount trace_chunk(rayna_renderer *r, FrameParams &fp, uint32_t s0, uint32
         if (ev) r->camera_at.push_back(depth == 0 && !rest);
         launched = true;
         if (rest) {
-            launch_trace(r->dev.view, fp, r->pb, qin, cin, depth, r->grid_extend, r->dev.overflow, work, r->claims,
-                         r->tune, adjoint, BatchView{}, r->stream);
+            launch_trace(r->dev.view, fp, r->pb, qin, cin, depth, r->grid_extend, r->dev.overflow, work, queries, r->tune,
+                         adjoint, BatchView{}, r->stream);
         } else {
             launch_extend(r->dev.view, fp, r->pb, qin, cin, depth, r->grid_extend, r->dev.overflow, work, r->tune,
                           BatchView{}, r->stream);
@@ -458,7 +459,7 @@ SegmentCount trace_chunk(rayna_renderer *r, FrameParams &fp, uint32_t s0, uint32
         mark();
         if (rest || fp.mode != RAYNA_MODE_PBR) break;
     }
-    return SegmentCount{r->queue_count, apart, apart > 0 ? fp.n_slots : 0u, r->claims, r->segments, first ? 1u : 0u};
+    return SegmentCount{r->queue_count, apart, apart > 0 ? fp.n_slots : 0u, queries, r->segments, first ? 1u : 0u};
 }
 
 rayna_status ensure_events(rayna_renderer *r, size_t n) {

@@ -32,11 +32,18 @@ struct TraceArgs {
     const uint32_t *count;
     uint32_t first_depth;
     int2 *overflow;
-    uint32_t *work, *segments;
+    uint32_t *work;
+    SegmentCounter *segments;
     ExtendTuning tune;
     AdjointParams ap;
     BatchView bv;
 };
+// Adds the closest-hit queries that the wave's lanes counted to one of the SEGMENT_PARTS counters.
+__device__ __forceinline__ void add_segments(SegmentCounter *segments, uint32_t lane_count) {
+    SegmentCounter n = lane_count;
+    for (int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o);
+    if (__lane_id() == 0u && n != 0) atomicAdd(segments + SEGMENT_STRIDE * (blockIdx.x % SEGMENT_PARTS), n);
+}
 // The arguments again, read where they are used: some ninety words of them serve the shading and refill alone, and
 // loaded once at the kernel's start they would hold (and spill, into vector registers) scalar registers through the
 // traversal loops.  The compiler cannot move these loads out of the loop, because it does not know the pointer.
@@ -218,7 +225,5 @@ __global__ __launch_bounds__(EXT_BLOCK) __attribute__((amdgpu_waves_per_eu(trace
         }
     }
     stats.flush();
-    // the wave's closest-hit queries, added to one of SEGMENT_PARTS counters a line apart
-    for (int o = 32; o > 0; o >>= 1) n_segments += __shfl_xor(n_segments, o);
-    if (lane == 0u && n_segments != 0u) atomicAdd(args.segments + 32 * (blockIdx.x % SEGMENT_PARTS), n_segments);
+    add_segments(args.segments, n_segments);
 }

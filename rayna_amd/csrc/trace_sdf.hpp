@@ -228,7 +228,5 @@ __global__ __launch_bounds__(EXT_BLOCK) __attribute__((amdgpu_waves_per_eu(SDF_T
         }
     }
     stats.flush();
-    // the wave's closest-hit queries, added to one of SEGMENT_PARTS counters a line apart
-    for (int o = 32; o > 0; o >>= 1) n_segments += __shfl_xor(n_segments, o);
-    if (lane == 0u && n_segments != 0u) atomicAdd(args.segments + 32 * (blockIdx.x % SEGMENT_PARTS), n_segments);
+    add_segments(args.segments, n_segments);
 }
