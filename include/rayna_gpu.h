@@ -340,8 +340,12 @@ rayna_status rayna_adjoint(rayna_renderer *r, uint32_t frame, const float *d_ima
 /* Launch shape of the wavefront kernels.  Zero fields keep the default. */
 typedef struct rayna_tuning {
     uint32_t chunk_slots;          /* paths in flight per chunk (default 2^27 for a renderer, 2^29 for a batch) */
-    uint32_t refill_lanes;         /* extend: idle lanes of a wave before it takes new rays, 1..64 (default 32) */
-    uint32_t wave_batch;           /* extend: queue positions a wave claims per atomic, 1..4096 (default 128) */
+    uint32_t refill_lanes;         /* extend, march: idle lanes of a wave before it takes new rays, 1..64 (default 32);
+                                    * the launches that take whole paths, where a refill shades too, wait for 5/4 as
+                                    * many lanes, with unbounded objects for 3/2, or half as many if one of them is
+                                    * a Mandelbulb */
+    uint32_t wave_batch;           /* extend: most queue positions a wave claims at a time, 1..4096 (default 128);
+                                    * march items: four times, paths with four lanes each: an eighth of it */
     uint32_t shade_blocks_per_cu;  /* shade: blocks of 256 threads per compute unit, 1..64 (default 16) */
     int32_t use_graph;             /* batches: capture the launch sequence in a hipGraph and replay it (1) */
     int32_t schedule;              /* batches: 0 = requests in the given order, 1 = fewest samples first,

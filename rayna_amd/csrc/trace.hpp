@@ -21,7 +21,10 @@ constexpr int trace_waves(bool inst, bool sph, bool vol) { return inst || vol ? 
 constexpr uint32_t TRACE_CLAIM_LEAST = 4;
 // With four lanes to a path a wave holds sixteen: more at a time would leave the others idle (the four mesh preview
 // frames at most 8, 16 and 32: 2.74, 2.73 and 3.18 ms; the sphere thumbnail at least 1, 2 and 4: 161, 171 and 170 us).
-constexpr uint32_t QUAD_CLAIM_LEAST = 1, QUAD_CLAIM_MOST = 16;
+constexpr uint32_t QUAD_CLAIM_LEAST = 1;
+__device__ __forceinline__ uint32_t quad_claim_most(const ExtendTuning &tune) {  // 16 for the default of 128
+    return tune.wave_batch / 8u > QUAD_CLAIM_LEAST ? tune.wave_batch / 8u : QUAD_CLAIM_LEAST;
+}
 
 // The arguments of k_trace and k_trace_sdf, one struct so that a kernel finds them at the start of its argument segment.
 struct TraceArgs {
@@ -87,7 +90,7 @@ __global__ __launch_bounds__(EXT_BLOCK) __attribute__((amdgpu_waves_per_eu(trace
     LeafRange leaf;
     TravStats stats;
     WaveClaims claims(count, EXT_BLOCK / 64, QUAD ? QUAD_CLAIM_LEAST : TRACE_CLAIM_LEAST,
-                      QUAD ? QUAD_CLAIM_MOST : args.tune.wave_batch, args.work);
+                      QUAD ? quad_claim_most(args.tune) : args.tune.wave_batch, args.work);
     // the path's RNG key, pixel and sample, and in a batch its request
     auto identify = [&](const TraceArgs &A, dm::Key *key, uint32_t *pixel, uint32_t *sample) -> const RequestParams * {
         if (BATCH) {

@@ -25,7 +25,11 @@
 // take, a quarter of its paths (the 161x91, 9-sample frame at half, a quarter, an eighth and a sixty-fourth: 4.31, 4.19,
 // 4.20 and 4.28 ms).
 constexpr int SDF_TRACE_WAVES = 5;
-constexpr uint32_t SDF_REFILL_LANES = 48, BULB_REFILL_LANES = 16;
+__device__ __forceinline__ uint32_t sdf_refill_lanes(const ExtendTuning &tune, bool mandelbulbs) {
+    const uint32_t n = tune.refill_lanes;  // 32 by default: 16 and 48 then
+    if (mandelbulbs) return n > 1u ? n / 2u : 1u;
+    return n + n / 2u < 64u ? n + n / 2u : 64u;
+}
 
 template <bool BATCH, bool INST, bool SPH, bool VOL, bool TEX, bool ADJOINT>
 __global__ __launch_bounds__(EXT_BLOCK) __attribute__((amdgpu_waves_per_eu(SDF_TRACE_WAVES))) void k_trace_sdf(
@@ -48,7 +52,7 @@ __global__ __launch_bounds__(EXT_BLOCK) __attribute__((amdgpu_waves_per_eu(SDF_T
     int step = 0;                     // the march's step; the normal's estimate (0..5: +x -x +y -y +z -z)
     f3 g{0.0f, 0.0f, 0.0f};           // the estimate's differences, then the normal
     WaveClaims claims(count, EXT_BLOCK / 64, TRACE_CLAIM_LEAST, args.tune.wave_batch, args.work);
-    const uint32_t refill_lanes = args.sv.mandelbulbs ? BULB_REFILL_LANES : SDF_REFILL_LANES;
+    const uint32_t refill_lanes = sdf_refill_lanes(args.tune, args.sv.mandelbulbs != 0);
     TravStats stats;
     // the path's RNG key, pixel and sample, and in a batch its request
     auto identify = [&](const TraceArgs &A, dm::Key *key, uint32_t *pixel, uint32_t *sample) -> const RequestParams * {

@@ -83,3 +83,20 @@ def test_quad_stacks_past_their_lds_share(gpu, width, height, samples):
         ref, segments, _, _ = oracle.TwinScene(scene).render(cam, opts, precision=32, box_mode=oracle.BOX_TIGHT)
         assert np.array_equal(out.img, ref)
         assert out.stats.segments == segments
+
+
+@pytest.mark.parametrize("scene,width,height,samples,knob", [("mixed", 640, 360, 64, "refill_lanes"),
+                                                            ("cornell", 360, 360, 1, "wave_batch")])
+def test_tuning_reaches_the_whole_path_launches(gpu, scene, width, height, samples, knob):
+    """Scenes with unbounded objects heed refill_lanes and paths with four lanes wave_batch: one lane, or one path, at a
+    time takes far longer than the default (1.6 and 2.2 times; a fifth is asked for), and no value changes the image."""
+    sc, cam, opts = SCENES[scene](width=width, height=height, samples=samples)
+    times, images = [], []
+    with Renderer(sc, cam, opts) as r:
+        for v in (0, 1, 64 if knob == "refill_lanes" else 4096):
+            r.set_tuning(**{knob: v})
+            r.clear_accumulation()
+            images.append(r.render(layout="rowmajor").img)
+            times.append(np.median([r.render(to_host=False).stats.kernel_ms for _ in range(7)]))
+    assert all(np.array_equal(images[0], i) for i in images[1:])
+    assert times[1] > 1.2 * times[0]
