@@ -189,7 +189,7 @@ rayna_status alloc_pipe(rayna_batch *b, int p, uint64_t slots, uint32_t max_dept
         else BHIP(b, hipStreamCreateWithFlags(&P.stream, hipStreamNonBlocking));
     }
     if (!P.done) BHIP(b, hipEventCreateWithFlags(&P.done, hipEventDisableTiming));
-    if (P.capacity >= slots && P.queue_count_len >= 3 * (max_depth + 2)) return RAYNA_OK;
+    if (P.capacity >= slots && P.queue_count_len >= 2 * (max_depth + 2)) return RAYNA_OK;
     free_pipe(b, P);
     auto alloc = [&](size_t bytes, void **out) -> rayna_status {
         BHIP(b, hipMalloc(out, std::max<size_t>(bytes, 4)));
@@ -207,10 +207,10 @@ rayna_status alloc_pipe(rayna_batch *b, int p, uint64_t slots, uint32_t max_dept
     if ((st = alloc(slots * sizeof(uint32_t), (void **)&P.slot_req)) != RAYNA_OK) return st;
     for (int q = 0; q < 2; ++q)
         if ((st = alloc(slots * sizeof(int32_t), (void **)&P.queue[q])) != RAYNA_OK) return st;
-    // [0, D+2) paths entering each depth; [2(D+2), 3(D+2)) SDF hits at each depth
-    const uint32_t qlen = 3 * (std::max<uint32_t>(max_depth, 16) + 2);
+    // [0, D+2) paths entering each depth; [D+2, 2(D+2)) SDF hits at each depth
+    const uint32_t qlen = 2 * (std::max<uint32_t>(max_depth, 16) + 2);
     if ((st = alloc(qlen * sizeof(uint32_t), (void **)&P.queue_count)) != RAYNA_OK) return st;
-    if ((st = alloc((SEGMENT_WORDS + (size_t)(qlen / 3) * 2 * CLAIM_WORDS) * sizeof(uint32_t), (void **)&P.claims)) != RAYNA_OK)
+    if ((st = alloc((SEGMENT_WORDS + (size_t)qlen * CLAIM_WORDS) * sizeof(uint32_t), (void **)&P.claims)) != RAYNA_OK)
         return st;
     if ((st = alloc(sizeof(unsigned long long), (void **)&P.segments)) != RAYNA_OK) return st;
     if (b->n_sdf_max) {
@@ -476,7 +476,7 @@ hipError_t enqueue(rayna_batch *b, const Plan &pl, int used, bool timing) {
         fp.ray_depth = pl.depth[c];
         const uint32_t D = pl.depth[c];
         const SceneView cv = chunk_view(b->view, pl.features[c], pl.n_nodes[c]);
-        launch_fill_u32(P.queue_count, 0u, 3 * (D + 2), s);
+        launch_fill_u32(P.queue_count, 0u, 2 * (D + 2), s);
         launch_fill_u32(P.claims, 0u, SEGMENT_WORDS + (D + 1) * 2 * CLAIM_WORDS, s);
         SegmentCounter *queries = reinterpret_cast<SegmentCounter *>(P.claims);
         uint32_t *claims = P.claims + SEGMENT_WORDS;
@@ -499,7 +499,7 @@ hipError_t enqueue(rayna_batch *b, const Plan &pl, int used, bool timing) {
             launch_extend(cv, fp, P.pb, qin, cin, depth, b->grid_extend, P.overflow, work, b->tune, bv, s);
             launch_march(cv, fp, P.pb, qin, cin, pl.n_sdf[c], P.mt, P.capacity * b->n_sdf_max,
                          work + CLAIM_WORDS, b->grid_march, b->grid_shade, b->tune, bv, P.sdf_queue,
-                         P.queue_count + 2 * (D + 2) + depth, s);
+                         P.queue_count + D + 2 + depth, s);
             launch_shade(cv, fp, P.pb, qin, cin, qout, cout, depth, b->grid_shade, nullptr, bv, s);
         }
         launch_count_segments(SegmentCount{P.queue_count, apart, apart > 0 ? fp.n_slots : 0u, queries, P.segments, 0u}, s);

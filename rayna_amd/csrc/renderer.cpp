@@ -318,9 +318,9 @@ rayna_status alloc_paths(rayna_renderer *r) {
     const uint64_t slots = P * chunk;
     if (slots > 0x7fffffffull || slots * n_sdf > 0xffffffffull)
         return fail(r, RAYNA_UNSUPPORTED, "image too large for one chunk of paths");
-    // [0, D+2) paths entering each depth; [2(D+2), 3(D+2)) SDF hits at each depth; [3(D+2)]: the primary-hit
-    // query's SDF hits
-    const uint32_t qlen = 3 * (o.ray_depth + 2) + 2;
+    // [0, D+2) paths entering each depth; [D+2, 2(D+2)) SDF hits at each depth; [2(D+2)]: the primary-hit query's
+    // SDF hits
+    const uint32_t qlen = 2 * (o.ray_depth + 2) + 1;
     if (slots <= r->slot_capacity && P <= r->alloc_pixels && qlen <= r->queue_count_len) {
         // the buffers are large enough: keep them (grow-only)
         r->chunk_samples = (uint32_t)chunk;
@@ -447,7 +447,7 @@ SegmentCount trace_chunk(rayna_renderer *r, FrameParams &fp, uint32_t s0, uint32
                           BatchView{}, r->stream);
             launch_march(r->dev.view, fp, r->pb, qin, cin, (uint32_t)r->dev.view.n_sdfs, r->mt, r->mt_cap,
                          work + CLAIM_WORDS, r->grid_march, r->grid_shade, r->tune, BatchView{}, r->sdf_queue,
-                         r->queue_count + 2 * D2 + depth, r->stream);
+                         r->queue_count + D2 + depth, r->stream);
         }
         mark();
         launched = fp.mode != RAYNA_MODE_PBR || !rest;
@@ -942,7 +942,7 @@ rayna_status rayna_primary_hits(rayna_renderer *r, uint32_t sample_index, int32_
     pb.hit_rank = rank_dev;
     r->primal_frame = -1;
     launch_generate(fp, pb, BatchView{}, r->stream);
-    uint32_t *sdf_count = r->queue_count + 3 * (r->opts.ray_depth + 2);
+    uint32_t *sdf_count = r->queue_count + 2 * (r->opts.ray_depth + 2);
     uint32_t *claims = r->claims + SEGMENT_WORDS + (size_t)(r->opts.ray_depth + 2) * 2 * CLAIM_WORDS;
     launch_fill_u32(sdf_count, 0u, 1, r->stream);
     launch_fill_u32(claims, 0u, 2 * CLAIM_WORDS, r->stream);
