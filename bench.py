@@ -21,16 +21,27 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, HERE)
 
 HBM_PEAK_GBPS = 8000.0
-# Algorithmic bytes of one closest-hit query in the extend kernel: queue entry 4 B + ray origin and direction
-# 24 B read, hit distance, reference and flags 12 B written.
-EXTEND_BYTES_PER_SEGMENT = 40
-# Algorithmic bytes of the whole frame, as if every vertex went through memory between two launches (k_trace keeps the
-# later ones in registers), per segment (extend + shade) and per sample (generate + resolve):
-# extend 40 B; shade reads queue 4, ray 24, hit 12, throughput 12, radiance 12 and writes ray 24,
-# throughput 12, radiance 12, queue entry 4 -> 116 B; generate writes the 24 B camera ray per sample, resolve
-# reads 12 B.
-FRAME_BYTES_PER_SEGMENT = 40 + 116
-FRAME_BYTES_PER_SAMPLE = 24 + 12
+# What a frame of a workload must move between its launches, from the rays that go through memory (the others stay in
+# k_trace's registers): camera rays, first-bounce rays (the queue into depth 1) and paths handed to k_trace (the queue
+# into depth 2), counted on the frame of seed 1; the frames after it differ by the noise of 10^8 paths.
+FRAME_RAYS = {"triangle_mesh": (132710400, 92991142, 22352437)}
+
+
+def frame_bytes(workload: str):
+    """(extend stage, whole frame) algorithmic bytes of a frame, or None where the launches are not known here.
+    Extend: a camera ray's hit written (12 B, the ray is computed), a first-bounce ray read and its hit written (queue 4,
+    ray 24, hit 12), a later path's start read and its radiance read and written once (queue 4, ray 24, throughput 12,
+    radiance 24).  Shade: a camera vertex's hit read and radiance written, a bounce's queue entry, ray, hit and throughput
+    read and the radiance of a path that ends there read and written, a surviving path's ray, throughput and queue entry
+    written.  Resolve: a sample's radiance read."""
+    if workload not in FRAME_RAYS:
+        return None
+    camera, bounce, later = FRAME_RAYS[workload]
+    extend = 12 * camera + 40 * bounce + 64 * later
+    shade = 24 * camera + 40 * bounce + 52 * bounce + 24 * (bounce - later) + 40 * later
+    return extend, extend + shade + 12 * camera
+
+
 # Counter-derived figures of the extend stage on the 1080p triangle-mesh frame, from rocprofv3 passes over two
 # frames of 263,040,107 closest-hit queries each (132,710,400 of them camera rays) at the commit that added them;
 # the times they are divided by are measured live.  The stage is k_extend_packet (camera rays), k_extend (the first
@@ -457,11 +468,10 @@ def main(argv=None):
     _progress(f"{a.workload}: {a.steps} timed frames, {secs * 1e3 / a.steps:.2f} ms each")
     samples_per_frame = opts.width * opts.height * opts.samples
     value = samples_per_frame * a.steps / secs / 1e6
-    ext_bytes = EXTEND_BYTES_PER_SEGMENT * segs
-    achieved = ext_bytes / (ext_ms * 1e-3) / 1e9 if ext_ms > 0 else 0.0
+    alg = frame_bytes(a.workload)
+    achieved = alg[0] * a.steps / (ext_ms * 1e-3) / 1e9 if alg and ext_ms > 0 else None
     per_seg = EXTEND_FABRIC_BYTES_PER_SEGMENT.get(a.workload)
     traffic = per_seg * segs / launches if per_seg and launches else None
-    frame_bytes = FRAME_BYTES_PER_SEGMENT * segs + FRAME_BYTES_PER_SAMPLE * samples_per_frame * a.steps
     line = {
         "metric": "Msamples/s at 1080p (triangle-mesh workload, equal-seed parity with the fp32 CPU restatement)",
         "value": value,
@@ -486,18 +496,18 @@ def main(argv=None):
         "render_call_ms_per_frame": call_ms / a.steps,
         "step_ms_min_median_max": [min(step_ms), sorted(step_ms)[len(step_ms) // 2], max(step_ms)],
         "extend_launches_per_frame": launches // max(1, a.steps),
-        "frame_alg_gbps": frame_bytes / secs / 1e9,
+        "frame_alg_gbps": alg[1] * a.steps / secs / 1e9 if alg else None,
         "to_host": {"msamples_per_s": samples_per_frame * a.steps / (t3 - t2) / 1e6,
                     "ms_per_step": (t3 - t2) * 1e3 / a.steps,
                     "note": "each frame's image copied to host memory (x-major float32), as Renderer::render hands it"},
         "scene_build_s": t_build,
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBPS, "unit": "GB/s",
-                     "frac": achieved / HBM_PEAK_GBPS, "traffic": traffic,
+                     "frac": achieved / HBM_PEAK_GBPS if achieved is not None else None, "traffic": traffic,
                      "traffic_kind": "L2-miss (fabric) bytes per depth: rocprofv3 FETCH_SIZE + WRITE_SIZE, "
                                      "calibrated on a 256 MiB copy; Infinity Cache hits included",
                      "kernel": "extend: k_extend_packet (camera rays) + k_extend (first bounce) + k_trace (later "
                                "vertices, shading included)",
-                     "bytes_per_segment": EXTEND_BYTES_PER_SEGMENT},
+                     "bytes_per_frame": alg[0] if alg else None},
     }
     valu = valu_roofline(a.workload, samples_per_frame * a.steps, segs, ext_ms, cam_ms)
     if valu:

@@ -1105,7 +1105,7 @@ __device__ __forceinline__ bool shade_vertex(const SceneView &sv, uint32_t *chec
 }
 
 // One bounce of ray_colour_recursive in forward form: L += T * Le; scatter; T = reflected(T); paths that
-// scatter below the depth limit are compacted into the next queue (one atomic per wave).
+// scatter below the depth limit are compacted into the next queue (one atomic per block and strip).
 //
 // ADJOINT: the same bounce replayed for path replay backpropagation (Vicini, Speierer and Jakob 2021,
 // algorithm 2).  The radiance field holds R, the radiance the path still gathers from this vertex on (the

@@ -125,9 +125,20 @@ void launch_extend(const SceneView &sv, const FrameParams &fp, const PathBuffers
 // With unbounded objects: k_march's waves are full and each at one SDF, k_trace_sdf's do not wait for a depth's
 // longest march.  So the largest chunks launch the camera rays and the first bounce, where most of the work is; small
 // ones the camera rays, most of which march past everything; the smallest, where every launch is a wait, and those in
-// between none.  (The SDF scene with 0, 1, 2 and all depths launched: 64x36x2 3.2, 3.7, 4.3 and 6.2 ms; 640x360x4 8.1,
-// 6.7, 6.9 and 11.3; 640x360x64 18.0, 18.5, 19.2 and 23.4; 1280x720x128 83.1, 75.4, 71.9 and 76.1.  A scene of mostly
-// bounded objects and one SDF: 161x91x9 1.20, 1.04, 0.89 and 1.16; 1280x720x32 7.1, 8.5, 8.3 and 8.1.)
+// between none.  The lines were drawn on the first of these scenes; device ms with 0, 1, 2 and all depths launched:
+//                          64x36x2                 161x91x9                640x360x4               640x360x8
+//   bulb, blobs, medium    3.19 3.50 3.87 6.11     4.52 4.55 5.03 8.79     7.24 6.33 7.06 11.2     9.64 7.40 7.88 12.8
+//   the bulb alone         2.61 3.51 3.64 5.79     3.08 3.92 4.60 8.37     4.34 4.84 5.27 9.88     5.51 5.47 6.04 11.4
+//   the blobs alone        0.65 0.98 1.16 1.44     1.13 1.80 2.25 3.63     1.60 2.22 2.87 4.83     2.28 2.62 3.42 5.74
+//   60 bounded, a sphere   0.52 0.54 0.60 0.75     0.91 0.93 0.82 1.00     1.77 1.71 1.39 1.49     1.87 2.15 1.76 1.84
+//                          640x360x24              640x360x64              1280x720x64             1280x720x128
+//   bulb, blobs, medium    12.0 11.9 10.7 16.5     17.5 18.2 18.5 23.7     44.1 42.4 40.5 49.9     81.2 72.2 67.4 76.9
+//   the bulb alone         7.19 7.42 8.12 14.6     9.79 12.0 12.6 19.3     22.0 23.5 24.4 34.3     36.9 37.9 40.6 52.8
+//   the blobs alone        2.69 4.03 4.54 7.89     4.49 5.58 6.23 10.4     12.9 13.2 13.5 19.1     24.5 23.6 23.0 29.3
+//   60 bounded, a sphere   2.44 2.78 2.65 2.53     3.83 4.59 4.89 4.87     12.2 13.5 13.0 13.9     24.0 25.5 24.0 25.6
+// So between 2^14 and 2^21 paths a scene of one kind of SDF would do better with no launch apart, and one of mostly
+// bounded objects with two; the rule's choice is within 5% of a launch per depth or faster on all of them but the last
+// at 320x180x8 and 640x360x4 and x8 (1.38 against 1.29, 1.71 against 1.49, 2.15 against 1.84).
 constexpr uint32_t SDF_CAMERA_SLOTS = 1u << 14, SDF_WHOLE_SLOTS = 1u << 21, SDF_BOUNCE_SLOTS = 1u << 26;
 constexpr uint32_t FIRST_BOUNCE_SLOTS = 1u << 24;
 constexpr int32_t FIRST_BOUNCE_NODES = 256;

@@ -21,9 +21,10 @@
 // hit wins.
 
 constexpr int MARCH_BLOCK = 256;
-// A wave's march claim takes this many times the extend kernels' claim (tuning's wave_batch) from the one shared
-// counter: with claims as small as the extend kernels' the waves waited on that counter (the SDF frame at 128,
-// 512, 1024 and 2048 items per claim for both kinds of kernel: 85.6, 76.7, 79.3 and 89.3 ms).
+// The most march items a wave claims at a time, as a multiple of the extend kernels' (tuning's wave_batch): an item is
+// less work than a ray's traversal, and with claims as small the waves waited on the counters, one for the whole
+// launch then and CLAIM_PARTS of them now (the SDF frame at 128, 512, 1024 and 2048 items per claim from one counter:
+// 85.6, 76.7, 79.3 and 89.3 ms).
 constexpr uint32_t MARCH_CLAIM_FACTOR = 4;
 // Fewest items a wave claims (the 161x91, 9-sample SDF frame at 32, 16 and 8: 9.68, 9.39 and 9.26 ms).
 constexpr uint32_t MARCH_CLAIM_LEAST = 8;

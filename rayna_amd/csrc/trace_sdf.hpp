@@ -11,8 +11,8 @@
 // bounded objects' tree once enough lanes wait for that.
 //
 // Each march is k_march's (the same steps, exits and outcomes), each normal sdf_normal's, and the merge's order is
-// kept: object by object, strict < against the closest hit so far.  Bound by VALU issue (1.5 wave64 instructions per
-// CU per cycle, 43% of lanes active, on the 720p frame) and, for small frames, by the serial chain of the longest
+// kept: object by object, strict < against the closest hit so far.  Bound by VALU issue (1.366 wave64 instructions per
+// CU per cycle, 41.0% of lanes active, on the 720p frame) and, for small frames, by the serial chain of the longest
 // path's estimates.  Per call, before and after: the 161x91, 9-sample SDF frame 8.9 -> 4.4 ms, the 720p, 128-sample
 // one 76.1 -> 71.9 (launched_depths says which depths stay apart), the batch of 16 requests 29.1 -> 20.3.
 
@@ -21,7 +21,10 @@
 // paths and traces their rays through the tree: fewer where that is cheap beside a pass of estimates, as it is beside a
 // Mandelbulb's iterations, more where it is the work and estimates are cheap.  (At 16, 32 and 48: the Mandelbulb scene
 // at 1280x720x128 71.8, 76.0 and above 81 ms, at 640x360x64 17.2, 17.9 and 19.5; a scene of 60 bounded objects and one
-// sphere SDF at 1280x720x64 19.0, 14.2 and 13.5 ms, at 333x217x30 3.20, 2.72 and 2.64.)  Once there are no paths left to
+// sphere SDF at 1280x720x64 19.0, 14.2 and 13.5 ms, at 333x217x30 3.20, 2.72 and 2.64.  "No Mandelbulb" stands for cheap
+// estimates: sixteen smooth-min spheres alone, whose estimates are not, would rather wait for fewer, at 16, 24, 48 and 63
+// lanes 12.4, 12.1, 12.8 and 16.0 ms at 1280x720x64 and 4.21, 4.23, 4.61 and 5.35 at 640x360x64.)  The lanes are shares of
+// refill_lanes, 32 by default.  Once there are no paths left to
 // take, a quarter of its paths (the 161x91, 9-sample frame at half, a quarter, an eighth and a sixty-fourth: 4.31, 4.19,
 // 4.20 and 4.28 ms).
 constexpr int SDF_TRACE_WAVES = 5;
