@@ -36,6 +36,7 @@ enum : uint32_t {
     SCENE_SDFS = 8u,
     SCENE_TEXTURED = 16u,
     SCENE_MANDELBULBS = 32u,
+    SCENE_NO_SDFS = 64u,
 };
 
 // One request's share of a chunk: samples [s0, s0 + n) of request `req`.
@@ -430,6 +431,7 @@ SceneView chunk_view(const SceneView &merged, uint32_t features, int32_t n_nodes
     v.textured = (features & SCENE_TEXTURED) ? merged.textured : 0;
     v.n_sdfs = (features & SCENE_SDFS) ? merged.n_sdfs : 0;
     v.mandelbulbs = (features & SCENE_MANDELBULBS) ? merged.mandelbulbs : 0;
+    v.mixed = (features & SCENE_SDFS) && (features & SCENE_NO_SDFS) ? 1 : 0;
     return v;
 }
 
@@ -585,6 +587,7 @@ rayna_status rayna_batch_create(const rayna_scene_desc *scenes, int32_t n_scenes
         if (has_spheres(p)) f |= SCENE_SPHERES;
         if (!p.volumes.empty()) f |= SCENE_MEDIA;
         if (!p.sdfs.empty()) f |= SCENE_SDFS;
+        else f |= SCENE_NO_SDFS;
         if (has_mandelbulbs(p)) f |= SCENE_MANDELBULBS;
         if (has_textures(p) || p.skybox == RAYNA_SKY_HDRI) f |= SCENE_TEXTURED;
         b->scene_features[i] = f;

@@ -1628,6 +1628,7 @@ void launch_extend(const SceneView &sv, const FrameParams &fp, const PathBuffers
 uint32_t launched_depths(const SceneView &sv, const FrameParams &fp, const ExtendTuning &tune, const BatchView &bv) {
     if (fp.mode != RAYNA_MODE_PBR || fp.checks) return 0xffffffffu;
     if (sv.n_sdfs > 0) {
+        if (sv.mixed && fp.n_slots >= SDF_BOUNCE_SLOTS) return MIXED_DEPTHS;
         const bool camera_rays = fp.n_slots >= SDF_CAMERA_SLOTS && fp.n_slots < SDF_WHOLE_SLOTS;
         return fp.n_slots >= SDF_BOUNCE_SLOTS ? 2 : camera_rays ? 1 : 0;
     }

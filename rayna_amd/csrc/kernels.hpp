@@ -139,7 +139,14 @@ void launch_extend(const SceneView &sv, const FrameParams &fp, const PathBuffers
 // So between 2^14 and 2^21 paths a scene of one kind of SDF would do better with no launch apart, and one of mostly
 // bounded objects with two; the rule's choice is within 5% of a launch per depth or faster on all of them but the last
 // at 320x180x8 and 640x360x4 and x8 (1.38 against 1.29, 1.71 against 1.49, 2.15 against 1.84).
+//
+// A batch's chunk of that size that mixes scenes with and without unbounded objects launches four depths: in one wave of
+// k_trace_sdf a mesh's traversal stalls the marches and the other way round, where k_extend and k_march take each kind
+// in full waves.  (64 requests of three scenes, two of them without SDFs, in chunks of up to 2^29 paths, three in flight,
+// with 2, 3, 4 and all depths launched: shortest first 1972, 1844, 1760 and 1701 ms, in the order given 2115, 1956, 1871
+// and 1799; 24 smaller requests in one chunk 74.1, 71.8, 71.0 and 76.9.)
 constexpr uint32_t SDF_CAMERA_SLOTS = 1u << 14, SDF_WHOLE_SLOTS = 1u << 21, SDF_BOUNCE_SLOTS = 1u << 26;
+constexpr uint32_t MIXED_DEPTHS = 4;
 constexpr uint32_t FIRST_BOUNCE_SLOTS = 1u << 24;
 constexpr int32_t FIRST_BOUNCE_NODES = 256;
 uint32_t launched_depths(const SceneView &sv, const FrameParams &fp, const ExtendTuning &tune, const BatchView &bv);

@@ -205,6 +205,7 @@ struct SceneView {
     int32_t root;        // -1: no bounded object
     int32_t n_nodes;
     int32_t n_sdfs;
+    int32_t mixed;       // a batch's chunk: 1 if it holds paths of scenes without unbounded objects beside those with
     int32_t mandelbulbs; // 1 if some unbounded object is a Mandelbulb (its estimate is an iteration)
     int32_t skybox;
     int32_t stack_need;   // deepest per-lane stack k_extend can need (speculative traversal)

@@ -128,3 +128,21 @@ def test_a_chunk_is_launched_as_its_own_scenes_ask(gpu):
             images.append(imgs[0])
     assert launches[0] == launches[1]
     assert np.array_equal(*images)
+
+
+@pytest.mark.parametrize("mixed", [True, False])
+def test_large_chunks_that_mix_scenes(gpu, mixed):
+    """From 2^26 paths on, a chunk of scenes with and without unbounded objects gives four depths launches of their own, one
+    of a scene with unbounded objects two; each image is its single render's."""
+    kinds = [presets.sdf_volume(max_iterations=64), presets.cornell() if mixed else presets.sdf_volume(max_iterations=64)]
+    reqs = []
+    for k, (_, cam, opts) in enumerate(kinds):
+        opts = replace(opts, width=1024, height=1024, samples=33, ray_depth=5, seed=k)
+        reqs.append(Request(k, cam, opts, "rowmajor"))
+    scenes = [k[0] for k in kinds]
+    with BatchRenderer(scenes) as b:
+        imgs, st = b.render(reqs)
+    # fills, generate, five or six kernels to a depth, the rest in one, count, resolve, finalize, the call's fill
+    assert st.chunks == 1 and st.launches == 3 + 5 * (4 if mixed else 2) + 1 + 3 + 1
+    for q, img in zip(reqs, imgs):
+        assert np.array_equal(img, _single(scenes, q)[0])
