@@ -420,16 +420,17 @@ void make_plan(rayna_batch *b, const rayna_request *reqs, int n, const std::vect
 // The merged scene set's view as one chunk sees it: the kernels compile out the sphere test, media, instance
 // and texture code and, without SDFs, the SDF normal code (k_shade's eight-wave form), so a chunk whose requests'
 // scenes hold none of these runs the forms a single render of those scenes would.  A request's rays only reach
-// its own scene's tree, so the other scenes' items never meet the compiled-out code.  n_nodes: the rules on the size of
-// a tree (launched_depths, launch_trace) go by the largest that rays of the chunk enter.
-SceneView chunk_view(const SceneView &merged, uint32_t features, int32_t n_nodes) {
+// its own scene's tree, so the other scenes' items never meet the compiled-out code.  n_nodes, n_sdfs: the
+// rules on the size of a tree and on the unbounded objects (launched_depths, launch_trace) go by the most that a path of
+// the chunk meets.
+SceneView chunk_view(const SceneView &merged, uint32_t features, int32_t n_nodes, uint32_t n_sdfs) {
     SceneView v = merged;
     v.n_nodes = n_nodes;
+    v.n_sdfs = (int32_t)n_sdfs;
     v.instances = (features & SCENE_INSTANCES) ? merged.instances : 0;
     v.sphere_tests = (features & SCENE_SPHERES) ? merged.sphere_tests : 0;
     v.media = (features & SCENE_MEDIA) ? merged.media : 0;
     v.textured = (features & SCENE_TEXTURED) ? merged.textured : 0;
-    v.n_sdfs = (features & SCENE_SDFS) ? merged.n_sdfs : 0;
     v.mandelbulbs = (features & SCENE_MANDELBULBS) ? merged.mandelbulbs : 0;
     v.mixed = (features & SCENE_SDFS) && (features & SCENE_NO_SDFS) ? 1 : 0;
     return v;
@@ -439,10 +440,11 @@ SceneView chunk_view(const SceneView &merged, uint32_t features, int32_t n_nodes
 uint32_t plan_launches(const rayna_batch *b, const Plan &pl, int used) {
     uint32_t n = (uint32_t)used;  // segment counters
     for (size_t c = 0; c < pl.chunks.size(); ++c) {
-        const SceneView cv = chunk_view(b->view, pl.features[c], pl.n_nodes[c]);
+        const SceneView cv = chunk_view(b->view, pl.features[c], pl.n_nodes[c], pl.n_sdf[c]);
         const BatchView bv{b->table, (uint32_t)pl.chunks[c].size(), nullptr};
         FrameParams fp{};
         fp.n_slots = pl.slots[c];
+        fp.ray_depth = pl.depth[c];
         const uint32_t depths = pl.depth[c] + 1, apart = std::min(depths, launched_depths(cv, fp, b->tune, bv));
         const uint32_t nf = pl.first_final[c + 1] - pl.first_final[c];
         const uint32_t traced = (pl.n_sdf[c] ? 5 : 2) * apart + (apart < depths ? 1 : 0);
@@ -477,7 +479,7 @@ hipError_t enqueue(rayna_batch *b, const Plan &pl, int used, bool timing) {
         fp.n_slots = pl.slots[c];
         fp.ray_depth = pl.depth[c];
         const uint32_t D = pl.depth[c];
-        const SceneView cv = chunk_view(b->view, pl.features[c], pl.n_nodes[c]);
+        const SceneView cv = chunk_view(b->view, pl.features[c], pl.n_nodes[c], pl.n_sdf[c]);
         launch_fill_u32(P.queue_count, 0u, 2 * (D + 2), s);
         launch_fill_u32(P.claims, 0u, SEGMENT_WORDS + (D + 1) * 2 * CLAIM_WORDS, s);
         SegmentCounter *queries = reinterpret_cast<SegmentCounter *>(P.claims);

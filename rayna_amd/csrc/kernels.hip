@@ -1629,6 +1629,12 @@ uint32_t launched_depths(const SceneView &sv, const FrameParams &fp, const Exten
     if (fp.mode != RAYNA_MODE_PBR || fp.checks) return 0xffffffffu;
     if (sv.n_sdfs > 0) {
         if (sv.mixed && fp.n_slots >= SDF_BOUNCE_SLOTS) return MIXED_DEPTHS;
+        if (sv.n_nodes <= MARCHED_NODES) {
+            const bool several = sv.n_sdfs > 1;
+            const uint32_t shallow = !several ? 0 : fp.n_slots < SDF_WHOLE_SLOTS ? 1 : 2;
+            if ((several || !sv.mandelbulbs) && fp.ray_depth <= shallow) return 0xffffffffu;
+            if (several && fp.n_slots >= (sv.mandelbulbs ? BULB_BOUNCE_SLOTS : SDF_WHOLE_SLOTS)) return 2;
+        }
         const bool camera_rays = fp.n_slots >= SDF_CAMERA_SLOTS && fp.n_slots < SDF_WHOLE_SLOTS;
         return fp.n_slots >= SDF_BOUNCE_SLOTS ? 2 : camera_rays ? 1 : 0;
     }

@@ -136,9 +136,19 @@ void launch_extend(const SceneView &sv, const FrameParams &fp, const PathBuffers
 //   the bulb alone         7.19 7.42 8.12 14.6     9.79 12.0 12.6 19.3     22.0 23.5 24.4 34.3     36.9 37.9 40.6 52.8
 //   the blobs alone        2.69 4.03 4.54 7.89     4.49 5.58 6.23 10.4     12.9 13.2 13.5 19.1     24.5 23.6 23.0 29.3
 //   60 bounded, a sphere   2.44 2.78 2.65 2.53     3.83 4.59 4.89 4.87     12.2 13.5 13.0 13.9     24.0 25.5 24.0 25.6
-// So between 2^14 and 2^21 paths a scene of one kind of SDF would do better with no launch apart, and one of mostly
-// bounded objects with two; the rule's choice is within 5% of a launch per depth or faster on all of them but the last
-// at 320x180x8 and 640x360x4 and x8 (1.38 against 1.29, 1.71 against 1.49, 2.15 against 1.84).
+// So between 2^14 and 2^21 paths a scene of one SDF would do better with no launch apart, and one of mostly bounded
+// objects with two; the rule's choice is within 5% of a launch per depth or faster on all of them but the last at
+// 320x180x8 and 640x360x4 and x8 (1.38 against 1.29, 1.71 against 1.49, 2.15 against 1.84).
+//
+// Of scenes that are all but nothing else than marches (at most MARCHED_NODES tree nodes), those of several unbounded
+// objects leave a k_trace_sdf wave's lanes at different ones, so they launch the first bounce from fewer paths on
+// (with 0 and 2 depths launched: two sets of blobs 640x360x16 7.0 and 5.9 ms, x64 13.2 and 11.0, 1280x720x32 20.7 and
+// 16.5; six spheres 640x360x16 2.32 and 2.17, 1280x720x32 8.1 and 7.6; the bulb and the blobs 640x360x64 17.5 and 18.5,
+// 1280x720x32 26.7 and 25.9: BULB_BOUNCE_SLOTS with a Mandelbulb, SDF_WHOLE_SLOTS without) and, where paths end after two
+// or three vertices, every depth (with none and all launched, depth limits 0, 1 and 2: two sets of blobs 640x360x16 3.8
+// and 1.9, 5.0 and 3.1, 5.6 and 4.0 ms; the bulb and the blobs 640x360x64 6.1 and 4.5, 7.9 and 7.5, 9.2 and 9.3,
+// 1280x720x40 10.8 and 8.3, 15.6 and 12.5, 17.9 and 15.7).  Camera rays alone: one set of blobs 1280x720x40 6.1 and 5.7,
+// the bulb 5.1 and 5.8.
 //
 // A batch's chunk of that size that mixes scenes with and without unbounded objects launches four depths: in one wave of
 // k_trace_sdf a mesh's traversal stalls the marches and the other way round, where k_extend and k_march take each kind
@@ -146,7 +156,8 @@ void launch_extend(const SceneView &sv, const FrameParams &fp, const PathBuffers
 // with 2, 3, 4 and all depths launched: shortest first 1972, 1844, 1760 and 1701 ms, in the order given 2115, 1956, 1871
 // and 1799; 24 smaller requests in one chunk 74.1, 71.8, 71.0 and 76.9.)
 constexpr uint32_t SDF_CAMERA_SLOTS = 1u << 14, SDF_WHOLE_SLOTS = 1u << 21, SDF_BOUNCE_SLOTS = 1u << 26;
-constexpr uint32_t MIXED_DEPTHS = 4;
+constexpr uint32_t MIXED_DEPTHS = 4, BULB_BOUNCE_SLOTS = 3u << 23;
+constexpr int32_t MARCHED_NODES = 4;
 constexpr uint32_t FIRST_BOUNCE_SLOTS = 1u << 24;
 constexpr int32_t FIRST_BOUNCE_NODES = 256;
 uint32_t launched_depths(const SceneView &sv, const FrameParams &fp, const ExtendTuning &tune, const BatchView &bv);

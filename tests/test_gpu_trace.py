@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 
 import oracle
-from rayna_amd import Camera, Renderer, RenderOpts, presets
+from rayna_amd import Camera, Renderer, RenderOpts, Scene, presets
 from tests.test_stack_bound import deep_scene
 
 pytestmark = pytest.mark.gpu
@@ -100,3 +100,29 @@ def test_tuning_reaches_the_whole_path_launches(gpu, scene, width, height, sampl
             times.append(np.median([r.render(to_host=False).stats.kernel_ms for _ in range(7)]))
     assert all(np.array_equal(images[0], i) for i in images[1:])
     assert times[1] > 1.2 * times[0]
+
+
+@pytest.mark.parametrize("width,samples,depth,apart", [(40, 1, 0, True), (40, 1, 1, True), (40, 1, 2, False),
+                                                       (1449, 1, 2, True), (1449, 1, 3, True), (1448, 1, 3, True),
+                                                       (200, 6, 2, True), (200, 6, 0, True)])
+@pytest.mark.parametrize("scene", ["two sets of blobs", "bulb and blobs", "blobs"])
+def test_scenes_of_marches(gpu, scene, width, samples, depth, apart):
+    """Scenes of nothing but marches: several unbounded objects' depths get launches of their own in frames of few vertices
+    to a path and from 2^21 paths on (1449 * 1449; with a Mandelbulb from 3 * 2^23), between 2^14 paths and those the
+    camera rays do; the frames equal those of a launch per depth."""
+    sc, cam, opts = presets.sdf_volume(width=width, height=width, samples=samples, ray_depth=depth, max_iterations=48)
+    bulb, blobs = sc.objects[:2]
+    moved, _, _ = presets.sdf_volume(seed=9, max_iterations=48)
+    sc = Scene({"two sets of blobs": [blobs, moved.objects[1]], "bulb and blobs": [bulb, blobs], "blobs": [blobs]}[scene],
+               sc.skybox)
+    with Renderer(sc, cam, opts) as r:
+        out = r.render(layout="rowmajor")
+        r.clear_accumulation()
+        r.set_validate(True)
+        ref = r.render(layout="rowmajor")
+    assert np.array_equal(out.img, ref.img) and out.stats.segments == ref.stats.segments
+    if scene == "blobs":
+        apart = depth == 0 or 1 << 14 <= width * width * samples < 1 << 21
+    elif scene == "bulb and blobs" and width == 1449 and depth == 3:
+        apart = False
+    assert (out.stats.shade_ms > 0.0) == apart
