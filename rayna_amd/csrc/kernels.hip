@@ -1662,8 +1662,9 @@ void launch_trace(const SceneView &sv, const FrameParams &fp, const PathBuffers 
                                              : TRACE_KERNELS[k][t][i][f];
     const int resident = sv.n_sdfs > 0 ? o.trace_sdf[k][fs] : quad ? o.quad[k][t][f] : o.trace[k][t][i][f];
     const int g = std::max(1, std::min(grid, grid / o.most * resident));
-    const TraceArgs args{sv,   fp,   pb,       queue, count,    first_depth,
-                         overflow, work, segments, tune,  adjoint ? *adjoint : AdjointParams{}, bv};
+    const int sdf = sv.n_sdfs == 0 ? 0 : sv.mandelbulbs ? 2 : 1;
+    const TraceArgs args{sv, fp, pb, queue, count, first_depth, overflow, work, segments,
+                         trace_tuning(tune, sdf, quad && sdf == 0), adjoint ? *adjoint : AdjointParams{}, bv};
     hipLaunchKernelGGL(kernel, dim3(g), dim3(EXT_BLOCK), 0, s, args);
 }
 

@@ -22,8 +22,14 @@ constexpr uint32_t TRACE_CLAIM_LEAST = 4;
 // With four lanes to a path a wave holds sixteen: more at a time would leave the others idle (the four mesh preview
 // frames at most 8, 16 and 32: 2.74, 2.73 and 3.18 ms; the sphere thumbnail at least 1, 2 and 4: 161, 171 and 170 us).
 constexpr uint32_t QUAD_CLAIM_LEAST = 1;
-__device__ __forceinline__ uint32_t quad_claim_most(const ExtendTuning &tune) {  // 16 for the default of 128
-    return tune.wave_batch / 8u > QUAD_CLAIM_LEAST ? tune.wave_batch / 8u : QUAD_CLAIM_LEAST;
+
+// The launch's shares of the tunables, 32 lanes and 128 positions by default (worked out on the host: in the kernels they
+// would hold registers).  sdf: 1 for k_trace_sdf, 2 if there is a Mandelbulb too.
+inline ExtendTuning trace_tuning(ExtendTuning t, int sdf, bool quad) {
+    const uint32_t n = t.refill_lanes;
+    t.refill_lanes = sdf == 2 ? std::max(1u, n / 2u) : std::min(64u, sdf == 1 ? n + n / 2u : n + n / 4u);
+    if (quad) t.wave_batch = std::max(QUAD_CLAIM_LEAST, t.wave_batch / 8u);
+    return t;
 }
 
 // The arguments of k_trace and k_trace_sdf, one struct so that a kernel finds them at the start of its argument segment.
@@ -37,7 +43,7 @@ struct TraceArgs {
     int2 *overflow;
     uint32_t *work;
     SegmentCounter *segments;
-    ExtendTuning tune;
+    ExtendTuning tune;  // trace_tuning's
     AdjointParams ap;
     BatchView bv;
 };
@@ -77,9 +83,7 @@ __global__ __launch_bounds__(EXT_BLOCK) __attribute__((amdgpu_waves_per_eu(trace
     // take, idle lanes say nothing: half of the wave's paths then wait (against refill_lanes waiting or idle, where a
     // wave with few paths shaded them one by one: the preview frames 4.24 -> 3.96 ms, the inverse-rendering step 3.97 ->
     // 3.80; at a third 4.01 and 3.77, at a twelfth 4.18 and 3.95).
-    const uint32_t refill_lanes = args.tune.refill_lanes + args.tune.refill_lanes / 4u < 64u
-                                      ? args.tune.refill_lanes + args.tune.refill_lanes / 4u
-                                      : 64u;
+    const uint32_t refill_lanes = args.tune.refill_lanes;
     const uint32_t gid = blockIdx.x * EXT_BLOCK + threadIdx.x;
     const uint32_t lane = __lane_id();
     const bool lead = !QUAD || (lane & 3u) == 0u;
@@ -93,7 +97,7 @@ __global__ __launch_bounds__(EXT_BLOCK) __attribute__((amdgpu_waves_per_eu(trace
     LeafRange leaf;
     TravStats stats;
     WaveClaims claims(count, EXT_BLOCK / 64, QUAD ? QUAD_CLAIM_LEAST : TRACE_CLAIM_LEAST,
-                      QUAD ? quad_claim_most(args.tune) : args.tune.wave_batch, args.work);
+                      args.tune.wave_batch, args.work);
     // the path's RNG key, pixel and sample, and in a batch its request
     auto identify = [&](const TraceArgs &A, dm::Key *key, uint32_t *pixel, uint32_t *sample) -> const RequestParams * {
         if (BATCH) {

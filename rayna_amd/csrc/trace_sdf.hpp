@@ -23,16 +23,10 @@
 // at 1280x720x128 71.8, 76.0 and above 81 ms, at 640x360x64 17.2, 17.9 and 19.5; a scene of 60 bounded objects and one
 // sphere SDF at 1280x720x64 19.0, 14.2 and 13.5 ms, at 333x217x30 3.20, 2.72 and 2.64.  "No Mandelbulb" stands for cheap
 // estimates: sixteen smooth-min spheres alone, whose estimates are not, would rather wait for fewer, at 16, 24, 48 and 63
-// lanes 12.4, 12.1, 12.8 and 16.0 ms at 1280x720x64 and 4.21, 4.23, 4.61 and 5.35 at 640x360x64.)  The lanes are shares of
-// refill_lanes, 32 by default.  Once there are no paths left to
-// take, a quarter of its paths (the 161x91, 9-sample frame at half, a quarter, an eighth and a sixty-fourth: 4.31, 4.19,
-// 4.20 and 4.28 ms).
+// lanes 12.4, 12.1, 12.8 and 16.0 ms at 1280x720x64 and 4.21, 4.23, 4.61 and 5.35 at 640x360x64; trace_tuning has the
+// shares of refill_lanes.)  Once there are no paths left to take, a quarter of its paths (the 161x91, 9-sample frame at
+// half, a quarter, an eighth and a sixty-fourth: 4.31, 4.19, 4.20 and 4.28 ms).
 constexpr int SDF_TRACE_WAVES = 5;
-__device__ __forceinline__ uint32_t sdf_refill_lanes(const ExtendTuning &tune, bool mandelbulbs) {
-    const uint32_t n = tune.refill_lanes;  // 32 by default: 16 and 48 then
-    if (mandelbulbs) return n > 1u ? n / 2u : 1u;
-    return n + n / 2u < 64u ? n + n / 2u : 64u;
-}
 
 template <bool BATCH, bool INST, bool SPH, bool VOL, bool TEX, bool ADJOINT>
 __global__ __launch_bounds__(EXT_BLOCK) __attribute__((amdgpu_waves_per_eu(SDF_TRACE_WAVES))) void k_trace_sdf(
@@ -55,7 +49,7 @@ __global__ __launch_bounds__(EXT_BLOCK) __attribute__((amdgpu_waves_per_eu(SDF_T
     int step = 0;                     // the march's step; the normal's estimate (0..5: +x -x +y -y +z -z)
     f3 g{0.0f, 0.0f, 0.0f};           // the estimate's differences, then the normal
     WaveClaims claims(count, EXT_BLOCK / 64, TRACE_CLAIM_LEAST, args.tune.wave_batch, args.work);
-    const uint32_t refill_lanes = sdf_refill_lanes(args.tune, args.sv.mandelbulbs != 0);
+    const uint32_t refill_lanes = args.tune.refill_lanes;
     TravStats stats;
     // the path's RNG key, pixel and sample, and in a batch its request
     auto identify = [&](const TraceArgs &A, dm::Key *key, uint32_t *pixel, uint32_t *sample) -> const RequestParams * {
