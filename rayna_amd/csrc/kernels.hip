@@ -1520,11 +1520,9 @@ const TraceKernel TRACE_SDF_KERNELS[3][3] = {RAYNA_TRACE_SDF_FORMS(false, false)
                                                 RAYNA_TRACE_SDF_FORMS(false, true)};
 #undef RAYNA_TRACE_SDF_FORMS
 
-using ExtendKernel = void (*)(SceneView, FrameParams, PathBuffers, const int32_t *, const uint32_t *, uint32_t,
-                              int2 *, uint32_t *, ExtendTuning, BatchView);
 // The k_extend instantiations, [batch][instances][form]: form 0 neither spheres nor media, 1 spheres, 2 media
 // (with the sphere tests, which sphere-bounded media need).
-const ExtendKernel EXTEND_KERNELS[2][2][3] = {
+const TraceKernel EXTEND_KERNELS[2][2][3] = {
     {{k_extend<false, false, false, false>, k_extend<false, false, true, false>, k_extend<false, false, true, true>},
      {k_extend<false, true, false, false>, k_extend<false, true, true, false>, k_extend<false, true, true, true>}},
     {{k_extend<true, false, false, false>, k_extend<true, false, true, false>, k_extend<true, false, true, true>},
@@ -1617,8 +1615,8 @@ void launch_extend(const SceneView &sv, const FrameParams &fp, const PathBuffers
     // `grid` is the CU count times the largest residency of any form, which the overflow columns are sized
     // for; each form launches as many blocks as stay resident (never more than `grid`)
     const int g = std::max(1, std::min(grid, std::max(1, grid / extend_blocks_per_cu()) * extend_occupancy().n[b][i][f]));
-    hipLaunchKernelGGL(EXTEND_KERNELS[b][i][f], dim3(g), dim3(EXT_BLOCK), 0, s, sv, fp, pb, queue, count, depth,
-                       overflow, work, tune, bv);
+    hipLaunchKernelGGL(EXTEND_KERNELS[b][i][f], dim3(g), dim3(EXT_BLOCK), 0, s,
+                       TraceArgs{sv, fp, pb, queue, count, depth, overflow, work, nullptr, tune, AdjointParams{}, bv});
 }
 
 uint32_t launched_depths(const SceneView &sv, const FrameParams &fp, const ExtendTuning &tune, const BatchView &bv) {

@@ -32,21 +32,6 @@ inline ExtendTuning trace_tuning(ExtendTuning t, int sdf, bool quad) {
     return t;
 }
 
-// The arguments of k_trace and k_trace_sdf, one struct so that a kernel finds them at the start of its argument segment.
-struct TraceArgs {
-    SceneView sv;
-    FrameParams fp;
-    PathBuffers pb;
-    const int32_t *queue;
-    const uint32_t *count;
-    uint32_t first_depth;
-    int2 *overflow;
-    uint32_t *work;
-    SegmentCounter *segments;
-    ExtendTuning tune;  // trace_tuning's
-    AdjointParams ap;
-    BatchView bv;
-};
 // Adds the closest-hit queries that the wave's lanes counted to one of the SEGMENT_PARTS counters.  A wave's own sum fits
 // 32 bits with room to spare: 2^31 paths (no GPU holds more) of a thousand vertices, over the thousands of waves that
 // share them evenly, are 2^29 a wave.  (Summed in 64 bits the kernels' register allocation changed throughout: the
@@ -56,16 +41,6 @@ __device__ __forceinline__ void add_segments(SegmentCounter *segments, uint32_t 
     if (__lane_id() == 0u && lane_count != 0u)
         atomicAdd(segments + SEGMENT_STRIDE * (blockIdx.x % SEGMENT_PARTS), (SegmentCounter)lane_count);
 }
-// The arguments again, read where they are used: some ninety words of them serve the shading and refill alone, and
-// loaded once at the kernel's start they would hold (and spill, into vector registers) scalar registers through the
-// traversal loops.  The compiler cannot move these loads out of the loop, because it does not know the pointer.
-__device__ __forceinline__ const TraceArgs &cold_args() {
-    typedef __attribute__((address_space(4))) const TraceArgs *Segment;
-    Segment p = (Segment)__builtin_amdgcn_kernarg_segment_ptr();
-    asm volatile("" : "+s"(p));
-    return *(const TraceArgs *)p;
-}
-
 // first_depth 0: the paths are the chunk's slots, from their camera rays (computed here).  first_depth > 0: the paths
 // are queue[0 .. *count_ptr), which k_shade kept at depth 0, from their stored rays and throughputs.
 //

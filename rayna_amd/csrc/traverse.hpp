@@ -351,6 +351,34 @@ __device__ __forceinline__ void traverse_pass(const SceneView &sv, const PathBuf
     } while ((uint32_t)__popcll(__ballot(leaf.code != 0)) > EXTEND_PRIM_EXIT);
 }
 
+// The arguments of k_extend, k_trace and k_trace_sdf (k_extend: of one depth, first_depth), one struct so that a kernel
+// finds them at the start of its argument segment.
+struct TraceArgs {
+    SceneView sv;
+    FrameParams fp;
+    PathBuffers pb;
+    const int32_t *queue;
+    const uint32_t *count;
+    uint32_t first_depth;
+    int2 *overflow;
+    uint32_t *work;
+    SegmentCounter *segments;
+    ExtendTuning tune;  // k_extend: the renderer's or batch's; else trace_tuning's
+    AdjointParams ap;
+    BatchView bv;
+};
+// The arguments again, read where they are used: some ninety words of them serve the shading and refill alone, and
+// loaded once at the kernel's start they would hold (and spill, into vector registers) scalar registers through the
+// traversal loops.  The compiler cannot move these loads out of the loop, because it does not know the pointer.  (k_extend
+// with its refill's words read this way: no scalar register spilled without media or instances instead of 12-25, 17
+// instead of 44 with both; the 1080p mesh frame 44.5 -> 44.0 ms, camera rays of a 1080p, 33-sample RTTNW frame 3.5 -> 3.2.)
+__device__ __forceinline__ const TraceArgs &cold_args() {
+    typedef __attribute__((address_space(4))) const TraceArgs *Segment;
+    Segment p = (Segment)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return *(const TraceArgs *)p;
+}
+
 // Fewest queue positions a wave claims: below 4 * 7000 paths the launch runs on fewer waves instead of on waves of one
 // or two lanes.  (Four 641x359, 1-sample mesh frames at 32, 16, 8 and 4: 5.89, 5.79, 5.62 and 5.39 ms; the 64x36,
 // 2-sample sphere frame 0.57, 0.58, 0.58, 0.53; larger frames within 1%.)
@@ -373,41 +401,41 @@ constexpr uint32_t EXTEND_CLAIM_LEAST = 4;
 template <bool BATCH, bool INST, bool SPH, bool VOL>
 __global__ __launch_bounds__(EXT_BLOCK) __attribute__((amdgpu_waves_per_eu(
     (INST || SPH || VOL) ? RAYNA_EXT_WAVES : RAYNA_EXT_WAVES_LEAN))) void k_extend(
-    SceneView sv, FrameParams fp, PathBuffers pb, const int32_t *queue, const uint32_t *count_ptr, uint32_t depth,
-    int2 *overflow, uint32_t *work, ExtendTuning tune, BatchView bv) {
+    TraceArgs args) {
     __shared__ unsigned long long s_entry[EXT_LDS_STACK * EXT_BLOCK];
-    const uint32_t count = queue ? *count_ptr : fp.n_slots;
-    const uint32_t refill_lanes = tune.refill_lanes;
-    dm::Key key{fp.key0, fp.key1};
+    const uint32_t count = args.queue ? *args.count : args.fp.n_slots;
+    const uint32_t refill_lanes = args.tune.refill_lanes;
+    dm::Key key{args.fp.key0, args.fp.key1};
     const uint32_t gid = blockIdx.x * EXT_BLOCK + threadIdx.x;
-    LaneStack st{(lds_u64 *)s_entry, overflow + gid, gridDim.x * EXT_BLOCK, 0};
+    LaneStack st{(lds_u64 *)s_entry, args.overflow + gid, gridDim.x * EXT_BLOCK, 0};
     bool active = false;
     uint32_t slot = 0, pixel = 0, sample = 0;
     DRay ray{};
     Best b{FLT_MAX, -1, 0u, 0u};
     LeafRange leaf;
-    WaveClaims claims(count, EXT_BLOCK / 64, EXTEND_CLAIM_LEAST, tune.wave_batch, work);
+    WaveClaims claims(count, EXT_BLOCK / 64, EXTEND_CLAIM_LEAST, args.tune.wave_batch, args.work);
     TravStats stats;
     for (;;) {
         const unsigned long long idle = __ballot(!active);
         if (!claims.exhausted && (idle == ~0ull || (uint32_t)__popcll(idle) >= refill_lanes)) {
+            const TraceArgs &A = cold_args();
             const uint32_t q = claims.hand_out(idle);
             if (!active) {
                 if (q != 0xffffffffu) {
-                    slot = queue ? (uint32_t)queue[q] : q;
-                    ray = ray_from_dir(f3{pb.ox[slot], pb.oy[slot], pb.oz[slot]},
-                                       f3{pb.dx[slot], pb.dy[slot], pb.dz[slot]});
-                    int32_t root = sv.root;
+                    slot = A.queue ? (uint32_t)A.queue[q] : q;
+                    ray = ray_from_dir(f3{A.pb.ox[slot], A.pb.oy[slot], A.pb.oz[slot]},
+                                       f3{A.pb.dx[slot], A.pb.dy[slot], A.pb.dz[slot]});
+                    int32_t root = A.sv.root;
                     if (BATCH) {
-                        const RequestParams &R = bv.reqs[bv.slot_req[slot]];
+                        const RequestParams &R = A.bv.reqs[A.bv.slot_req[slot]];
                         const uint32_t l = slot - R.slot_base;
                         pixel = l / R.n_spp;
                         sample = R.s0 + l % R.n_spp;
                         key = dm::Key{R.key0, R.key1};
                         root = R.root;
                     } else {
-                        pixel = slot / fp.n_spp;
-                        sample = fp.s0 + slot % fp.n_spp;
+                        pixel = slot / A.fp.n_spp;
+                        sample = A.fp.s0 + slot % A.fp.n_spp;
                     }
                     b = Best{FLT_MAX, -1, 0u, 0u, 0u};
                     st.sp = 0;
@@ -424,13 +452,14 @@ __global__ __launch_bounds__(EXT_BLOCK) __attribute__((amdgpu_waves_per_eu(
         }
         RAYNA_STAT(iterations);
         if (active) {
-            traverse_pass<INST, SPH, VOL>(sv, pb, slot, ray, b, leaf, st, key, pixel, sample, depth, stats);
+            traverse_pass<INST, SPH, VOL>(args.sv, args.pb, slot, ray, b, leaf, st, key, pixel, sample, args.first_depth,
+                                          stats);
             if (st.sp == 0 && leaf.code == 0) {
-                pb.hit_t[slot] = b.t;
-                pb.hit_ref[slot] = b.ref;
-                pb.hit_aux[slot] = b.aux;
-                if (INST && b.sub) pb.hit_sub[slot] = b.sub;
-                if (pb.hit_rank) pb.hit_rank[slot] = b.rank;
+                args.pb.hit_t[slot] = b.t;
+                args.pb.hit_ref[slot] = b.ref;
+                args.pb.hit_aux[slot] = b.aux;
+                if (INST && b.sub) args.pb.hit_sub[slot] = b.sub;
+                if (args.pb.hit_rank) args.pb.hit_rank[slot] = b.rank;
                 active = false;
             }
         }
