@@ -1632,8 +1632,9 @@ uint32_t launched_depths(const SceneView &sv, const FrameParams &fp, const Exten
         const bool camera_rays = fp.n_slots >= SDF_CAMERA_SLOTS && fp.n_slots < SDF_WHOLE_SLOTS;
         return fp.n_slots >= SDF_BOUNCE_SLOTS ? 2 : camera_rays ? 1 : 0;
     }
-    if (!extend_packets(sv, fp, tune, bv, 0)) return 0;
-    const uint32_t n = fp.n_slots >= FIRST_BOUNCE_SLOTS && sv.n_nodes >= FIRST_BOUNCE_NODES ? 2 : 1;
+    const bool four_waves = sv.media || sv.instances;  // k_trace's forms with either
+    if (!extend_packets(sv, fp, tune, bv, 0)) return four_waves && fp.n_slots >= LANES_BOUNCE_SLOTS ? 2 : 0;
+    const uint32_t n = fp.n_slots >= FIRST_BOUNCE_SLOTS && (four_waves || sv.n_nodes >= FIRST_BOUNCE_NODES) ? 2 : 1;
     return std::max(n, tune.packet_depths);
 }
 

@@ -119,8 +119,13 @@ void launch_extend(const SceneView &sv, const FrameParams &fp, const PathBuffers
 // Without unbounded objects: the camera rays where they are traced as packets, and for a large chunk over a tree that
 // is not small the first bounce too: its rays start from one point per wave, which k_extend's seven waves per SIMD use
 // better than k_trace's mix of depths.  (1080p, 64 samples, first bounce apart against not: 45.6 and 48.6 ms with
-// 1.3 M triangles, 34.6 and 36.5 with 1290, 28.2 and 28.3 with 480 spheres, 27.3 and 25.9 in the Cornell box; at
-// 640x360x64, 8.04 and 7.99 ms with 1.3 M triangles.)
+// 1.3 M triangles, 34.6 and 36.5 with 1290 (235 nodes), 28.2 and 28.3 with 480 spheres (40 nodes), 27.3 and 25.9 in the
+// Cornell box; at 640x360x64, 8.04 and 7.99 ms with 1.3 M triangles.)  With media or instances k_trace has four waves
+// per SIMD against k_extend's six, and the size of the tree does not matter: 521 spheres with a medium 1080p at 16, 33
+// and 64 samples 12.0 and 12.6, 23.8 and 25.1, 45.8 and 48.4 ms, transformed objects 5.44 and 5.69, 10.5 and 11.4, 19.8
+// and 21.7.  Without packets the camera rays are a launch of their own then as well, which pays later: RTTNW 1080p at 16,
+// 33 and 64 samples, depth limit 10, 10.53 and 10.30, 19.8 and 20.4, 36.8 and 38.5 ms, depth limit 2, 6.44 and 6.40, 12.5
+// and 12.8, 23.6 and 24.4.
 //
 // With unbounded objects: k_march's waves are full and each at one SDF, k_trace_sdf's do not wait for a depth's
 // longest march.  So the largest chunks launch the camera rays and the first bounce, where most of the work is; small
@@ -159,7 +164,8 @@ constexpr uint32_t SDF_CAMERA_SLOTS = 1u << 14, SDF_WHOLE_SLOTS = 1u << 21, SDF_
 constexpr uint32_t MIXED_DEPTHS = 4, BULB_BOUNCE_SLOTS = 3u << 23;
 constexpr int32_t MARCHED_NODES = 4;
 constexpr uint32_t FIRST_BOUNCE_SLOTS = 1u << 24;
-constexpr int32_t FIRST_BOUNCE_NODES = 256;
+constexpr uint32_t LANES_BOUNCE_SLOTS = 1u << 26;
+constexpr int32_t FIRST_BOUNCE_NODES = 128;
 uint32_t launched_depths(const SceneView &sv, const FrameParams &fp, const ExtendTuning &tune, const BatchView &bv);
 // first_depth 0: every slot's path from its camera ray; first_depth > 0: the paths launch_shade kept at the depth before.
 // The radiance field holds each path's radiance at the end.  overflow and work as for launch_extend; segments:

@@ -8,6 +8,7 @@ import pytest
 
 import oracle
 from rayna_amd import Camera, Renderer, RenderOpts, Scene, presets
+from rayna_amd.batch import BatchRenderer, Request
 from tests.test_stack_bound import deep_scene
 
 pytestmark = pytest.mark.gpu
@@ -126,3 +127,22 @@ def test_scenes_of_marches(gpu, scene, width, samples, depth, apart):
     elif scene == "bulb and blobs" and width == 1449 and depth == 3:
         apart = False
     assert (out.stats.shade_ms > 0.0) == apart
+
+
+@pytest.mark.parametrize("scene,width,samples,apart", [("mesh", 1024, 16, 2), ("mesh", 1023, 16, 1), ("inverse", 1024, 16, 2),
+                                                       ("cornell", 1024, 16, 1), ("rttnw", 1024, 64, 2),
+                                                       ("rttnw", 1023, 64, 0)])
+def test_first_bounce_of_large_frames(gpu, scene, width, samples, apart):
+    """From 2^24 paths on, the first bounce gets launches of its own in trees of some size and in scenes with media or
+    instances (without camera-ray packets from 2^26 on); the frames equal those of a launch per depth."""
+    sc, cam, opts = SCENES[scene](width=width, height=width, samples=samples, ray_depth=3)
+    with Renderer(sc, cam, opts) as r:
+        out = r.render(layout="rowmajor")
+        r.set_validate(True)
+        r.clear_accumulation()
+        ref = r.render(layout="rowmajor")
+    assert np.array_equal(out.img, ref.img) and out.stats.segments == ref.stats.segments
+    with BatchRenderer([sc]) as b:
+        imgs, st = b.render([Request(0, cam, opts)])
+    assert np.array_equal(imgs[0], ref.img)
+    assert st.launches == 3 + 2 * apart + 1 + 3 + 1
