@@ -486,13 +486,15 @@ __device__ __forceinline__ uint32_t queue_strip(uint32_t count, uint32_t most) {
 // every claim of the launch.  A wave's first claim is fixed by its place in the grid and costs no atomic; the
 // counters hand out what is left after those.  Atomics on one address are served one at a time, about 7 ns each, so
 // where the first claims cover a part nobody touches its counter (a launch over a few thousand positions spent
-// 50-75 us on some 7000 waves each asking every counter).  A wave does not look at another part's counter before it
-// adds to it: a load of that line holds the adds up as another add does (with looks and without, the camera rays of a
-// 1080p, 33-sample RTTNW frame, 160 M claims a second, 5.0 and 3.5 ms, four 641x359, 1-sample mesh frames 2.71 and 2.48;
-// 960x540, 4-sample outward normals, where a wave's last adds find nothing, 0.545 and 0.555).  A claim is the wave's even share of the launch, within bounds: a small launch runs on every wave with
-// few lanes each, instead of on the few waves that full claims would feed.  (Against claims of 128 rays or 512 march
-// items and one atomic each: the 64x36, 2-sample sphere frame 1074 -> 525 us, the 161x91, 9-sample SDF frame 13.7 ->
-// 9.3 ms; shares a half or a quarter as large were 1-10% slower below 400x225x32.)  Every field is wave-uniform.
+// 50-75 us on some 7000 waves each asking every counter), and the wave that takes a part's last claim says so on
+// another line, which waves of other parts look at before they add.  (Not at the counter: a load of that line holds
+// the adds up as another add does.  With looks at the counter, no looks, and looks at the word: the camera rays of a
+// 1080p, 33-sample RTTNW frame, 160 M claims a second, 4.5, 3.2 and 3.3 ms; four 641x359, 1-sample mesh frames 2.71,
+// 2.47 and 2.47; one sphere 640x360x4, where most waves' last adds would find nothing, 88, 106 and 70 us.)  A claim is
+// the wave's even share of the launch, within bounds: a small launch runs on every wave with few lanes each, instead
+// of on the few waves that full claims would feed.  (Against claims of 128 rays or 512 march items and one atomic
+// each: the 64x36, 2-sample sphere frame 1074 -> 525 us, the 161x91, 9-sample SDF frame 13.7 -> 9.3 ms; shares a half
+// or a quarter as large were 1-10% slower below 400x225x32.)  Every field is wave-uniform.
 struct WaveClaims {
     uint32_t count, claim, waves_per_block;
     uint32_t *work;
@@ -529,9 +531,15 @@ struct WaveClaims {
                 first = false;
             } else if (fixed < size) {
                 const uint32_t left = size - (uint32_t)fixed;
-                uint32_t taken = 0;
-                if ((int)__lane_id() == leader) taken = atomicAdd(work + 32 * part, claim);
-                taken = __builtin_amdgcn_readlane(taken, leader);
+                uint32_t taken = left;
+                uint32_t *used_up = work + 32 * CLAIM_PARTS + part;
+                if (parts_done == 0u || __builtin_amdgcn_readfirstlane(__hip_atomic_load(
+                                            used_up, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) == 0u) {
+                    if ((int)__lane_id() == leader) taken = atomicAdd(work + 32 * part, claim);
+                    taken = __builtin_amdgcn_readlane(taken, leader);
+                    if (taken < left && left - taken <= claim)
+                        __hip_atomic_store(used_up, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
                 if (taken < left) base = (uint32_t)fixed + taken;
             }
             const bool got = base < size;

@@ -88,12 +88,13 @@ constexpr int SHADE_BLOCKS_PER_CU = 16;
 // fp.n_slots is the chunk's slot count and the requests come from bv.
 void launch_generate(const FrameParams &fp, const PathBuffers &pb, const BatchView &bv, hipStream_t s);
 // Claim counters of one k_extend or k_march launch: its work is cut into CLAIM_PARTS contiguous parts, each with its
-// own counter, one 128-byte line apart (CLAIM_WORDS words in all, zeroed before the launch).
+// own counter, one 128-byte line apart, and on a line after them a word per part that is set once its last claim is
+// taken (CLAIM_WORDS words in all, zeroed before the launch).
 #ifndef RAYNA_CLAIM_PARTS
 #define RAYNA_CLAIM_PARTS 4
 #endif
 constexpr uint32_t CLAIM_PARTS = RAYNA_CLAIM_PARTS;
-constexpr uint32_t CLAIM_WORDS = CLAIM_PARTS * 32;
+constexpr uint32_t CLAIM_WORDS = (CLAIM_PARTS + 1) * 32;
 
 // Deepest ray_depth that options may ask for.
 constexpr uint32_t MAX_RAY_DEPTH = 1000;
