@@ -46,16 +46,16 @@ def frame_bytes(workload: str):
 # frames of 263,040,107 closest-hit queries each (132,710,400 of them camera rays) at the commit that added them;
 # the times they are divided by are measured live.  The stage is k_extend_packet (camera rays), k_extend (the first
 # bounce) and k_trace (every later vertex, traversed and shaded).  Traffic: what leaves L2 for the fabric, FETCH_SIZE
-# 3.9936e7 KiB read as 64-byte units (x2.0: a 256 MiB copy reads 131,087 KiB) plus WRITE_SIZE 1.0291e7 KiB (x1.0: the
+# 3.9101e7 KiB read as 64-byte units (x2.0: a 256 MiB copy reads 131,087 KiB) plus WRITE_SIZE 1.0651e7 KiB (x1.0: the
 # copy writes 262,143 KiB); it counts hits in the Infinity Cache as well as HBM, so it bounds the HBM bytes from above.
-# VALU (k_extend and k_trace, depths 1-8): SQ_INSTS_VALU 2.3102e10 + 1.4481e10 wave64 instructions over 2 x 130,329,707
-# queries; lanes active SQ_THREAD_CYCLES_VALU / (64 SQ_ACTIVE_INST_VALU) = (6.4028e11 + 3.0339e11) / (64 x 3.7870e10);
-# instructions per CU per cycle from GRBM_GUI_ACTIVE 6.9357e8 + 4.9982e8 over 8 XCDs, 256 CUs.
+# VALU (k_extend and k_trace, depths 1-8): SQ_INSTS_VALU 2.2943e10 + 1.4487e10 wave64 instructions over 2 x 130,329,707
+# queries; lanes active SQ_THREAD_CYCLES_VALU / (64 SQ_ACTIVE_INST_VALU) = (6.4011e11 + 3.0394e11) / (64 x 3.7717e10);
+# instructions per CU per cycle from GRBM_GUI_ACTIVE 6.7131e8 + 5.0384e8 over 8 XCDs, 256 CUs.
 EXTEND_COUNTER_FRAMES = 2 * 263040107
-EXTEND_FABRIC_BYTES_PER_SEGMENT = {"triangle_mesh": (3.9936e7 * 2.0 + 1.0291e7) * 1024 / EXTEND_COUNTER_FRAMES}
-K_EXTEND_VALU_PER_QUERY = {"triangle_mesh": 3.7583e10 / (2 * 130329707)}
-K_EXTEND_LANES_ACTIVE = {"triangle_mesh": 9.4367e11 / (64 * 3.7870e10)}
-K_EXTEND_VALU_PER_CU_CYCLE = {"triangle_mesh": 3.7583e10 / (1.19339e9 / 8 * 256)}
+EXTEND_FABRIC_BYTES_PER_SEGMENT = {"triangle_mesh": (3.9101e7 * 2.0 + 1.0651e7) * 1024 / EXTEND_COUNTER_FRAMES}
+K_EXTEND_VALU_PER_QUERY = {"triangle_mesh": 3.7430e10 / (2 * 130329707)}
+K_EXTEND_LANES_ACTIVE = {"triangle_mesh": 9.4405e11 / (64 * 3.7717e10)}
+K_EXTEND_VALU_PER_CU_CYCLE = {"triangle_mesh": 3.7430e10 / (1.17515e9 / 8 * 256)}
 # VALU issue peak: one wave64 instruction per CU per cycle -- the rate the calibration kernel
 # (rayna_measure_valu_peak: independent fp32 multiply-add chains, no packed or fused forms) reaches per active
 # cycle (0.977 by the same counters) -- at MI355X's published 256 CUs and 2.4 GHz.

@@ -12,9 +12,9 @@
 //
 // Each march is k_march's (the same steps, exits and outcomes), each normal sdf_normal's, and the merge's order is
 // kept: object by object, strict < against the closest hit so far.  Bound by VALU issue (1.366 wave64 instructions per
-// CU per cycle, 41.0% of lanes active, on the 720p frame) and, for small frames, by the serial chain of the longest
+// CU per cycle, 45.2% of lanes active, on the 720p frame) and, for small frames, by the serial chain of the longest
 // path's estimates.  Per call, before and after: the 161x91, 9-sample SDF frame 8.9 -> 4.4 ms, the 720p, 128-sample
-// one 76.1 -> 71.9 (launched_depths says which depths stay apart), the batch of 16 requests 29.1 -> 20.3.
+// one 76.1 -> 66 (launched_depths says which depths stay apart), the batch of 16 requests 29.1 -> 20.3.
 
 // Waves per SIMD (the 161x91, 9-sample SDF frame at 4, 5 and 6: 4.6, 4.5 and 4.2 ms, the 64x36, 2-sample one at 5 and
 // 6: 3.2 and 3.4, the 720p, 128-sample one 83 and 82), and the lanes that wait before a wave shades, takes new
